@@ -1185,8 +1185,9 @@ vox_status node_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, const uint3
     for (uint32_t j = 0; j < nj; j++) {
         const Job &J = P.jobs[j];
         if (!J.pnodes) continue;
-        const size_t n = (size_t)J.gd.X * J.gd.Y * J.gd.Z;
-        k_nodes_partial<<<grid_for(n, 256, 16384), 256, 0, ctx->stream>>>(D.jobs, j);
+        const uint32_t words = J.gd.W * J.gd.Y * J.gd.Z;
+        k_nodes_partial<<<(words + kPartialWords - 1u) / kPartialWords, 256, 0, ctx->stream>>>(
+            D.jobs, j);
         VOX_HIP(hipGetLastError());
     }
     return VOX_OK;

@@ -534,6 +534,7 @@ __global__ void k_nodes_cart_pre(const Job *__restrict__ jobs,
 // for a solid or empty node and the winner triangle's cut ratio for a
 // surface node (0 on a cleared partition border).
 __global__ void k_nodes_partial(const Job *__restrict__ jobs, uint32_t j);
+constexpr uint32_t kPartialWords = 64;  // bit words per block
 inline uint32_t node_blocks(const GridDims &g) {
     return plane_chunks(g.W, g.Y) * ((g.Z + kNodeZ - 1u) / kNodeZ);
 }

@@ -1793,44 +1793,104 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 5))) voi
 
 // PartialNode expansion (processVoxel<PartialNode>, src/voxelizer.cu:
 // 2997-3033; r = float(solid) from constructNodeList2, 1675, which erosion
-// leaves alone, so the bits are read from the pre-erosion copy): one thread
-// per node.  A surface node's winner key comes from the keygrid at the node's
-// position in its brick (as its material in matgrid); the ratio is computed for
-// the winner at the node's alloc coordinates.  A cleared partition border
-// keeps r = 0 (zeroPadding stores Node()).
+// leaves alone, so the bits are read from the pre-erosion copy).  A surface
+// node's winner key comes from the keygrid at the node's position in its
+// brick (as its material in matgrid); the ratio is computed for the winner at
+// the node's alloc coordinates.  A cleared partition border keeps r = 0
+// (zeroPadding stores Node()).
+//
+// A block takes kPartialWords words.  The cut volume is over a thousand
+// instructions and few nodes need it (about one in eight of a furnished
+// room's, mostly one or two per 32-voxel word of a wall), so the block first
+// lists its surface nodes in LDS and then computes their ratios with full
+// waves, where a thread per node ran the whole path for a few lanes; the
+// nodes are written once, two per lane.  Room at 2 cm (256x203x153 nodes,
+// 64 MB): 579 us with a thread per node, 265 us with the list, 82 us with
+// the cut polygons in registers too (vox_math.h), bound by the VALU work of
+// about a million cut volumes.
 __global__ __launch_bounds__(256) void k_nodes_partial(const Job *__restrict__ jobs, uint32_t j) {
+    __shared__ uint32_t s_bits[kPartialWords], s_surf[kPartialWords], s_key[kPartialWords];
+    __shared__ uint32_t s_pos[kPartialWords];
+    __shared__ uint32_t s_y[kPartialWords], s_z[kPartialWords];
+    __shared__ uint16_t s_queue[kPartialWords * 32];
+    __shared__ float s_ratio[kPartialWords * 32];
+    __shared__ uint32_t s_n;
     const Job &J = jobs[j];
     const GridDims g = J.gd;
     const BrickDims bd = J.bdn;
-    const size_t n = (size_t)g.X * g.Y * g.Z;
-    const VK_G uint16_t *ln = (const VK_G uint16_t *)gptr(J.nodes);
-    VK_G u32x2 *out = (VK_G u32x2 *)J.pnodes;
-    const VK_G uint32_t *bits = gptr(J.pbits);  // before erosion
-    const bool zbrd = J.zero_border != 0, mats = J.use_mats != 0, embed = J.embed != 0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t x = (uint32_t)(i % g.X), y = (uint32_t)((i / g.X) % g.Y);
-        const uint32_t z = (uint32_t)(i / ((size_t)g.X * g.Y));
-        const uint32_t w = x >> 5;
-        const uint32_t bit =
-            (bits[((size_t)z * g.Y + y) * g.W + w] >> (31u - (x & 31u))) & 1u;
-        float r = bit ? 1.0f : 0.0f;
-        if (mats && bit) {
-            const uint32_t b = brick_of_word(bd, w, y, z);
-            const size_t wi = ((size_t)z * g.Y + y) * g.W + w;
-            if (gptr(J.bhist)[b] && ((gptr(J.surf)[wi] >> (31u - (x & 31u))) & 1u)) {
-                const uint32_t lvox = bd.lwx + bd.lby + bd.lbz + 5u;  // log2 voxels per brick
-                const uint32_t key = gptr(J.keygrid)[((size_t)b << lvox) +
-                                                     (word_in_brick(bd, w, y, z) << 5) + (x & 31u)];
-                const uint32_t t = embed ? (key >> 8) & 0x3FFFFFu : key & 0x3FFFFFFFu;
-                const int32_t node[3] = {(int32_t)x, (int32_t)y, (int32_t)z};
-                r = partial_ratio(J.V, J.I, t, key >> 30, node, J.m, J.fd);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const bool mats = J.use_mats != 0, embed = J.embed != 0;
+    const uint32_t nwords = g.W * g.Y * g.Z;  // < 2^27: at most 2^32 nodes
+    const uint32_t wi0 = blockIdx.x * kPartialWords;
+    const uint32_t lvox = bd.lwx + bd.lby + bd.lbz + 5u;  // log2 voxels per brick
+    if (tid == 0) s_n = 0u;
+    static_assert(kPartialWords == kWave, "one wave loads the block's words");
+    if (tid < kPartialWords) {
+        const uint32_t wi = wi0 + tid;
+        uint32_t bits = 0u, surf = 0u, key = 0u, w = 0u, y = 0u, z = 0u;
+        if (wi < nwords) {
+            const uint32_t row = wi / g.W;
+            w = wi - row * g.W;
+            z = row / g.Y;
+            y = row - z * g.Y;
+            bits = gptr(J.pbits)[wi];  // before erosion
+            if (mats) {
+                const uint32_t b = brick_of_word(bd, w, y, z);
+                if (gptr(J.bhist)[b]) surf = gptr(J.surf)[wi] & bits;
+                // Word index in the keygrid: grids hold fewer than 2^32 voxels,
+                // brick padding at most doubles each axis.
+                key = (b << (lvox - 5u)) + word_in_brick(bd, w, y, z);
+            }
+            if (J.zero_border) {
+                uint32_t keep = y == 0u || y + 1u == g.Y || z == 0u || z + 1u == g.Z ? 0u : ~0u;
+                if (w == 0u) keep &= 0x7FFFFFFFu;
+                if (w + 1u == g.W) keep &= ~1u;
+                bits &= keep;
+                surf &= keep;
             }
         }
-        if (zbrd && (x == 0u || x + 1u == g.X || y == 0u || y + 1u == g.Y || z == 0u ||
-                     z + 1u == g.Z))
-            r = 0.0f;
-        out[i] = u32x2{(uint32_t)ln[i], __float_as_uint(r)};
+        s_bits[tid] = bits;
+        s_surf[tid] = surf;
+        s_key[tid] = key;
+        s_pos[tid] = w;
+        s_y[tid] = y;
+        s_z[tid] = z;
+    }
+    __syncthreads();
+    // The block's surface nodes, in no particular order.
+    for (uint32_t p = tid; p < kPartialWords * 32u; p += 256u) {
+        const bool on = ((s_surf[p >> 5] >> (31u - (p & 31u))) & 1u) != 0u;
+        const unsigned long long m = __ballot(on);
+        if (!m) continue;
+        uint32_t base = 0u;
+        if (lane == 0u) base = atomicAdd(&s_n, (uint32_t)__popcll(m));
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+            (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (on) s_queue[base + below] = (uint16_t)p;
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    for (uint32_t q = tid; q < n; q += 256u) {
+        const uint32_t p = s_queue[q], k = p >> 5, x = p & 31u;
+        const uint32_t key = gptr(J.keygrid)[((size_t)s_key[k] << 5) + x];
+        const uint32_t t = embed ? (key >> 8) & 0x3FFFFFu : key & 0x3FFFFFFFu;
+        const int32_t node[3] = {(int32_t)(s_pos[k] * 32u + x), (int32_t)s_y[k], (int32_t)s_z[k]};
+        s_ratio[p] = partial_ratio(J.V, J.I, t, key >> 30, node, J.m, J.fd);
+    }
+    __syncthreads();
+    const VK_G uint32_t *ln = (const VK_G uint32_t *)gptr(J.nodes);
+    VK_G u32x4 *out = (VK_G u32x4 *)J.pnodes;
+    const size_t h0 = (size_t)wi0 * 16u;  // first pair of nodes
+    const uint32_t halves = min(kPartialWords, nwords - wi0) * 16u;
+    for (uint32_t h = tid; h < halves; h += 256u) {
+        const uint32_t p = 2u * h, k = p >> 5, s = 31u - (p & 31u);
+        const uint32_t bits = s_bits[k], surf = s_surf[k];
+        const uint32_t two = ln[h0 + h];
+        const float r0 = (surf >> s) & 1u ? s_ratio[p] : (bits >> s) & 1u ? 1.0f : 0.0f;
+        const float r1 = (surf >> (s - 1u)) & 1u ? s_ratio[p + 1u]
+                         : (bits >> (s - 1u)) & 1u ? 1.0f : 0.0f;
+        out[h0 + h] = u32x4{two & 0xFFFFu, __float_as_uint(r0), two >> 16, __float_as_uint(r1)};
     }
 }
 

@@ -356,32 +356,76 @@ __device__ __forceinline__ F3 rot_y(F3 v, float s, float c) {
 __device__ __forceinline__ float len2f(float a, float b) { return sqrtf(a * a + b * b); }
 
 // Turns the polygon and the apex so that rotN points along z, then returns
-// the pyramid's volume (surveyor's formula times a third of the height).
-__device__ __noinline__ float turned_pyramid(F3 *poly, int n, F3 rotN, F3 apex) {
+// the pyramid's volume (surveyor's formula times a third of the height).  The
+// polygon is the points of pt with their `on` flag set, in order: with every
+// index a constant the points stay in registers, where a list with a running
+// count would live in scratch memory.
+__device__ __forceinline__ float turned_pyramid(const F3 (&pt)[6], const bool (&on)[6], F3 rotN,
+                                                F3 apex) {
     F3 h = apex;
-    if (rotN.y != 0.0f) {
-        const float pl = len2f(rotN.y, rotN.z), s = rotN.y / pl, c = rotN.z / pl;
-        h = rot_x(h, s, c);
-        for (int i = 0; i < n; i++) poly[i] = rot_x(poly[i], s, c);
-        rotN = rot_x(rotN, s, c);
+    float sx = 0.0f, cx = 0.0f, sy = 0.0f, cy = 0.0f;
+    const bool turn_x = rotN.y != 0.0f;
+    if (turn_x) {
+        const float pl = len2f(rotN.y, rotN.z);
+        sx = rotN.y / pl;
+        cx = rotN.z / pl;
+        h = rot_x(h, sx, cx);
+        rotN = rot_x(rotN, sx, cx);
     }
-    if (rotN.x != 0.0f) {
-        const float pl = len2f(rotN.z, rotN.x), s = -rotN.x / pl, c = rotN.z / pl;
-        h = rot_y(h, s, c);
-        for (int i = 0; i < n; i++) poly[i] = rot_y(poly[i], s, c);
+    const bool turn_y = rotN.x != 0.0f;
+    if (turn_y) {
+        const float pl = len2f(rotN.z, rotN.x);
+        sy = -rotN.x / pl;
+        cy = rotN.z / pl;
+        h = rot_y(h, sy, cy);
     }
-    float area = 0.0f;
-    for (int i = 0; i < n; i++) {
-        const F3 a = poly[i], b = poly[(i + 1) % n];
-        area += 0.5f * (a.x * b.y - b.x * a.y);
+    float area = 0.0f, z0 = 0.0f;  // an empty polygon keeps area 0 and height h.z
+    F3 first = {0.0f, 0.0f, 0.0f}, prev = first;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        if (!on[i]) continue;
+        F3 q = pt[i];
+        if (turn_x) q = rot_x(q, sx, cx);
+        if (turn_y) q = rot_y(q, sy, cy);
+        if (any)
+            area += 0.5f * (prev.x * q.y - q.x * prev.y);
+        else {
+            first = q;
+            z0 = q.z;
+        }
+        prev = q;
+        any = true;
     }
-    return fabsf((1.0f / 3.0f) * area * (h.z - poly[0].z));
+    if (any) area += 0.5f * (prev.x * first.y - first.x * prev.y);
+    return fabsf((1.0f / 3.0f) * area * (h.z - z0));
+}
+
+// Volume of the pyramid over one face of the cut box (nothing for fewer than
+// three points); the normal comes from its first three points.
+__device__ __forceinline__ void face_pyramid(const F3 (&pt)[6], const bool (&on)[6], F3 apex,
+                                             float &vol) {
+    F3 p[3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+        if (on[i]) {
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                if (n == k) p[k] = pt[i];
+            n++;
+        }
+    if (n > 2) {
+        const F3 e = fcross(fsub(p[0], p[2]), fsub(p[1], p[0]));
+        const float inv = 1.0f / sqrtf(fdot3(e, e));
+        vol += turned_pyramid(pt, on, F3{e.x * inv, e.y * inv, e.z * inv}, apex);
+    }
 }
 
 // Volume the reference computes for the box centred at m + d * node, cut by
 // the plane through t0 with normal n (the part the normal points into for
 // a plane through the box).
-__device__ __noinline__ float cut_volume(F3 t0, const int32_t node[3], F3 n, F3 m, float d) {
+__device__ __forceinline__ float cut_volume(F3 t0, const int32_t node[3], F3 n, F3 m, float d) {
     const F3 vc = fadd3(m, fscale3(d, F3{float(node[0]), float(node[1]), float(node[2])}));
     if (fabsf(n.x) == 1.0f) return (d * d) * ((d / 2.0f) + t0.x - vc.x);
     if (fabsf(n.y) == 1.0f) return (d * d) * ((d / 2.0f) + t0.y - vc.y);
@@ -404,59 +448,69 @@ __device__ __noinline__ float cut_volume(F3 t0, const int32_t node[3], F3 n, F3 
     v[5] = fadd3(v[2], dx);
     v[6] = fadd3(v[3], dy);
     v[7] = fadd3(v[4], dy);
-    // Three paths from v0 (edges (0,a), (a,b), (b,7) and (a,c)) build the cut
-    // polygon and faces 1-3; the arrays start zeroed (an empty cut polygon
-    // still reads its first entry's z).
-    F3 ip[6], face[3][6];
-    for (int i = 0; i < 6; i++) {
-        ip[i] = F3{0.0f, 0.0f, 0.0f};
-        for (int f = 0; f < 3; f++) face[f][i] = F3{0.0f, 0.0f, 0.0f};
-    }
-    int ni = 0, nf[3] = {0, 0, 0};
-    const int pa[3] = {1, 2, 3}, pb[3] = {4, 5, 6}, pc[3] = {5, 6, 4}, partner[3] = {2, 0, 1};
+    // Three paths from v0 (edges (0,a), (a,b), (b,7) and (a,c)).  Path k's
+    // first crossed edge among the first three is `hit` (0, 1, 2; 3 if none),
+    // crossed at ip; qp is the crossing of (a,c), if `cut`.
+    constexpr int pa[3] = {1, 2, 3}, pb[3] = {4, 5, 6}, pc[3] = {5, 6, 4};
+    F3 ip[3], qp[3];
+    int hit[3];
+    bool cut[3];
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-        const int a = pa[k], b = pb[k], c = pc[k], f = k, g = partner[k];
-        float t = fdot3(n, fsub(t0, v[0])) / fdot3(n, fsub(v[a], v[0]));
+        const F3 va = v[pa[k]], vb = v[pb[k]], vc2 = v[pc[k]];
+        ip[k] = F3{0.0f, 0.0f, 0.0f};
+        qp[k] = ip[k];
+        float t = fdot3(n, fsub(t0, v[0])) / fdot3(n, fsub(va, v[0]));
         if (t < 0.0f || t > 1.0f) {
-            face[f][nf[f]++] = v[a];
-            t = fdot3(n, fsub(t0, v[a])) / fdot3(n, fsub(v[b], v[a]));
+            t = fdot3(n, fsub(t0, va)) / fdot3(n, fsub(vb, va));
             if (t < 0.0f || t > 1.0f) {
-                t = fdot3(n, fsub(t0, v[b])) / fdot3(n, fsub(v[7], v[b]));
+                t = fdot3(n, fsub(t0, vb)) / fdot3(n, fsub(v[7], vb));
+                hit[k] = 3;
                 if (t >= 0.0f && t <= 1.0f) {
-                    ip[ni] = fadd3(v[b], fscale3(t, fsub(v[7], v[b])));
-                    face[f][nf[f]++] = v[b];
-                    face[f][nf[f]++] = ip[ni];
-                    face[g][nf[g]++] = ip[ni];
-                    face[g][nf[g]++] = v[b];
-                    ni++;
-                } else {
-                    face[f][nf[f]++] = v[b];
-                    face[g][nf[g]++] = v[b];
+                    hit[k] = 2;
+                    ip[k] = fadd3(vb, fscale3(t, fsub(v[7], vb)));
                 }
             } else {
-                ip[ni] = fadd3(v[a], fscale3(t, fsub(v[b], v[a])));
-                face[f][nf[f]++] = ip[ni];
-                ni++;
+                hit[k] = 1;
+                ip[k] = fadd3(va, fscale3(t, fsub(vb, va)));
             }
         } else {
-            ip[ni] = fadd3(v[0], fscale3(t, fsub(v[a], v[0])));
-            ni++;
+            hit[k] = 0;
+            ip[k] = fadd3(v[0], fscale3(t, fsub(va, v[0])));
         }
-        t = fdot3(n, fsub(t0, v[a])) / fdot3(n, fsub(v[c], v[a]));
-        if (t >= 0.0f && t <= 1.0f) {
-            ip[ni] = fadd3(v[a], fscale3(t, fsub(v[c], v[a])));
-            face[f][nf[f]++] = ip[ni];
-            ni++;
-        }
+        t = fdot3(n, fsub(t0, va)) / fdot3(n, fsub(vc2, va));
+        cut[k] = t >= 0.0f && t <= 1.0f;
+        if (cut[k]) qp[k] = fadd3(va, fscale3(t, fsub(vc2, va)));
     }
+    // The cut polygon: each path's crossings in path order.
     float vol = 0.0f;
-    vol += turned_pyramid(ip, ni, n, v[0]);
-    for (int f = 0; f < 3; f++)
-        if (nf[f] > 2) {
-            const F3 e = fcross(fsub(face[f][0], face[f][2]), fsub(face[f][1], face[f][0]));
-            const float inv = 1.0f / sqrtf(fdot3(e, e));
-            vol += turned_pyramid(face[f], nf[f], F3{e.x * inv, e.y * inv, e.z * inv}, v[0]);
+    {
+        const F3 pt[6] = {ip[0], qp[0], ip[1], qp[1], ip[2], qp[2]};
+        const bool on[6] = {hit[0] < 3, cut[0], hit[1] < 3, cut[1], hit[2] < 3, cut[2]};
+        vol += turned_pyramid(pt, on, n, v[0]);
+    }
+    // Face f: its own path's corners up to the crossing, the crossing and the
+    // one of (a,c); and from the path whose third edge it shares (path 1 for
+    // face 0, 2 for 1, and 0, walked before its own, for 2) that edge's
+    // crossing and corner.
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        const int o = f == 2 ? 0 : f + 1;
+        const F3 own[4] = {v[pa[f]], v[pb[f]], ip[f], qp[f]};
+        const bool own_on[4] = {hit[f] >= 1, hit[f] >= 2, hit[f] == 1 || hit[f] == 2, cut[f]};
+        const F3 sh[2] = {ip[o], v[pb[o]]};
+        const bool sh_on[2] = {hit[o] == 2, hit[o] >= 2};
+        F3 pt[6];
+        bool on[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            const bool mine = f == 2 ? i >= 2 : i < 4;
+            const int q = f == 2 ? (mine ? i - 2 : i) : (mine ? i : i - 4);
+            pt[i] = mine ? own[q & 3] : sh[q & 1];
+            on[i] = mine ? own_on[q & 3] : sh_on[q & 1];
         }
+        face_pyramid(pt, on, v[0], vol);
+    }
     return vol;
 }
 

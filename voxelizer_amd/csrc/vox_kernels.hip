@@ -1501,6 +1501,9 @@ __global__ __launch_bounds__(256) void k_erode(const Job *__restrict__ jobs,
 // ---------------------------------------------------------------------------
 // Node writing
 // ---------------------------------------------------------------------------
+// 16-byte slots between the pieces of a word in a wave's staging run: 64 lanes
+// plus a shift of 16 LDS banks.
+constexpr uint32_t kStagePitch = kWave + 4u;
 // Buffer offset past every range used below: loads there return 0 and
 // stores there are dropped (raw buffer range check, offset >= size).
 constexpr uint32_t kOob = 0x80000000u;
@@ -1519,16 +1522,47 @@ __device__ __forceinline__ void st128(Rsrc r, uint32_t off, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, 0);
 }
 
-// Nibble n (bit i = voxel i) -> 4 bytes holding 27 where the bit is set.
-// The multiply moves bit i to bit 8i (its four partial products occupy
-// disjoint bits, so nothing carries); 27 = 0b11011 is then two shifted ORs.
-// The empty asm keeps them apart: folded together they become one 32-bit
-// multiply by 27, which issues at a quarter of the rate of the two ORs.
-__device__ __forceinline__ uint32_t nibble_27(uint32_t n) {
-    const uint32_t s = __umul24(n, 0x204081u) & 0x01010101u;
-    uint32_t t = s | (s << 1);
-    __asm__("" : "+v"(t));
-    return t | (t << 3);
+// (m & a) | (~m & b): one v_bfi_b32.
+__device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
+    return (m & a) | (~m & b);
+}
+// Exchanges the bits of a above each group of kS bits with the bits of b
+// below them: one step of a bit-matrix transpose (kM: the low kS bits of
+// every 2 kS).
+template <uint32_t kS, uint32_t kM>
+__device__ __forceinline__ void swap_bits(uint32_t &a, uint32_t &b) {
+    const uint32_t t = bfi(kM, a, b << kS);
+    b = bfi(kM, a >> kS, b);
+    a = t;
+}
+// Id bytes of a word's 32 voxels (four per dword, voxel order; voxel i at bit
+// 31 - i of the planes): the five bit planes, padded to eight, are transposed
+// as four 8x8 bit matrices side by side (bytes of the words), then the bytes
+// are put in voxel order.  61 operations for any number of boundary voxels.
+__device__ __forceinline__ void id_bytes(const IdPlanes &o, uint32_t idw[8]) {
+    uint32_t r[8] = {o.b[0], o.b[1], o.b[2], o.b[3], o.b[4], 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 4; i++) swap_bits<4, 0x0F0F0F0Fu>(r[i], r[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        swap_bits<2, 0x33333333u>(r[i], r[i + 2]);
+        swap_bits<2, 0x33333333u>(r[i + 4], r[i + 6]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) swap_bits<1, 0x55555555u>(r[i], r[i + 1]);
+    // r[j] byte k: the id of bit position 8 k + j.
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const uint32_t a = r[7 - 4 * h], b = r[6 - 4 * h], c = r[5 - 4 * h], d = r[4 - 4 * h];
+        const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u);
+        const uint32_t ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+        const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u);
+        const uint32_t cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+        idw[6 + h] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+        idw[4 + h] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+        idw[2 + h] = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+        idw[0 + h] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+    }
 }
 
 // Cartesian node write: a block takes kChunk consecutive words of a plane
@@ -1542,12 +1576,14 @@ __device__ __forceinline__ uint32_t nibble_27(uint32_t n) {
 // adjacent lanes.
 //
 // A word whose 32 voxels are all empty or all fully surrounded (the bulk of
-// a grid) is stored as a constant.  Otherwise the fully surrounded voxels
-// get id 27 by a nibble spread, boundary voxels (solid, some neighbour
-// missing) get the id of their neighbour permutation from the bit-sliced
-// table (orient_planes), patched byte-wise into the thread's LDS slot, and
-// surface voxels OR in their material (bytes of the word's other voxels are
-// 0 in the material grid).
+// a grid) is stored as a constant.  Otherwise the bit planes of the ids come
+// from the bit-sliced table (orient_planes; all six neighbours give id 27)
+// and are transposed into bytes in registers (id_bytes), and surface voxels
+// OR in their material (bytes of the word's other voxels are 0 in the
+// material grid).  The transpose replaced a loop over the boundary voxels
+// that patched their bytes in LDS: room at 1 cm (512x403x303 LongNodes) 38.9
+// -> 31.2 us, hall (1536x1024x768 ShortNodes) 385 -> 362 us, there bound by
+// its 1.7 GB of reads and writes (4.8 TB/s, where a large copy runs at 5.0).
 //
 // With several erosion subspaces (voxSplitRes y/z smaller than the grid) the
 // reference computes a subspace's ids before later subspaces erode
@@ -1561,9 +1597,10 @@ __device__ __forceinline__ void nodes_cart(const Job *__restrict__ jobs,
                                            uint32_t njobs, const uint32_t *__restrict__ pre,
                                            const uint8_t *__restrict__ ystart,
                                            const uint8_t *__restrict__ zstart) {
-    // Per wave 4 KB: the id bytes of each thread's word while boundary ids go
-    // in (32 B per thread), then the wave's node run on its way out.
-    __shared__ uint4 stage[256 * 4];
+    // A wave's node run of one plane on its way out: the 16-byte pieces of a
+    // word kStagePitch apart, so that lanes write consecutive slots and the
+    // pieces of neighbouring words read back from other banks.
+    __shared__ uint4 stage[256 / kWave][4 * kStagePitch];
     const uint32_t GL = xcd_logical_block(node_bases[njobs]);  // bases[njobs] = all blocks
     if (GL == UINT32_MAX) return;  // uniform over the block
     const Job &J = jobs[job_of(node_bases, njobs, GL)];
@@ -1670,8 +1707,7 @@ __device__ __forceinline__ void nodes_cart(const Job *__restrict__ jobs,
     const uint32_t nbw = kind == 0 ? 32u : 64u;  // node bytes per word
     VK_G uint8_t *nodes = (VK_G uint8_t *)gptr(J.nodes);
     const uint32_t lane = tx;
-    uint4 *wst = &stage[(tid - lane) * 4u];  // this wave's staging run
-    uint8_t *sb = (uint8_t *)&wst[2u * lane];
+    uint4 *wst = stage[tid / kWave];  // this wave's staging run
     // The wave's 64 words are consecutive, so its nodes of a plane are one
     // run (2 KB ShortNode, 4 KB LongNode) starting at byte wrun: staged in
     // LDS in node order and stored lane by lane, each store writes 1 KB of
@@ -1706,31 +1742,14 @@ __device__ __forceinline__ void nodes_cart(const Job *__restrict__ jobs,
 #pragma unroll
             for (int j = 0; j < 8; j++) idw[j] = v;
         } else {
-            const uint32_t ir = __brev(interior);  // bit i = voxel i
+            // A model rotated about z (x slices) takes its ids in the
+            // un-rotated frame: its -x/+x are the rotated -y/+y, its -y/+y
+            // the rotated +x/-x.
+            IdPlanes op = rot ? orient_planes(Yn, Yp, R, L, Zn, Zp)
+                              : orient_planes(L, R, Yn, Yp, Zn, Zp);
 #pragma unroll
-            for (int j = 0; j < 8; j++) idw[j] = nibble_27((ir >> (4 * j)) & 15u);
-            if (bnd) {
-                // A model rotated about z (x slices) takes its ids in the
-                // un-rotated frame: its -x/+x are the rotated -y/+y, its -y/+y
-                // the rotated +x/-x.
-                const IdPlanes op = rot ? orient_planes(Yn, Yp, R, L, Zn, Zp)
-                                        : orient_planes(L, R, Yn, Yp, Zn, Zp);
-                wst[2u * lane] = make_uint4(idw[0], idw[1], idw[2], idw[3]);
-                wst[2u * lane + 1u] = make_uint4(idw[4], idw[5], idw[6], idw[7]);
-                uint32_t m = bnd;
-                while (m) {
-                    const uint32_t s = 31u - (uint32_t)__clz(m);  // voxel 31 - s
-                    const uint32_t id = ((op.b[0] >> s) & 1u) | (((op.b[1] >> s) & 1u) << 1) |
-                                        (((op.b[2] >> s) & 1u) << 2) |
-                                        (((op.b[3] >> s) & 1u) << 3) |
-                                        (((op.b[4] >> s) & 1u) << 4);
-                    sb[31u - s] = (uint8_t)id;
-                    m ^= 1u << s;
-                }
-                const uint4 q0 = wst[2u * lane], q1 = wst[2u * lane + 1u];
-                idw[0] = q0.x; idw[1] = q0.y; idw[2] = q0.z; idw[3] = q0.w;
-                idw[4] = q1.x; idw[5] = q1.y; idw[6] = q1.z; idw[7] = q1.w;
-            }
+            for (int j = 0; j < 5; j++) op.b[j] &= G;
+            id_bytes(op, idw);
         }
         const uint32_t md[8] = {ma[k].x, ma[k].y, ma[k].z, ma[k].w,
                                 mb[k].x, mb[k].y, mb[k].z, mb[k].w};
@@ -1747,13 +1766,14 @@ __device__ __forceinline__ void nodes_cart(const Job *__restrict__ jobs,
             for (int j = 0; j < 8; j++) out[j] = (idw[j] | ((md[j] << 5) & 0xE0E0E0E0u)) & all;
             if (x0) out[0] &= 0xFFFFFF00u;
             if (x1) out[7] &= 0x00FFFFFFu;
-            wst[2u * lane] = make_uint4(out[0], out[1], out[2], out[3]);
-            wst[2u * lane + 1u] = make_uint4(out[4], out[5], out[6], out[7]);
+            wst[lane] = make_uint4(out[0], out[1], out[2], out[3]);
+            wst[kStagePitch + lane] = make_uint4(out[4], out[5], out[6], out[7]);
             wave_lds_sync();
 #pragma unroll
             for (uint32_t q = 0; q < 2u; q++) {
-                const uint4 v = wst[q * kWave + lane];
-                st128(nr, wrun + (q * kWave + lane) * 16u, u32x4{v.x, v.y, v.z, v.w});
+                const uint32_t piece = q * kWave + lane;
+                const uint4 v = wst[(piece & 1u) * kStagePitch + (piece >> 1)];
+                st128(nr, wrun + piece * 16u, u32x4{v.x, v.y, v.z, v.w});
             }
         } else {  // LongNode halfword: id | material << 8
             uint32_t out[16];
@@ -1766,12 +1786,14 @@ __device__ __forceinline__ void nodes_cart(const Job *__restrict__ jobs,
             if (x1) out[15] &= 0x0000FFFFu;
 #pragma unroll
             for (uint32_t q = 0; q < 4u; q++)
-                wst[4u * lane + q] = make_uint4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+                wst[q * kStagePitch + lane] =
+                    make_uint4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
             wave_lds_sync();
 #pragma unroll
             for (uint32_t q = 0; q < 4u; q++) {
-                const uint4 v = wst[q * kWave + lane];
-                st128(nr, wrun + (q * kWave + lane) * 16u, u32x4{v.x, v.y, v.z, v.w});
+                const uint32_t piece = q * kWave + lane;
+                const uint4 v = wst[(piece & 3u) * kStagePitch + (piece >> 2)];
+                st128(nr, wrun + piece * 16u, u32x4{v.x, v.y, v.z, v.w});
             }
         }
         wave_lds_sync();  // the run is read out before the next plane's writes

@@ -509,9 +509,9 @@ vox_status split_table(vox_ctx *ctx, const uint32_t res[3], const uint32_t matSp
     return VOX_OK;
 }
 
-// The FCC interleave and the PartialNode expansion read surface bit words;
-// the Cartesian node pass reads only the per-brick word masks.
-inline bool job_needs_surf(const Job &J) { return J.pnodes != nullptr || J.kind >= 3; }
+// The PartialNode expansion reads surface bit words; the node passes read only
+// the per-brick word masks.
+inline bool job_needs_surf(const Job &J) { return J.pnodes != nullptr; }
 
 // Adds one grid with layout L; shift is the FCC sub-grid offset (zero for
 // Cartesian).  cart: the job gets erosion and Cartesian node blocks.
@@ -599,9 +599,8 @@ vox_status add_job(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, uin
     P.surf_off.push_back(P.surf_words);
     P.mat_off.push_back(P.mat_bytes);
     if (use_mats) {
-        // Surface bit words in the layout of the solid grid (for the FCC and
-        // PartialNode passes); one material byte per brick voxel,
-        // brick-major.
+        // Surface bit words in the layout of the solid grid (for the
+        // PartialNode pass); one material byte per brick voxel, brick-major.
         if (job_needs_surf(J)) P.surf_words += words;
         P.mat_bytes += (size_t)nbt * (size_t)(bdim[0] * bdim[1] * bdim[2]);
         P.any_mats = true;
@@ -1178,7 +1177,7 @@ vox_status node_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, const uint3
         VOX_HIP(hipGetLastError());
     }
     if (nf > 0) {
-        k_nodes_fcc<<<xcd_grid(P.fcc_b.back()), dim3(kWave, 4), 0, ctx->stream>>>(
+        k_nodes_fcc<<<xcd_grid(P.fcc_b.back()), 256, 0, ctx->stream>>>(
             D.jobs, D.fcc_first, D.fcc_b, nf);
         VOX_HIP(hipGetLastError());
     }

@@ -44,19 +44,6 @@ __device__ __forceinline__ uint32_t xcd_logical_block(uint32_t n) {
 }
 inline uint32_t xcd_grid(uint32_t n) { return kXcds * ((n + kXcds - 1) / kXcds); }
 
-// Logical row block -> (word chunk, 4-row group, plane).
-struct RowBlock {
-    uint32_t xc, y4, z;
-};
-__device__ __forceinline__ RowBlock row_block(uint32_t L, uint32_t nxc, uint32_t ny4) {
-    RowBlock r;
-    r.xc = L % nxc;
-    const uint32_t q = L / nxc;
-    r.y4 = q % ny4;
-    r.z = q / ny4;
-    return r;
-}
-
 // Plane-linear blocks of the erosion and Cartesian node passes: the words of
 // a plane are numbered i = y * W + w and cut into chunks of kChunk
 // consecutive words; a 256-thread block takes one chunk over a group of
@@ -158,7 +145,7 @@ struct Job {
     uint32_t brick_base;   // first brick
     BrickDims bdn;         // brick geometry for the node passes
     const SplitTable *splits;  // matSplitRes intervals
-    uint32_t *surf;        // surface bit words (the layout of bits); FCC and PartialNode only
+    uint32_t *surf;        // surface bit words (the layout of bits); PartialNode only
     const uint32_t *bhist; // per brick: (triangle, brick) pairs; 0 = not visited
     uint32_t *wmask;       // per brick, 4 words: bit i set where brick word i holds a surface voxel
     uint8_t *matgrid;      // per voxel, brick-major: winner material (surface words)
@@ -490,20 +477,6 @@ __host__ __device__ inline IdPlanes orient_planes(uint32_t mx, uint32_t px, uint
     return o;
 }
 
-// Surface data of one grid as the node passes read it.  Brick b's voxels
-// occupy bytes [b * nvox, (b + 1) * nvox) of matgrid in the brick's word
-// order (z, y, x-word), 32 bytes per word.  A word that holds a surface
-// voxel has all 32 bytes written in the call (0 for its other voxels); the
-// rest may be stale.  Bricks the surface pass did not visit (bhist == 0)
-// hold stale surface words, so the readers check bhist first.
-struct MatSource {
-    const VK_G uint32_t *surf;   // surface bit words (same layout as bits)
-    const VK_G uint32_t *bhist;  // per brick: nonzero if visited
-    const VK_G uint8_t *matgrid;
-};
-__device__ __forceinline__ MatSource mat_source(const Job &J) {
-    return MatSource{gptr(J.surf), gptr(J.bhist), gptr(J.matgrid)};
-}
 // Index of word (w, y, z) of a grid within its brick's block of words, and
 // the brick: brick-major, words in (z, y, x-word) order inside a brick.
 __device__ __forceinline__ uint32_t brick_of_word(const BrickDims &bd, uint32_t w, uint32_t y,
@@ -540,8 +513,17 @@ inline uint32_t node_blocks(const GridDims &g) {
 }
 __global__ void k_nodes_fcc(const Job *__restrict__ jobs, const uint32_t *__restrict__ fcc_first,
                             const uint32_t *__restrict__ fcc_bases, uint32_t nfcc);
+// FCC planes per thread (even: a thread's planes start at an even one), FCC
+// words a wave writes per plane (its end lanes hold the neighbours) and the
+// 16-byte slots between a word's pieces in its staging run (64 lanes plus a
+// shift of 8 LDS banks).
+constexpr uint32_t kFccZ = 2, kFccRun = kWave - 2, kFccPitch = kWave + 2;
+static_assert(kFccZ % 2 == 0, "plane k of a thread has the parity of k");
+__host__ __device__ __forceinline__ uint32_t fcc_chunks(const GridDims &g) {
+    return (2u * g.W * g.Y + 4u * kFccRun - 1u) / (4u * kFccRun);
+}
 inline uint32_t fcc_node_blocks(const GridDims &g) {
-    return ((2u * g.W + kWave - 1u) / kWave) * ((g.Y + 3u) / 4u) * 2u * g.Z;
+    return fcc_chunks(g) * ((2u * g.Z + kFccZ - 1u) / kFccZ);
 }
 
 // Cost model kernels (vox_cost.hip).

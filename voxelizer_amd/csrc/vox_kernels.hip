@@ -1919,197 +1919,229 @@ __global__ __launch_bounds__(256) void k_nodes_partial(const Job *__restrict__ j
 // ---------------------------------------------------------------------------
 // FCC nodes
 // ---------------------------------------------------------------------------
-// Spreads 16 bits to the even positions: bit j -> bit 2j.
-__device__ __forceinline__ uint32_t spread16(uint32_t x) {
-    x &= 0xFFFFu;
-    x = (x | (x << 8)) & 0x00FF00FFu;
-    x = (x | (x << 4)) & 0x0F0F0F0Fu;
-    x = (x | (x << 2)) & 0x33333333u;
-    x = (x | (x << 1)) & 0x55555555u;
-    return x;
+// 32 FCC nodes of one row: even x from the sub-grid with x shift 0 (word e),
+// odd x from the one with x shift d/2 (word o), 16 voxels of each
+// (convertToFCCGrid, src/voxelizer.cu:1756-1772).  half picks the 16: the
+// bytes are laid out e o e o by one v_perm_b32, then the bits inside each
+// 16-bit half are interleaved (a perfect shuffle).
+__device__ __forceinline__ uint32_t fcc_word(uint32_t e, uint32_t o, uint32_t half) {
+    uint32_t x = __builtin_amdgcn_perm(e, o, half);  // e1 o1 e0 o0
+    x = (x & 0xF00FF00Fu) | ((x & 0x00F000F0u) << 4) | ((x >> 4) & 0x00F000F0u);
+    x = (x & 0xC3C3C3C3u) | ((x & 0x0C0C0C0Cu) << 2) | ((x >> 2) & 0x0C0C0C0Cu);
+    return (x & 0x99999999u) | ((x & 0x22222222u) << 1) | ((x >> 1) & 0x22222222u);
 }
 
-struct FccGrids {
-    const VK_G uint32_t *s[4];  // per-grid solid|surface bits (grid 1..4)
-};
-
-// 32 FCC nodes of row (y, fz), x in [32*fw, 32*fw+32): even x from the
-// sub-grid with x shift 0, odd x from the one with x shift d/2
-// (convertToFCCGrid, src/voxelizer.cu:1756-1772).
-__device__ __forceinline__ uint32_t fcc_word(const FccGrids &G, const GridDims &g, int64_t fw,
-                                             int64_t y, int64_t fz) {
-    if (fw < 0 || fw >= (int64_t)(2 * g.W) || y < 0 || y >= (int64_t)g.Y || fz < 0 ||
-        fz >= (int64_t)(2 * g.Z))
-        return 0u;
-    const int odd = (int)(fz & 1);
-    // Picked by arithmetic: a select between elements of the pointer array
-    // becomes a computed index, which puts the array in scratch.
-    const uintptr_t e0 = (uintptr_t)G.s[0], o0 = (uintptr_t)G.s[1];
-    const uintptr_t k = (uintptr_t)odd;
-    const VK_G uint32_t *ge = (const VK_G uint32_t *)(e0 + k * ((uintptr_t)G.s[2] - e0));
-    const VK_G uint32_t *go = (const VK_G uint32_t *)(o0 + k * ((uintptr_t)G.s[3] - o0));
-    const size_t wi = ((size_t)(fz >> 1) * g.Y + (size_t)y) * g.W + (size_t)(fw >> 1);
-    const int sh = (fw & 1) ? 0 : 16;
-    const uint32_t e = (ge[wi] >> sh) & 0xFFFFu, o = (go[wi] >> sh) & 0xFFFFu;
-    return (spread16(e) << 1) | spread16(o);
-}
-
-// Left/right shifted FCC row words: neighbours at x-1 / x+1 (the word of the
-// adjacent lane supplies the carried bit).
-__device__ __forceinline__ void lr_shift(const FccGrids &G, const GridDims &g, uint32_t word,
-                                         int64_t fw, int64_t y, int64_t fz, uint32_t &Lw,
-                                         uint32_t &Rw) {
-    const uint32_t tx = threadIdx.x;
-    uint32_t prev = (uint32_t)__shfl_up((int)word, 1);
-    uint32_t next = (uint32_t)__shfl_down((int)word, 1);
-    if (tx == 0) prev = fcc_word(G, g, fw - 1, y, fz);
-    if (tx == kWave - 1) next = fcc_word(G, g, fw + 1, y, fz);
-    Lw = (word >> 1) | (prev << 31);
-    Rw = (word << 1) | (next >> 31);
-}
-
-// FCC node write, row-major like k_nodes_cart: the 12-bit neighbour mask of
-// calculateFCCBoundaries (src/voxelizer.cu:1930-2048) as bitwise selects by
-// the (x+z) parity mask, materials from the four sub-grids' surface lists.
+// FCC node write: the 12-bit neighbour mask of calculateFCCBoundaries
+// (src/voxelizer.cu:1930-2048) as bitwise selects by the (x+z) parity mask,
+// materials from the four sub-grids' material grids.
+//
+// Plane-linear like the Cartesian pass: the FCC words of a plane are numbered
+// i = y * FW + fw, a wave takes kFccRun consecutive ones over kFccZ planes,
+// its first and last lane hold the words before and after the run (so every
+// x neighbour comes from an adjacent lane) and write nothing.  The words of a
+// plane's three rows are interleaved from the sub-grids once and serve as the
+// plane itself and as its neighbours' neighbour.  The twelve neighbour words
+// of 32 nodes are turned into node masks by a bit-matrix transpose in
+// registers (144 operations whatever the number of boundary nodes), and the
+// wave's nodes go through LDS so that each store writes 1 KB of whole lines.
+// Room at 1.6 cm (640x255x384 LongFCCNodes, 251 MB): 54 us, 4.7 TB/s of node
+// writes; a wave per 64 words of one row (20 of them there), nine interleaved
+// words per plane and a loop over the boundary nodes took 163 us.
 __global__ __launch_bounds__(256) void k_nodes_fcc(const Job *__restrict__ jobs,
                                                    const uint32_t *__restrict__ fcc_first,
                                                    const uint32_t *__restrict__ fcc_bases,
                                                    uint32_t nfcc) {
-    __shared__ uint4 fslot[256][4];  // 32 node masks (u16) per thread while boundary ids go in
+    __shared__ uint4 stage[256 / kWave][8 * kFccPitch];
     const uint32_t GL = xcd_logical_block(fcc_bases[nfcc]);  // bases[nfcc] = all blocks
     if (GL == UINT32_MAX) return;
     const uint32_t f = job_of(fcc_bases, nfcc, GL);
     const Job *__restrict__ Js = jobs + fcc_first[f];
     const GridDims g = Js[0].gd;
     const int use_mats = Js[0].use_mats, kind = Js[0].kind;
-    VK_G void *__restrict__ nodes = gptr(Js[0].nodes);
     const BrickDims bd = Js[0].bdn;
-    const VK_G uint32_t *s1 = gptr(Js[0].bits), *s2 = gptr(Js[1].bits), *s3 = gptr(Js[2].bits),
-                        *s4 = gptr(Js[3].bits);
-    const uint32_t FW = 2 * g.W, FY = g.Y;
-    const uint32_t nxc = (FW + kWave - 1) / kWave, ny4 = (FY + 3) / 4;
+    const uint32_t FW = 2u * g.W, P = FW * g.Y, FZ = 2u * g.Z;
+    const uint32_t nch = fcc_chunks(g);
     const uint32_t L = GL - fcc_bases[f];  // block within the lattice
-    const RowBlock rb = row_block(L, nxc, ny4);
-    const int64_t fw = (int64_t)rb.xc * kWave + threadIdx.x;
-    const int64_t y = (int64_t)rb.y4 * 4 + threadIdx.y;
-    const int64_t fz = rb.z;
-    const bool valid = fw < (int64_t)FW && y < (int64_t)FY;
-    FccGrids G{{s1, s2, s3, s4}};
-    // All lanes take part in the shuffles; invalid lanes hold zero words.
-    auto word = [&](int64_t yy, int64_t zz) { return valid ? fcc_word(G, g, fw, yy, zz) : 0u; };
-    const uint32_t M0 = word(y, fz), Mm = word(y - 1, fz), Mp = word(y + 1, fz);
-    const uint32_t D0 = word(y, fz - 1), Dm = word(y - 1, fz - 1), Dp = word(y + 1, fz - 1);
-    const uint32_t U0 = word(y, fz + 1), Um = word(y - 1, fz + 1), Up = word(y + 1, fz + 1);
-    uint32_t LD0, RD0, LMm, RMm, LM0, RM0, LMp, RMp, LU0, RU0;
-    lr_shift(G, g, D0, fw, y, fz - 1, LD0, RD0);
-    lr_shift(G, g, Mm, fw, y - 1, fz, LMm, RMm);
-    lr_shift(G, g, M0, fw, y, fz, LM0, RM0);
-    lr_shift(G, g, Mp, fw, y + 1, fz, LMp, RMp);
-    lr_shift(G, g, U0, fw, y, fz + 1, LU0, RU0);
-    if (!valid) return;
-    const uint32_t E = (fz & 1) ? 0x55555555u : 0xAAAAAAAAu;  // (x+z) even
-    const uint32_t NE = ~E;
-    uint32_t n[12];
-    n[0] = (E & Dm) | (NE & D0);
-    n[1] = LD0;
-    n[2] = RD0;
-    n[3] = (E & D0) | (NE & Dp);
-    n[4] = (E & LMm) | (NE & LM0);
-    n[5] = (E & RMm) | (NE & RM0);
-    n[6] = (E & LM0) | (NE & LMp);
-    n[7] = (E & RM0) | (NE & RMp);
-    n[8] = (E & Um) | (NE & U0);
-    n[9] = LU0;
-    n[10] = RU0;
-    n[11] = (E & U0) | (NE & Up);
-    uint32_t interior = M0;
+    const uint32_t lane = lane_id();
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const uint32_t base = (L % nch) * (kFccRun * 4u) + wave * kFccRun;  // first word of the run
+    const uint32_t z0 = (L / nch) * kFccZ;                              // first FCC plane
+    const uint32_t i = base + lane - 1u;  // UINT32_MAX before the first word
+    const bool valid = i < P;
+    const uint32_t y = valid ? i / FW : 0u, fw = valid ? i - y * FW : 0u;
+    const uint32_t gw = fw >> 1;
+    // Byte offsets of the word's sub-grid word and its y neighbours within a
+    // plane (row -1 wraps past the range, row Y lands past it: both read 0).
+    const uint32_t SP = g.W * g.Y, W4 = g.W * 4u;  // words per sub-grid plane
+    const uint32_t o0 = valid ? (y * g.W + gw) * 4u : kOob;
+    const uint32_t om = valid ? o0 - W4 : kOob, op = valid ? o0 + W4 : kOob;
+    const uint32_t half = (fw & 1u) ? 0x05010400u : 0x07030602u;  // odd words: the low half
+    const VK_G uint32_t *sub[4] = {gptr(Js[0].bits), gptr(Js[1].bits), gptr(Js[2].bits),
+                                   gptr(Js[3].bits)};
+    // Raw words of planes z0 - 1 .. z0 + kFccZ: sub-grids 0 and 1 hold the
+    // even planes, 2 and 3 the odd ones (z0 is even).
+    uint32_t re[kFccZ + 2][3], ro[kFccZ + 2][3];
 #pragma unroll
-    for (int j = 0; j < 12; j++) interior &= n[j];
-    const uint32_t boundary = M0 & ~interior;
-    // Neighbour masks, two nodes per dword (node 2d in the low half): 4095
-    // for fully surrounded nodes, 0 for empty ones; boundary nodes get their
-    // 12 neighbour bits, patched halfword-wise in the thread's LDS slot.
-    const uint32_t ir = __brev(interior);  // bit k = node k
-    uint32_t mk[16];
-#pragma unroll
-    for (int d = 0; d < 16; d++) {
-        const uint32_t two = (ir >> (2 * d)) & 3u;
-        mk[d] = ((two & 1u) ? 0x0FFFu : 0u) | ((two & 2u) ? 0x0FFF0000u : 0u);
+    for (uint32_t k = 0; k < kFccZ + 2u; k++) {
+        const uint32_t fz = z0 + k - 1u;  // wraps for z0 == 0
+        const uint32_t s = (k & 1u) ? 0u : 2u;
+        const uint32_t bytes = fz < FZ ? SP * 4u : 0u;
+        const size_t at = fz < FZ ? (size_t)(fz >> 1) * SP : 0u;
+        const Rsrc e = rsrc(sub[s] + at, bytes), o = rsrc(sub[s + 1u] + at, bytes);
+        re[k][0] = ld32(e, om); re[k][1] = ld32(e, o0); re[k][2] = ld32(e, op);
+        ro[k][0] = ld32(o, om); ro[k][1] = ld32(o, o0); ro[k][2] = ld32(o, op);
     }
-    if (boundary) {
-        uint4 *my = fslot[threadIdx.y * kWave + threadIdx.x];
+    // Surface words and then their material bytes: node k is voxel k / 2 of
+    // the sub-grid with x parity k & 1, whose word's half holds 16 voxels.  A
+    // word that holds a surface voxel has all 32 material bytes written in
+    // the call (0 for its other voxels), so its half is read as 16 bytes.
+    u32x4 ma[kFccZ][2];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            my[q] = make_uint4(mk[4 * q], mk[4 * q + 1], mk[4 * q + 2], mk[4 * q + 3]);
-        uint16_t *mh = (uint16_t *)my;
-        uint32_t m = boundary;
-        while (m) {
-            const uint32_t s = 31u - (uint32_t)__clz(m);  // node 31 - s
-            uint32_t v = 0u;
-#pragma unroll
-            for (int j = 0; j < 12; j++) v |= ((n[j] >> s) & 1u) << j;
-            mh[31u - s] = (uint16_t)v;
-            m ^= 1u << s;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint4 v = my[q];
-            mk[4 * q] = v.x; mk[4 * q + 1] = v.y; mk[4 * q + 2] = v.z; mk[4 * q + 3] = v.w;
-        }
-    }
-    // Materials: node k is voxel k / 2 of the sub-grid with x parity k & 1,
-    // whose surface word's half for this FCC word holds 16 voxels.  A word
-    // with a surface voxel has all 32 material bytes written in the call (0
-    // for its other voxels), so each half is read as 16 bytes, or taken as 0
-    // when it has no surface voxel.
-    uint32_t ma[2][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+    for (uint32_t k = 0; k < kFccZ; k++) ma[k][0] = ma[k][1] = u32x4{0u, 0u, 0u, 0u};
     if (use_mats) {
-        const int odd = (int)(fz & 1);
-        const uint64_t gw = (uint64_t)(fw >> 1), gz = (uint64_t)(fz >> 1);
-        const uint32_t b = (uint32_t)((((gz >> bd.lbz) * bd.nby + ((uint64_t)y >> bd.lby)) *
-                                       bd.nbx) + (gw >> bd.lwx));
-        const size_t bbase = ((size_t)b << (bd.lwx + bd.lby + bd.lbz + 5u)) +
-                             (size_t)word_in_brick(bd, (uint32_t)gw, y, (uint32_t)gz) * 32u +
-                             ((fw & 1) ? 16u : 0u);
-        const size_t gwi = (gz * g.Y + (uint64_t)y) * g.W + gw;
-        const int sh = (fw & 1) ? 0 : 16;
+        uint32_t wm[kFccZ][2];
 #pragma unroll
-        for (int par = 0; par < 2; par++) {
-            const MatSource src = mat_source(Js[odd ? 2 + par : par]);  // uniform
-            if (!src.bhist[b]) continue;
-            if (((src.surf[gwi] >> sh) & 0xFFFFu) == 0u) continue;
-            const u32x4 v = *(const VK_G u32x4 *)(src.matgrid + bbase);
-            ma[par][0] = v.x; ma[par][1] = v.y; ma[par][2] = v.z; ma[par][3] = v.w;
+        for (uint32_t k = 0; k < kFccZ; k++) {
+            const uint32_t gz = (z0 + k) >> 1, wib = word_in_brick(bd, gw, y, gz);
+            const size_t b = brick_of_word(bd, gw, y, gz);
+            const bool in = valid && z0 + k < FZ;
+#pragma unroll
+            for (uint32_t par = 0; par < 2u; par++) {
+                const Job &S = Js[2u * (k & 1u) + par];
+                wm[k][par] = in ? gptr(S.wmask)[b * 4u + (wib >> 5)] >> (wib & 31u) : 0u;
+            }
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kFccZ; k++) {
+            const uint32_t gz = (z0 + k) >> 1, wib = word_in_brick(bd, gw, y, gz);
+            const size_t b = brick_of_word(bd, gw, y, gz);
+            const size_t at = (b << (bd.lwx + bd.lby + bd.lbz + 5u)) + (size_t)wib * 32u +
+                              ((fw & 1u) ? 16u : 0u);
+#pragma unroll
+            for (uint32_t par = 0; par < 2u; par++)
+                if (wm[k][par] & 1u)
+                    ma[k][par] = *(const VK_G u32x4 *)(gptr(Js[2u * (k & 1u) + par].matgrid) + at);
         }
     }
-    const size_t node0 = (((size_t)fz * FY + (size_t)y) * FW + (size_t)fw) * 32u;
-    if (kind == 3) {  // ShortFCCNode: mat<<12 | bid&4095
-        uint32_t out[16];
+    uint32_t word[kFccZ + 2][3];
 #pragma unroll
-        for (int d = 0; d < 16; d++) {
-            const uint32_t a = (ma[0][d >> 2] >> (8 * (d & 3))) & 0xFu;
-            const uint32_t c = (ma[1][d >> 2] >> (8 * (d & 3))) & 0xFu;
-            out[d] = mk[d] | (a << 12) | (c << 28);
-        }
-        VK_G u32x4 *dst = (VK_G u32x4 *)((VK_G uint8_t *)gptr(nodes) + node0 * 2u);
+    for (uint32_t k = 0; k < kFccZ + 2u; k++)
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            dst[q] = u32x4{out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
-    } else {  // LongFCCNode: {u16 bid, u8 mat, u8 0}
-        VK_G u32x4 *dst = (VK_G u32x4 *)((VK_G uint8_t *)gptr(nodes) + node0 * 4u);
+        for (uint32_t r = 0; r < 3u; r++) word[k][r] = fcc_word(re[k][r], ro[k][r], half);
+    // The word shifted by one node: its -x (left) and +x (right) neighbours.
+    const bool first = fw == 0u, last = fw + 1u == FW;
+    auto left = [&](uint32_t w) {
+        uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppWaveShr1, 0xF, 0xF, false);
+        if (first) p = 0u;
+        return (w >> 1) | (p << 31);
+    };
+    auto right = [&](uint32_t w) {
+        uint32_t n = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppWaveShl1, 0xF, 0xF, false);
+        if (last) n = 0u;
+        return (w << 1) | (n >> 31);
+    };
+    const uint32_t nbw = kind == 3 ? 64u : 128u;  // node bytes per word
+    const uint32_t ppw = nbw / 16u;               // 16-byte pieces per word
+    const uint32_t run = base < P ? min(kFccRun, P - base) : 0u;
+    VK_G uint8_t *nodes = (VK_G uint8_t *)gptr(Js[0].nodes);
+    uint4 *wst = stage[wave];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            uint32_t o[4];
+    for (uint32_t k = 0; k < kFccZ; k++) {
+        const uint32_t fz = z0 + k;
+        if (fz >= FZ) break;  // uniform
+        const uint32_t Dm = word[k][0], D0 = word[k][1], Dp = word[k][2];
+        const uint32_t Mm = word[k + 1][0], M0 = word[k + 1][1], Mp = word[k + 1][2];
+        const uint32_t Um = word[k + 2][0], U0 = word[k + 2][1], Up = word[k + 2][2];
+        const uint32_t E = (k & 1u) ? 0x55555555u : 0xAAAAAAAAu;  // (x+z) even
+        const uint32_t LM0 = left(M0), RM0 = right(M0);
+        uint32_t n[16];
+        n[0] = bfi(E, Dm, D0);
+        n[1] = left(D0);
+        n[2] = right(D0);
+        n[3] = bfi(E, D0, Dp);
+        n[4] = bfi(E, left(Mm), LM0);
+        n[5] = bfi(E, right(Mm), RM0);
+        n[6] = bfi(E, LM0, left(Mp));
+        n[7] = bfi(E, RM0, right(Mp));
+        n[8] = bfi(E, Um, U0);
+        n[9] = left(U0);
+        n[10] = right(U0);
+        n[11] = bfi(E, U0, Up);
+        uint32_t interior = M0;
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int d = 2 * q + e;
-                const uint32_t a = (ma[0][d >> 2] >> (8 * (d & 3))) & 0xFFu;
-                const uint32_t c = (ma[1][d >> 2] >> (8 * (d & 3))) & 0xFFu;
-                o[2 * e] = (mk[d] & 0xFFFFu) | (a << 16);
-                o[2 * e + 1] = (mk[d] >> 16) | (c << 16);
+        for (int j = 0; j < 12; j++) interior &= n[j];
+        // Node masks, two per dword (node 2d in the low half).
+        uint32_t mk[16];
+        if (M0 == interior && (M0 == 0u || M0 == ~0u)) {  // all empty, or all surrounded
+#pragma unroll
+            for (int d = 0; d < 16; d++) mk[d] = M0 & 0x0FFF0FFFu;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 12; j++) n[j] &= M0;
+#pragma unroll
+            for (int j = 12; j < 16; j++) n[j] = 0u;
+            // Two 16x16 bit matrices side by side (the halves of the words).
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t t = __builtin_amdgcn_perm(n[j + 8], n[j], 0x06020400u);
+                n[j + 8] = __builtin_amdgcn_perm(n[j + 8], n[j], 0x07030501u);
+                n[j] = t;
             }
-            dst[q] = u32x4{o[0], o[1], o[2], o[3]};
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                if (!(j & 4)) swap_bits<4, 0x0F0F0F0Fu>(n[j], n[j + 4]);
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                if (!(j & 2)) swap_bits<2, 0x33333333u>(n[j], n[j + 2]);
+#pragma unroll
+            for (int j = 0; j < 16; j += 2) swap_bits<1, 0x55555555u>(n[j], n[j + 1]);
+            // n[j] half h: the mask of bit position 16 h + j; node 31 - that.
+#pragma unroll
+            for (int d = 0; d < 16; d++)
+                mk[d] = __builtin_amdgcn_perm(n[14 - 2 * (d & 7)], n[15 - 2 * (d & 7)],
+                                              d < 8 ? 0x07060302u : 0x05040100u);
         }
+        const uint32_t a4[4] = {ma[k][0].x, ma[k][0].y, ma[k][0].z, ma[k][0].w};
+        const uint32_t c4[4] = {ma[k][1].x, ma[k][1].y, ma[k][1].z, ma[k][1].w};
+        const Rsrc nr = rsrc(nodes + ((size_t)fz * P + base) * nbw, run * nbw);
+        if (kind == 3) {  // ShortFCCNode: mat<<12 | bid&4095
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                uint32_t o[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t a = (a4[q] >> (8 * e)) & 0xFu, c = (c4[q] >> (8 * e)) & 0xFu;
+                    o[e] = mk[4 * q + e] | (a << 12) | (c << 28);
+                }
+                wst[q * kFccPitch + lane] = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        } else {  // LongFCCNode: {u16 bid, u8 mat, u8 0}
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                uint32_t o[4];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int d = 2 * q + e;
+                    const uint32_t a = (a4[d >> 2] >> (8 * (d & 3))) & 0xFFu;
+                    const uint32_t c = (c4[d >> 2] >> (8 * (d & 3))) & 0xFFu;
+                    o[2 * e] = (mk[d] & 0xFFFFu) | (a << 16);
+                    o[2 * e + 1] = (mk[d] >> 16) | (c << 16);
+                }
+                wst[q * kFccPitch + lane] = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        }
+        wave_lds_sync();
+        // Pieces past the run's end lie outside the range and are dropped.
+        const uint32_t lp = kind == 3 ? 2u : 3u;
+#pragma unroll
+        for (uint32_t s = 0; s < 8u; s++) {
+            if (s >= ppw) break;  // uniform
+            const uint32_t piece = s * kWave + lane;
+            const uint32_t w = min((piece >> lp) + 1u, kWave - 1u);
+            const uint4 v = wst[(piece & (ppw - 1u)) * kFccPitch + w];
+            st128(nr, piece * 16u, u32x4{v.x, v.y, v.z, v.w});
+        }
+        wave_lds_sync();  // the run is read out before the next plane's writes
     }
 }
 

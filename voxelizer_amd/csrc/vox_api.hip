@@ -554,6 +554,14 @@ vox_status add_job(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, uin
     P.pad_b.push_back(J.pad_base + (pad_words(W, L.alloc[1], L.alloc[2]) + 255u) / 256u);
     J.m = F3{(float)J.em[0], (float)J.em[1], (float)J.em[2]};
     J.fd = (float)g.voxel_length;
+    J.frd = 1.0f / J.fd;
+    // With these bounds and those a triangle is tested for (surf_tri_setup),
+    // no quotient of the surface pass overflows: |p - m| < 2^25 and normals
+    // below 2^40 over components above 2^-40 give less than 2^127.
+    J.fdiv = J.fd >= 0x1p-20f;
+    for (int a = 0; a < 3; a++)
+        J.fdiv &= std::fabs(a == 0 ? J.m.x : a == 1 ? J.m.y : J.m.z) +
+                      (float)(L.res[a] + 2u) * J.fd <= 0x1p24f;
     uint32_t nbt = 1;
     for (int a = 0; a < 3; a++) {
         J.bdim[a] = bdim[a];

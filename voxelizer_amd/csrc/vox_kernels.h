@@ -97,6 +97,7 @@ struct SplitTable {
 struct SurfParams {
     F3 m;       // float(extMinVertex)
     float d;    // float(voxelLength)
+    float rd;   // 1 / d
     int32_t res[3];  // ext resolution (x, y, z)
     uint32_t alloc[3];
     int32_t bdim[3];  // brick dims in voxels
@@ -140,6 +141,8 @@ struct Job {
     // surface stage
     F3 m;                  // float(origin)
     float fd;              // float(voxel length)
+    float frd;             // 1 / fd
+    int32_t fdiv;          // origin, extent and voxel length lie where div_by is exact
     int32_t bdim[3];       // brick dims (voxels)
     uint32_t nb[3];        // bricks per axis
     uint32_t brick_base;   // first brick
@@ -183,6 +186,7 @@ __device__ __forceinline__ SurfParams surf_params(const Job &J) {
     SurfParams p;
     p.m = J.m;
     p.d = J.fd;
+    p.rd = J.frd;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         p.res[a] = J.res[a];

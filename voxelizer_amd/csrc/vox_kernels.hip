@@ -614,20 +614,10 @@ __device__ __forceinline__ bool surf_clip(const SurfParams &p, VoxBB &vb) {
     vb.max = {min(vb.max.x, p.res[0] - 1), min(vb.max.y, p.res[1] - 1), min(vb.max.z, p.res[2] - 1)};
     return true;
 }
-__device__ __forceinline__ bool surf_range(const SurfParams &p, const F3 tri[3], VoxBB &vb) {
-    F3 mn, mx;
-    tri_bounds(tri, mn, mx);
-    vb = voxel_bounds_half(mn, mx, p.m, p.d);
-    return surf_clip(p, vb);
-}
-
 // Axis helpers: for dominant axis a, u and v are the other two axes in
 // increasing order.
 __device__ __forceinline__ int axis_u(int a) { return a == AX_X ? AX_Y : AX_X; }
 __device__ __forceinline__ int axis_v(int a) { return a == AX_Z ? AX_Y : AX_Z; }
-__device__ __forceinline__ float pick3(const F3 &p, int a) {
-    return a == AX_X ? p.x : a == AX_Y ? p.y : p.z;
-}
 __device__ __forceinline__ int32_t pick3i(const I3 &p, int a) {
     return a == AX_X ? p.x : a == AX_Y ? p.y : p.z;
 }
@@ -777,36 +767,43 @@ __device__ __forceinline__ uint32_t winner_key(uint32_t bb, uint32_t lt, uint32_
 // Per-triangle data of one brick's chunk, set up once in LDS.  Coordinates
 // are named (u, v, a): a is the triangle's dominant axis, u and v the other
 // two in increasing axis order (u = x unless a = x; v = z unless a = z).
-// Every 2-term edge function of the reference, (ne.x*c0 + ne.y*c1) + de, is
-// kept as (c_first*p_first + c_second*p_second) + de with the two products
-// in either order: IEEE addition is commutative, so the value is identical.
-struct SurfTri {
-    float dom[3][3];    // dominant-plane edges: (coef of u, coef of v, de)
-    float pl[2][3][3];  // the two other planes (3D): (coef of a, coef of other, de)
-    float n[3], t0[3];  // normal, first vertex (x, y, z)
-    int32_t lo[3], hi[3];      // brick-clipped voxel range, (u, v, a) order
-    int32_t vmin_a, vmax_a;    // unclipped range along a
-    int32_t s[3];              // LDS key strides of (u, v, a)
-    int32_t base;              // LDS key index of (lo_u, lo_v, lo_a)
-    int32_t wu;                // columns along u
-    int32_t ngu;               // work items along u (kSurfCols columns each)
-    float rngu;                // 1 / ngu
-    uint32_t key;              // LDS winner key (winner_key)
-    uint32_t flags;            // bb | axis<<2 | (plane0 other is v)<<4 | (plane1 other is v)<<5
+// Every 2-term edge function of the reference, (ne.x*c0 + ne.y*c1) + de >= 0,
+// is kept as c_first*p_first + c_second*p_second >= t with the two products
+// in either order (IEEE addition is commutative) and t = overlap_bound(de).
+// 44 words: a lane's 16-byte reads of neighbouring slots fall into different
+// LDS banks.
+struct __align__(16) SurfTri {
+    float dom[3][3];    // dominant-plane edges: (coef of u, coef of v, t)
+    float lu, lv;       // brick-clipped lowest u and v, less 1/2
+    float rwu;          // ~ 1 / columns along u
+    uint32_t ext;       // columns along u | voxels along a << 16
+    uint32_t pk;        // LDS key index of the box's low corner (12 bits), log2 key strides of
+                        // u, v, a (4 bits each), class, axis, kSlowDiv, kManySplits
+    uint32_t key;       // LDS winner key (winner_key)
+    // 3D triangles
+    float nu, nv, na, rna;  // normal, 1 / na
+    float t0u, t0v, ta;     // first vertex along u and v; its (vertex * normal) along a
+    int32_t la;             // brick-clipped lowest a
+    int32_t va, vb;         // range along a of the triangle's box in the brick's matSplitRes
+                            // interval (kManySplits: of the box alone)
+    float pl[2][3][3];      // the two other planes: (coef of a, coef of other, t)
 };
+static_assert(sizeof(SurfTri) == 176, "an odd number of 16-byte slots");
 constexpr int kSurfChunk = 64;
-// Columns (or 1D voxels) per work item.  Grouping neighbouring columns
-// shares the item's lookup and v terms but lowers the parallelism the LDS
-// latency needs: on the large hall 1 column is fastest (2 and 4 measured
-// 9% and 13% slower).
-constexpr int kSurfCols = 1;
+constexpr uint32_t kPkU = 12, kPkV = 16, kPkA = 20, kPkClass = 24, kPkAxis = 26;
+constexpr uint32_t kSlowDiv = 1u << 28;     // coordinates too large or small for div_by
+constexpr uint32_t kManySplits = 1u << 29;  // the range along a crosses matSplitRes intervals
 
+__device__ __forceinline__ F3 rotate_axes(const F3 &p, int a) {  // (u, v, a) up to a swap of u, v
+    return a == AX_X ? F3{p.y, p.z, p.x} : a == AX_Y ? F3{p.z, p.x, p.y} : p;
+}
 
 // Sets up triangle t for the brick whose alloc-coordinate box starts at
 // (ext coordinates) (blx, bly, blz), restricted to its z layers [z0, z1)
 // (a sub-brick); returns its work items there: voxels along the axis for 1D,
 // dominant-plane columns for 2D/3D.
-__device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p,
+__device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p, bool fdiv,
+                                                   const SplitTable &spl,
                                                    const float4 *__restrict__ tri_rec, uint32_t t,
                                                    uint32_t tri_base, bool embed,
                                                    int32_t blx, int32_t bly, int32_t blz,
@@ -815,186 +812,224 @@ __device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p,
                  r2 = tri_rec[3 * (size_t)t + 2];
     const F3 tri[3] = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, {r1.z, r1.w, r2.x}};
     const uint32_t info = __float_as_uint(r2.y);
-    VoxBB vb;
-    if (!surf_range(p, tri, vb)) return 0u;
+    F3 mn, mx;
+    tri_bounds(tri, mn, mx);
+    const bool near0 = fdiv && mn.x >= -0x1p24f && mn.y >= -0x1p24f && mn.z >= -0x1p24f &&
+                       mx.x <= 0x1p24f && mx.y <= 0x1p24f && mx.z <= 0x1p24f;
+    VoxBB vb = near0 ? voxel_bounds_half_by(mn, mx, p.m, p.d, p.rd)
+                     : voxel_bounds_half(mn, mx, p.m, p.d);
+    if (!surf_clip(p, vb)) return 0u;
     const int bb = (int)(info >> 30), a = (int)((info >> 28) & 3u);
     const int ua = axis_u(a), va = axis_v(a);
-    const int32_t bd[3] = {p.bdim[0], p.bdim[1], p.bdim[2]};
-    const int32_t stride[3] = {1, bd[0], bd[0] * bd[1]};
+    const uint32_t lgx = 31u - (uint32_t)__clz(p.bdim[0]),
+                   lgz = lgx + 31u - (uint32_t)__clz(p.bdim[1]);
     const int ax3[3] = {ua, va, a};
     int32_t lo[3], hi[3];
+    uint32_t base = 0u, pk = (uint32_t)bb << kPkClass | (uint32_t)a << kPkAxis;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         const int ax = ax3[k];
-        const int32_t bl = ax == AX_X ? blx : ax == AX_Y ? bly : blz + z0;
-        const int32_t bs = ax == AX_X ? bd[0] : ax == AX_Y ? bd[1] : z1 - z0;
+        const int32_t b0 = ax == AX_X ? blx : ax == AX_Y ? bly : blz;
+        const int32_t bl = ax == AX_Z ? blz + z0 : b0;
+        const int32_t bs = ax == AX_X ? p.bdim[0] : ax == AX_Y ? p.bdim[1] : z1 - z0;
+        const uint32_t lg = ax == AX_X ? 0u : ax == AX_Y ? lgx : lgz;
         lo[k] = max(pick3i(vb.min, ax), bl);
         hi[k] = min(pick3i(vb.max, ax), bl + bs - 1);
         if (lo[k] > hi[k]) return 0u;
-        st.lo[k] = lo[k];
-        st.hi[k] = hi[k];
-        st.s[k] = ax == AX_X ? stride[0] : ax == AX_Y ? stride[1] : stride[2];
+        base += (uint32_t)(lo[k] - b0) << lg;
+        pk |= lg << (kPkU + 4u * (uint32_t)k);
     }
-    st.base = (lo[0] - (ua == AX_X ? blx : ua == AX_Y ? bly : blz)) * st.s[0] +
-              (lo[1] - (va == AX_X ? blx : va == AX_Y ? bly : blz)) * st.s[1] +
-              (lo[2] - (a == AX_X ? blx : a == AX_Y ? bly : blz)) * st.s[2];
-    st.vmin_a = pick3i(vb.min, a);
-    st.vmax_a = pick3i(vb.max, a);
+    const uint32_t wu = (uint32_t)(hi[0] - lo[0] + 1), wa = (uint32_t)(hi[2] - lo[2] + 1);
+    st.ext = wu | wa << 16;
     st.key = winner_key((uint32_t)bb, t - tri_base, __float_as_uint(r2.z), embed);
-    st.wu = hi[0] - lo[0] + 1;
-    st.ngu = (st.wu + kSurfCols - 1) / kSurfCols;
-    st.rngu = 1.0f / (float)st.ngu;
-    uint32_t flags = (uint32_t)bb | ((uint32_t)a << 2);
-    if (bb == BB_1D) {
-        st.flags = flags;
-        return (uint32_t)((hi[2] - lo[2] + kSurfCols) / kSurfCols);
-    }
+    st.pk = pk |= base;
+    if (bb == BB_1D) return wa;
+    st.lu = (float)lo[0] - 0.5f;
+    st.lv = (float)lo[1] - 0.5f;
+    st.rwu = __builtin_amdgcn_rcpf((float)wu);
     const F3 n = fcross(fsub(tri[0], tri[2]), fsub(tri[1], tri[0]));
-    st.n[0] = n.x; st.n[1] = n.y; st.n[2] = n.z;
-    st.t0[0] = tri[0].x; st.t0[1] = tri[0].y; st.t0[2] = tri[0].z;
-    // Plane P tests coordinates (c0, c1): plane 0 (y, z), 1 (z, x), 2 (x, y).
-    auto first_axis = [](int P) { return P == 0 ? AX_Y : P == 1 ? AX_Z : AX_X; };
-    auto second_axis = [](int P) { return P == 0 ? AX_Z : P == 1 ? AX_X : AX_Y; };
-    {
-        OverlapData o;
-        setup_overlap(tri, n, p.d, a, o);
-        const bool first_is_u = first_axis(a) == ua;
+    // With the axes rotated so that a comes last, (x, y) is the dominant
+    // plane in the reference's coordinate order, (y, z) the plane of x and
+    // (z, x) the plane of y.  u and v are x and y, or y and x for a = y.
+    const F3 rn = rotate_axes(n, a);
+    const F3 rt[3] = {rotate_axes(tri[0], a), rotate_axes(tri[1], a), rotate_axes(tri[2], a)};
+    const bool swap = a == AX_Y;
 #pragma unroll
-        for (int e = 0; e < 3; e++) {
-            st.dom[e][0] = first_is_u ? o.ne[e].x : o.ne[e].y;
-            st.dom[e][1] = first_is_u ? o.ne[e].y : o.ne[e].x;
-            st.dom[e][2] = o.de[e];
+    for (int e = 0; e < 3; e++) {
+        const F3 A = rt[e], B = rt[(e + 1) % 3];
+        float n0, n1, de;
+        overlap_edge(A.x, A.y, B.x, B.y, rn.z >= 0.0f, p.d, n0, n1, de);
+        st.dom[e][0] = swap ? n1 : n0;
+        st.dom[e][1] = swap ? n0 : n1;
+        st.dom[e][2] = overlap_bound(de);
+        if (bb == BB_3D) {
+            overlap_edge(A.y, A.z, B.y, B.z, rn.x >= 0.0f, p.d, n0, n1, de);
+            st.pl[0][e][0] = n1;
+            st.pl[0][e][1] = n0;
+            st.pl[0][e][2] = overlap_bound(de);
+            overlap_edge(A.z, A.x, B.z, B.x, rn.y >= 0.0f, p.d, n0, n1, de);
+            st.pl[1][e][0] = n0;
+            st.pl[1][e][1] = n1;
+            st.pl[1][e][2] = overlap_bound(de);
         }
     }
     if (bb == BB_3D) {
-        const int planes[2] = {a == AX_X ? 1 : 0, a == AX_Z ? 1 : 2};
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            OverlapData o;
-            setup_overlap(tri, n, p.d, planes[q], o);
-            const bool first_is_a = first_axis(planes[q]) == a;
-            const int other = first_is_a ? second_axis(planes[q]) : first_axis(planes[q]);
-            if (other == va) flags |= 1u << (4 + q);
-#pragma unroll
-            for (int e = 0; e < 3; e++) {
-                st.pl[q][e][0] = first_is_a ? o.ne[e].x : o.ne[e].y;
-                st.pl[q][e][1] = first_is_a ? o.ne[e].y : o.ne[e].x;
-                st.pl[q][e][2] = o.de[e];
-            }
+        st.nu = swap ? rn.y : rn.x;
+        st.nv = swap ? rn.x : rn.y;
+        st.na = rn.z;
+        st.rna = 1.0f / rn.z;
+        st.t0u = swap ? rt[0].y : rt[0].x;
+        st.t0v = swap ? rt[0].x : rt[0].y;
+        st.ta = rt[0].z * rn.z;
+        st.la = lo[2];
+        int32_t sa = pick3i(vb.min, a), sb = pick3i(vb.max, a);
+        const uint32_t ns = spl.n[a];
+        uint32_t si = 0;
+        while (si + 1u < ns && (uint32_t)lo[2] >= spl.hi[a][si]) si++;
+        if (si + 1u < ns && (uint32_t)hi[2] >= spl.hi[a][si]) {
+            pk |= kManySplits;
+        } else {
+            sa = max(sa, (int32_t)spl.lo[a][si]);
+            sb = min(sb, (int32_t)spl.hi[a][si] - 1);
         }
+        st.va = sa;
+        st.vb = sb;
+        const bool safe = near0 && fabsf(n.x) <= 0x1p40f && fabsf(n.y) <= 0x1p40f &&
+                          fabsf(n.z) <= 0x1p40f && fabsf(rn.z) >= 0x1p-40f;
+        st.pk = pk | (safe ? 0u : kSlowDiv);
     }
-    st.flags = flags;
-    return (uint32_t)(st.ngu * (hi[1] - lo[1] + 1));
+    return wu * (uint32_t)(hi[1] - lo[1] + 1);
 }
 
-__device__ __forceinline__ void key_write(uint32_t *keys, uint8_t *touched, int32_t idx,
-                                          int32_t nvox, int32_t row_shift, uint32_t key) {
-    if ((uint32_t)idx >= (uint32_t)nvox) return;  // unreachable: items lie in the brick
+__device__ __forceinline__ void key_write(uint32_t *keys, uint8_t *touched, uint32_t idx,
+                                          uint32_t nvox, uint32_t row_shift, uint32_t key) {
+    if (idx >= nvox) return;  // unreachable: items lie in the brick
     atomicMax(&keys[idx], key);
     touched[idx >> row_shift] = 1;
 }
 
-// One work item, following the 1D/2D/3D kernels of the reference
-// (src/voxelizer.cu:3307-3955) with their matSplitRes subspace clipping --
-// only the 3D single-voxel shortcut depends on the subspace, through the
-// dominant-axis interval the voxel falls in.
-__device__ __forceinline__ void surf_item(const SurfParams &p, const SplitTable &spl, const SurfTri &st,
-                          uint32_t k, uint32_t *keys, uint8_t *touched, int32_t nvox,
-                          int32_t row_shift) {
-    const uint32_t flags = st.flags;
-    const int bb = (int)(flags & 3u), a = (int)((flags >> 2) & 3u);
+// The dominant-plane half of work item k (a 1D triangle's voxel, or a column
+// of the others' box), following the 1D/2D/3D kernels of the reference
+// (src/voxelizer.cu:3307-3955).  1D and 2D hits are written; true for a 3D
+// triangle's column that passes, whose depth part follows (surf_depth).
+__device__ __forceinline__ bool surf_column(const SurfParams &p, const SurfTri &st, uint32_t k,
+                                            uint32_t *keys, uint8_t *touched, uint32_t nvox,
+                                            uint32_t row_shift, uint32_t &cu, uint32_t &cv) {
+    const uint32_t pk = st.pk, base = pk & 0xFFFu;
+    const uint32_t bb = (pk >> kPkClass) & 3u, a = (pk >> kPkAxis) & 3u;
     if (bb == BB_1D) {
-        const int32_t len = st.hi[2] - st.lo[2] + 1;
-        for (int j = 0; j < kSurfCols; j++) {
-            const int32_t kk = (int32_t)k * kSurfCols + j;
-            if (kk >= len) break;
-            key_write(keys, touched, st.base + (int32_t)__umul24(kk, st.s[2]), nvox, row_shift,
-                      st.key);
+        key_write(keys, touched, base + (k << ((pk >> kPkA) & 15u)), nvox, row_shift, st.key);
+        return false;
+    }
+    // k = cv * wu + cu
+    const int32_t wu = (int32_t)(st.ext & 0xFFFFu);
+    int32_t q = (int32_t)((float)k * st.rwu);
+    int32_t r = (int32_t)k - (int32_t)__umul24(q, wu);
+    if (r < 0) { q--; r += wu; }
+    if (r >= wu) { q++; r -= wu; }
+    cu = (uint32_t)r;
+    cv = (uint32_t)q;
+    const float mu = a == AX_X ? p.m.y : p.m.x, mv = a == AX_Z ? p.m.y : p.m.z;
+    const float pu = mu + (st.lu + (float)r) * p.d;  // vox_corner
+    const float pv = mv + (st.lv + (float)q) * p.d;
+    bool in = true;
+#pragma unroll
+    for (int e = 0; e < 3; e++) in &= st.dom[e][0] * pu + st.dom[e][1] * pv >= st.dom[e][2];
+    if (in && bb != BB_3D)
+        key_write(keys, touched,
+                  base + (cu << ((pk >> kPkU) & 15u)) + (cv << ((pk >> kPkV) & 15u)), nvox,
+                  row_shift, st.key);
+    return in && bb == BB_3D;
+}
+
+// The depth part of a 3D triangle's column (determineDepthRange{X,Y,Z},
+// src/voxelizer.cu:4004-4119, and the side-plane tests along the column).
+// It costs about four times the dominant-plane test and only half of a box's
+// columns reach it, so a wave queues those in LDS and works them off 64 at a
+// time; its four divisions go by reciprocals.  k_surf_brick: room at 1 cm
+// (512x403x303) 237 -> 198 us (89.4 -> 64.9 M wave instructions), hall
+// (1536x1024x768) 930 -> 849 us (354 -> 295 M), LongFCC room 640x255x384
+// 451 -> 417 us, 64-mesh batch 2002 -> 1835 us.
+// Only the single-voxel shortcut depends on the matSplitRes subspace, through
+// the interval along a that the voxel falls in.
+__device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable &spl,
+                                           const SurfTri &st, uint32_t cu, uint32_t cv,
+                                           uint32_t *keys, uint8_t *touched, uint32_t nvox,
+                                           uint32_t row_shift) {
+    const uint32_t pk = st.pk, a = (pk >> kPkAxis) & 3u, sa = (pk >> kPkA) & 15u;
+    const float mu = a == AX_X ? p.m.y : p.m.x, mv = a == AX_Z ? p.m.y : p.m.z;
+    const float ma = a == AX_X ? p.m.x : a == AX_Y ? p.m.y : p.m.z;
+    const float pu = mu + (st.lu + (float)cu) * p.d, pv = mv + (st.lv + (float)cv) * p.d;
+    // Depths of the plane over the column's two extreme corners: the dot
+    // product's terms in x, y, z order, (u + v) + a for a = z, (u + a) + v
+    // otherwise (IEEE addition is commutative).
+    const float pu1 = pu + p.d, pv1 = pv + p.d;
+    const bool fu = st.nu > 0.0f, fv = st.nv > 0.0f;
+    const float u0 = (st.t0u - (fu ? pu1 : pu)) * st.nu, u1 = (st.t0u - (fu ? pu : pu1)) * st.nu;
+    const float v0 = (st.t0v - (fv ? pv1 : pv)) * st.nv, v1 = (st.t0v - (fv ? pv : pv1)) * st.nv;
+    const bool az = a == AX_Z;
+    const float x0 = az ? v0 : st.ta, y0 = az ? st.ta : v0;
+    const float x1 = az ? v1 : st.ta, y1 = az ? st.ta : v1;
+    const float num0 = (u0 + x0) + y0, num1 = (u1 + x1) + y1;
+    int32_t lo, hi;
+    if (pk & kSlowDiv) {
+        float d0 = num0 / st.na, d1 = num1 / st.na;
+        if (d0 > d1) {
+            const float tmp = d0;
+            d0 = d1;
+            d1 = tmp;
+        }
+        lo = f2i(ceilf((d0 - ma) / p.d - 0.5f));
+        hi = f2i(floorf((d1 - ma) / p.d + 0.5f));
+    } else {  // finite throughout
+        const float d0 = div_by(num0, st.na, st.rna), d1 = div_by(num1, st.na, st.rna);
+        lo = f2i(ceilf(div_by(fminf(d0, d1) - ma, p.d, p.rd) - 0.5f));
+        hi = f2i(floorf(div_by(fmaxf(d0, d1) - ma, p.d, p.rd) + 0.5f));
+    }
+    const int32_t la = st.la;
+    const int32_t ilo = max(lo, la), ihi = min(hi, la + (int32_t)(st.ext >> 16) - 1);
+    if (ilo > ihi) return;
+    // The two side planes' edge functions along the column, c * pa + k >= t.
+    float sc[6], sk[6], se[6];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const float po = (q == 0) == (a == AX_Y) ? pu : pv;  // plane of v, then of u, for a = y
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            sc[3 * q + e] = st.pl[q][e][0];
+            sk[3 * q + e] = st.pl[q][e][1] * po;
+            se[3 * q + e] = st.pl[q][e][2];
+        }
+    }
+    uint32_t idx = (pk & 0xFFFu) + (cu << ((pk >> kPkU) & 15u)) + (cv << ((pk >> kPkV) & 15u)) +
+                   ((uint32_t)(ilo - la) << sa);
+    const uint32_t key = st.key;
+    float fa = (float)ilo - 0.5f;
+    auto inside = [&]() {
+        const float pa = ma + fa * p.d;  // vox_corner
+        bool in = true;
+#pragma unroll
+        for (int e = 0; e < 6; e++) in &= sc[e] * pa + sk[e] >= se[e];
+        return in;
+    };
+    if (!(pk & kManySplits)) {
+        const bool single = max(lo, st.va) == min(hi, st.vb);
+        for (int32_t i = ilo; i <= ihi; i++) {
+            if (single || inside()) key_write(keys, touched, idx, nvox, row_shift, key);
+            fa += 1.0f;
+            idx += 1u << sa;
         }
         return;
     }
-    // item k covers columns u0 .. u0+kSurfCols-1 of row v:
-    // k = (v - lo_v) * ngu + (u0 - lo_u) / kSurfCols
-    // Strides and indices here are below 2^24 (bricks hold at most 4096
-    // voxels), so products use the full-rate 24-bit multiply.
-    int32_t q = (int32_t)((float)k * st.rngu);
-    int32_t r = (int32_t)k - (int32_t)__umul24(q, st.ngu);
-    if (r < 0) { q--; r += st.ngu; }
-    if (r >= st.ngu) { q++; r -= st.ngu; }
-    const int32_t v = st.lo[1] + q;
-    const int ua = axis_u(a), va = axis_v(a);
-    const float mx = p.m.x, my = p.m.y, mz = p.m.z;
-    const float mu = ua == AX_X ? mx : (ua == AX_Y ? my : mz);
-    const float mv = va == AX_X ? mx : (va == AX_Y ? my : mz);
-    const float ma = a == AX_X ? mx : (a == AX_Y ? my : mz);
-    const float pv = vox_corner(v, mv, p.d);
-    float kdom[3];  // v terms of the dominant-plane edge functions
-#pragma unroll
-    for (int e = 0; e < 3; e++) kdom[e] = st.dom[e][1] * pv;
-    const bool threeD = bb == BB_3D;
-    const F3 t0 = {st.t0[0], st.t0[1], st.t0[2]}, nn = {st.n[0], st.n[1], st.n[2]};
     const uint32_t ns = spl.n[a];
-    for (int j = 0; j < kSurfCols; j++) {
-        const int32_t cu = r * kSurfCols + j;  // column offset along u
-        if (cu >= st.wu) break;
-        const int32_t u = st.lo[0] + cu;
-        const float pu = vox_corner(u, mu, p.d);
-        bool in = true;
-#pragma unroll
-        for (int e = 0; e < 3; e++) in &= (st.dom[e][0] * pu + kdom[e]) + st.dom[e][2] >= 0.0f;
-        if (!in) continue;
-        const int32_t col =
-            st.base + (int32_t)__umul24(cu, st.s[0]) + (int32_t)__umul24(q, st.s[1]);
-        if (!threeD) {
-            key_write(keys, touched, col, nvox, row_shift, st.key);
-            continue;
-        }
-        const F3 pp = {a == AX_X ? 0.0f : pu, a == AX_Y ? 0.0f : (a == AX_X ? pu : pv),
-                       a == AX_Z ? 0.0f : pv};
-        int32_t lo, hi;
-        depth_range(t0, pp, nn, p.m, p.d, a, lo, hi);
-        const int32_t ilo = max(lo, st.lo[2]), ihi = min(hi, st.hi[2]);
-        if (ilo > ihi) continue;
-        // The two side planes' edge functions along the column,
-        // (c * pa + k) + e, with their constant parts in registers.
-        float sc[6], sk[6], se[6];
-#pragma unroll
-        for (int q2 = 0; q2 < 2; q2++) {
-            const float po = (flags >> (4 + q2)) & 1u ? pv : pu;
-#pragma unroll
-            for (int e = 0; e < 3; e++) {
-                sc[3 * q2 + e] = st.pl[q2][e][0];
-                sk[3 * q2 + e] = st.pl[q2][e][1] * po;
-                se[3 * q2 + e] = st.pl[q2][e][2];
-            }
-        }
-        // matSplitRes interval of the voxel along a (advanced as i grows)
-        // and the single-voxel shortcut's range clipped to it.
-        uint32_t si = 0;
-        while (si + 1 < ns && (uint32_t)ilo >= spl.hi[a][si]) si++;
-        uint32_t shi = spl.hi[a][si];
-        int32_t rl = max(lo, max(st.vmin_a, (int32_t)spl.lo[a][si]));
-        int32_t rh = min(hi, min(st.vmax_a, (int32_t)shi - 1));
-        const int32_t sa = st.s[2], col0 = col - __mul24(st.lo[2], sa);  // lo may be -1
-        for (int32_t i = ilo; i <= ihi; i++) {
-            if (si + 1 < ns && (uint32_t)i >= shi) {
-                do si++;
-                while (si + 1 < ns && (uint32_t)i >= spl.hi[a][si]);
-                shi = spl.hi[a][si];
-                rl = max(lo, max(st.vmin_a, (int32_t)spl.lo[a][si]));
-                rh = min(hi, min(st.vmax_a, (int32_t)shi - 1));
-            }
-            bool write = rl == rh;
-            if (!write) {
-                const float pa = vox_corner(i, ma, p.d);
-                float f[6];
-#pragma unroll
-                for (int e = 0; e < 6; e++) f[e] = (sc[e] * pa + sk[e]) + se[e];
-                write = f[0] >= 0.0f && f[1] >= 0.0f && f[2] >= 0.0f && f[3] >= 0.0f &&
-                        f[4] >= 0.0f && f[5] >= 0.0f;
-            }
-            if (write) key_write(keys, touched, col0 + __mul24(i, sa), nvox, row_shift, st.key);
-        }
+    uint32_t si = 0;
+    for (int32_t i = ilo; i <= ihi; i++) {
+        while (si + 1u < ns && (uint32_t)i >= spl.hi[a][si]) si++;
+        const int32_t rl = max(lo, max(st.va, (int32_t)spl.lo[a][si]));
+        const int32_t rh = min(hi, min(st.vb, (int32_t)spl.hi[a][si] - 1));
+        if (rl == rh || inside()) key_write(keys, touched, idx, nvox, row_shift, key);
+        fa += 1.0f;
+        idx += 1u << sa;
     }
 }
 
@@ -1030,7 +1065,11 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
     __shared__ SurfTri tris[kSurfChunk];
     __shared__ uint32_t cstart[kSurfChunk], ctotal[2], smask[256 / kWave][2];
     __shared__ uint8_t cslot[kSurfChunk];
-    __shared__ uint32_t wsurf[kMaxBrickVox / 32];
+    // Per wave the columns that await their depth part; in the epilogue the
+    // brick's surface words.
+    __shared__ uint32_t wqueue[256 / kWave][2 * kWave];
+    uint32_t *wsurf = &wqueue[0][0];
+    static_assert(sizeof(wqueue) >= kMaxBrickVox / 8, "surface words fit the queues");
     __shared__ uint8_t touched[32];
     __shared__ uint32_t s_q, s_qe;
     __shared__ SplitTable spl;
@@ -1140,8 +1179,8 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
                     uint32_t items = 0u;
                     if (c0 + tid < cnt) {
                         const uint32_t t = blist[off + c0 + tid];
-                        items = surf_tri_setup(p, tri_rec, t, J.tri_base, embed, blx, bly, blz,
-                                               z0, z1, tris[tid]);
+                        items = surf_tri_setup(p, J.fdiv != 0, spl, tri_rec, t, J.tri_base, embed,
+                                               blx, bly, blz, z0, z1, tris[tid]);
                     }
                     static_assert(kSurfChunk == kWave, "one wave sets up a chunk");
                     const uint32_t incl = wave_incl_scan(items);
@@ -1169,7 +1208,12 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
                 // OR together in LDS.
                 const uint32_t cs = lane < ntri ? cstart[lane] : UINT32_MAX;
                 const uint32_t sl = lane < ntri ? (uint32_t)cslot[lane] : 0u;
-                uint32_t *sm = &smask[wave][0];
+                uint32_t *sm = &smask[wave][0], *wq = wqueue[wave];
+                uint32_t nq = 0u;  // columns in the wave's queue (uniform)
+                auto depth = [&](uint32_t e) {
+                    surf_depth(p, spl, tris[e >> 24], e & 0xFFFu, (e >> 12) & 0xFFFu, keys, touched,
+                               (uint32_t)nvox, (uint32_t)row_shift);
+                };
                 for (uint32_t w0 = wave * kWave; w0 < total; w0 += blockDim.x) {  // uniform
                     const uint32_t t0 = (uint32_t)__popcll(__ballot(cs <= w0)) - 1u;
                     const uint32_t ps = cs - w0 - 1u;  // start offset - 1, in 0..62
@@ -1184,9 +1228,25 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
                     const uint32_t slot = (uint32_t)__shfl((int)sl, (int)ti);
                     const uint32_t first = (uint32_t)__shfl((int)cs, (int)ti);
                     const uint32_t c = w0 + lane;
-                    if (c < total)
-                        surf_item(p, spl, tris[slot], c - first, keys, touched, nvox, row_shift);
+                    uint32_t cu = 0u, cv = 0u;
+                    const bool deep =
+                        c < total && surf_column(p, tris[slot], c - first, keys, touched,
+                                                 (uint32_t)nvox, (uint32_t)row_shift, cu, cv);
+                    const unsigned long long dm = __ballot(deep);
+                    if (deep)
+                        wq[nq + __builtin_amdgcn_mbcnt_hi(
+                                    (uint32_t)(dm >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((uint32_t)dm, 0u))] =
+                            slot << 24 | cv << 12 | cu;
+                    nq += (uint32_t)__popcll(dm);
+                    wave_lds_sync();
+                    if (nq >= (uint32_t)kWave) {
+                        nq -= (uint32_t)kWave;
+                        depth(wq[nq + lane]);
+                        wave_lds_sync();
+                    }
                 }
+                if (lane < nq) depth(wq[lane]);
             }
             __syncthreads();
             // Surface bit words and winner materials, 256 voxels per wave

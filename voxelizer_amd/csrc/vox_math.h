@@ -42,13 +42,12 @@ __device__ __forceinline__ uint32_t sat_u32(double v) {
     if (v <= -1.0) return 0u;
     return (uint32_t)v;
 }
-// sat_i32((double)v) without the double: NaN -> 0, v >= 2^31 -> INT32_MAX,
-// v < -2^31 -> INT32_MIN (the largest float below -2^31 is -2^31 - 128, so
-// the double bound -2^31 - 1 selects the same floats), else truncation.
-// Written as selects so that it compiles to compares, not branches.
+// sat_i32((double)v) without the double: v_cvt_i32_f32 truncates, saturates
+// and returns 0 for NaN (a C++ conversion leaves those cases undefined).
 __device__ __forceinline__ int32_t f2i(float v) {
-    const int32_t t = (v >= -2147483648.0f && v < 2147483648.0f) ? (int32_t)v : 0;
-    return v != v ? 0 : v >= 2147483648.0f ? INT32_MAX : v < -2147483648.0f ? INT32_MIN : t;
+    int32_t r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 
 __device__ __forceinline__ D3 fetch_d(const float *__restrict__ V, const uint32_t *__restrict__ I,
@@ -201,7 +200,6 @@ enum { BB_DEGEN = 0, BB_1D = 1, BB_2D = 2, BB_3D = 3 };
 enum { AX_X = 0, AX_Y = 1, AX_Z = 2 };
 
 struct VoxBB { I3 min, max; };
-struct OverlapData { F2 ne[3]; float de[3]; };
 
 __device__ __forceinline__ void tri_bounds(const F3 t[3], F3 &mn, F3 &mx) {
     mn = t[0];
@@ -216,6 +214,18 @@ __device__ __forceinline__ void tri_bounds(const F3 t[3], F3 &mn, F3 &mx) {
         if (t[i].z > mx.z) mx.z = t[i].z;
     }
 }
+// x / b, correctly rounded, from y = 1 / b correctly rounded: after the first
+// correction the quotient is within one unit in the last place, and from there
+// Markstein's theorem makes the second correction's result the rounded quotient
+// (P. Markstein, IBM J. Res. Dev. 34, 1990), provided nothing overflows; a
+// numerator so small that the residuals lose bits keeps its quotient tiny.  5
+// instructions in place of the 11 (one of them quarter rate) of a division.
+__device__ __forceinline__ float div_by(float x, float b, float y) {
+    float q = x * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, x), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, x), y, q);
+}
+
 // getVoxelBoundsHalf (src/voxelizer.cu:2471-2492).
 __device__ __forceinline__ VoxBB voxel_bounds_half(F3 mn, F3 mx, F3 m, float d) {
     VoxBB b;
@@ -223,6 +233,17 @@ __device__ __forceinline__ VoxBB voxel_bounds_half(F3 mn, F3 mx, F3 m, float d) 
              f2i(ceilf((mn.z - m.z) / d - 0.5f))};
     b.max = {f2i(floorf((mx.x - m.x) / d + 0.5f)), f2i(floorf((mx.y - m.y) / d + 0.5f)),
              f2i(floorf((mx.z - m.z) / d + 0.5f))};
+    return b;
+}
+// The same with div_by (rd = 1 / d).
+__device__ __forceinline__ VoxBB voxel_bounds_half_by(F3 mn, F3 mx, F3 m, float d, float rd) {
+    VoxBB b;
+    b.min = {f2i(ceilf(div_by(mn.x - m.x, d, rd) - 0.5f)),
+             f2i(ceilf(div_by(mn.y - m.y, d, rd) - 0.5f)),
+             f2i(ceilf(div_by(mn.z - m.z, d, rd) - 0.5f))};
+    b.max = {f2i(floorf(div_by(mx.x - m.x, d, rd) + 0.5f)),
+             f2i(floorf(div_by(mx.y - m.y, d, rd) + 0.5f)),
+             f2i(floorf(div_by(mx.z - m.z, d, rd) + 0.5f))};
     return b;
 }
 __device__ __forceinline__ float vox_corner(int32_t c, float m, float d) {
@@ -274,66 +295,23 @@ __device__ __forceinline__ void classify_vb(const F3 t[3], const VoxBB &vb, int 
     }
 }
 
-// setup{YZ,ZX,XY}OverlapTest (src/voxelizer.cu:2677-2757): plane 0 = YZ
-// (coordinates (y,z)), 1 = ZX ((z,x)), 2 = XY ((x,y)).
-__device__ __forceinline__ void setup_overlap(const F3 t[3], F3 n, float d, int plane,
-                                              OverlapData &o) {
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const F3 a = t[i], b = t[(i + 1) % 3];
-        float a0, a1, b0, b1;  // projected (first, second) coordinates
-        bool pos;
-        if (plane == 0) {
-            a0 = a.y; a1 = a.z; b0 = b.y; b1 = b.z; pos = n.x >= 0.0f;
-        } else if (plane == 1) {
-            a0 = a.z; a1 = a.x; b0 = b.z; b1 = b.x; pos = n.y >= 0.0f;
-        } else {
-            a0 = a.x; a1 = a.y; b0 = b.x; b1 = b.y; pos = n.z >= 0.0f;
-        }
-        if (pos)
-            o.ne[i] = {a1 - b1, b0 - a0};
-        else
-            o.ne[i] = {b1 - a1, a0 - b0};
-        o.de[i] = -(o.ne[i].x * a0 + o.ne[i].y * a1) + fmaxf(0.0f, d * o.ne[i].x) +
-                  fmaxf(0.0f, d * o.ne[i].y);
-    }
+// setup{YZ,ZX,XY}OverlapTest (src/voxelizer.cu:2677-2757) for one edge a -> b
+// of a triangle projected to the plane's (first, second) coordinates, pos =
+// (normal component along the plane's axis >= 0).
+__device__ __forceinline__ void overlap_edge(float a0, float a1, float b0, float b1, bool pos,
+                                             float d, float &ne0, float &ne1, float &de) {
+    const float s0 = a1 - b1, s1 = b0 - a0;  // exact negations below
+    ne0 = pos ? s0 : -s0;
+    ne1 = pos ? s1 : -s1;
+    de = -(ne0 * a0 + ne1 * a1) + fmaxf(0.0f, d * ne0) + fmaxf(0.0f, d * ne1);
 }
-__device__ __forceinline__ bool overlap2(const OverlapData &o, float p0, float p1) {
-    bool r = true;
-#pragma unroll
-    for (int i = 0; i < 3; i++) r &= (o.ne[i].x * p0 + o.ne[i].y * p1) + o.de[i] >= 0.0f;
-    return r;
-}
-
-// determineDepthRange{X,Y,Z} (src/voxelizer.cu:4004-4119) for a voxel column
-// whose corner is p along the dominant axis `axis`.
-__device__ __forceinline__ void depth_range(const F3 t0, F3 p, F3 n, F3 m, float d, int axis,
-                                            int32_t &lo, int32_t &hi) {
-    F3 pmin, pmax;
-    if (axis == AX_X) {
-        bool ny = n.y > 0.0f, nz = n.z > 0.0f;
-        pmin = {0.0f, p.y + float(ny) * d, p.z + float(nz) * d};
-        pmax = {0.0f, p.y + float(!ny) * d, p.z + float(!nz) * d};
-    } else if (axis == AX_Y) {
-        bool nx = n.x > 0.0f, nz = n.z > 0.0f;
-        pmin = {p.x + float(nx) * d, 0.0f, p.z + float(nz) * d};
-        pmax = {p.x + float(!nx) * d, 0.0f, p.z + float(!nz) * d};
-    } else {
-        bool nx = n.x > 0.0f, ny = n.y > 0.0f;
-        pmin = {p.x + float(nx) * d, p.y + float(ny) * d, 0.0f};
-        pmax = {p.x + float(!nx) * d, p.y + float(!ny) * d, 0.0f};
-    }
-    float na = axis == AX_X ? n.x : axis == AX_Y ? n.y : n.z;
-    float a = fdot3(fsub(t0, pmin), n) / na;
-    float b = fdot3(fsub(t0, pmax), n) / na;
-    if (a > b) {
-        float tmp = a;
-        a = b;
-        b = tmp;
-    }
-    float mc = axis == AX_X ? m.x : axis == AX_Y ? m.y : m.z;
-    lo = f2i(ceilf((a - mc) / d - 0.5f));
-    hi = f2i(floorf((b - mc) / d + 0.5f));
+// The t for which x + de >= 0 and x >= t agree for every x: the sign of a
+// rounded sum is that of the exact one, so t = -de; an infinite de takes its
+// sum's value with the other infinity (NaN: false), and a NaN de is never met.
+__device__ __forceinline__ float overlap_bound(float de) {
+    return de == __builtin_inff()    ? -3.402823466e38f
+           : de == -__builtin_inff() ? __builtin_nanf("")
+                                     : -de;
 }
 
 // ---------------------------------------------------------------------------

@@ -1,4 +1,4 @@
-"""The brick pass's depth part off its usual path, bit-compared with the oracle:
+"""The brick pass off its usual path, bit-compared with the oracle: its list, and
 coordinates, voxel lengths and normals too large or too small for the reciprocal
 divisions (whole grids, and single triangles of a grid), and matSplitRes
 intervals that end inside a brick."""
@@ -58,3 +58,20 @@ def test_slivers_match_oracle(gpu_ctx, oracle):
         [m.indices.reshape(-1, 3), (base + np.arange(3 * n, dtype=np.uint32)).reshape(-1, 3)])
     m.materials = np.concatenate([m.materials, rng.integers(1, 8, n).astype(np.uint8)])
     check(gpu_ctx, oracle, m, 90)
+
+
+@pytest.mark.parametrize("ext", [(20, 1, 1), (20, 9, 17), (61, 150, 150), (200, 149, 301),
+                                 (200, 161, 317), (200, 163, 325), (330, 201, 333)])
+def test_brick_lists_match_oracle(gpu_ctx, oracle, ext):
+    """Boxes whose shells take from one brick to about three per resident
+    workgroup (1280), on either side of one each, so that the parts of the
+    list are empty, short and of uneven length."""
+    m = W.box(hi=ext, subdiv=3)
+    m.materials = (1 + np.arange(m.nt) % 7).astype(np.uint8)
+    gpu_ctx.set_mesh(m.vertices, m.indices)
+    gpu_ctx.set_materials(m.materials, 8)
+    g = gpu_ctx.plan_grid(va.PLAN_CUBE_LENGTH, 1.0)
+    og = oracle.plan_grid(m.vertices, va.PLAN_CUBE_LENGTH, 1.0)
+    assert g.same(og)
+    got = gpu_ctx.voxelize_nodes(g, va.NODE_SHORT, True)
+    assert np.array_equal(got, oracle.voxelize_nodes(m, og, va.NODE_SHORT, True))

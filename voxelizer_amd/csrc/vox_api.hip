@@ -968,13 +968,13 @@ vox_status surface_prep(vox_ctx *ctx, const Plan &P, const PlanDev &D, SurfPass 
     // Everything this stage and the brick pass count into starts at zero.
     uint32_t *wmask, *next, *cnt = nullptr;
     VOX_TRY(buf(ctx, "f_wmask", (size_t)nbt * 4u, &wmask));
-    VOX_TRY(buf(ctx, "f_next", 1, &next));
+    VOX_TRY(buf(ctx, "f_next", kBrickLists * kBrickListPitch, &next));
     if (learned && !ctx->record) VOX_TRY(buf(ctx, "f_cnt", 2, &cnt));
     VOX_TRY(fill_many(ctx, {{brick_hist, nbt, 0u},
                             {brick_cursor, nbt, 0u},
                             {wmask, (size_t)nbt * 4u, 0u},
                             {stats, 1, 0u},
-                            {next, 1, 0u},
+                            {next, kBrickLists * kBrickListPitch, 0u},
                             {cnt, cnt ? 2u : 0u, 0u}}));
     auto bin = [&](int scatter) -> vox_status {
         if (total == 0) return VOX_OK;
@@ -1070,12 +1070,12 @@ vox_status surface_brick(vox_ctx *ctx, const Plan &P, const PlanDev &D, const Su
     if (ctx->record) VOX_TRY(buf(ctx, "f_cycles", nbt, &cycles));
     const uint32_t blocks = std::min<uint32_t>(nbt, (uint32_t)(ctx->n_cu * ctx->surf_blocks_per_cu));
     if (P.any_partial)
-        k_surf_brick<true><<<blocks, 256, 0, ctx->stream>>>(
+        k_surf_brick<true><<<blocks, kBrickThreads, 0, ctx->stream>>>(
             D.jobs, D.brick_b, nj, ctx->rec, S.brick_off, S.brick_hist, S.blist,
             ctx->timing ? S.stats : nullptr, S.blist_order, S.n_list, S.hlist, S.hsub, S.n_heavy,
             S.skip, S.next, cycles);
     else
-        k_surf_brick<false><<<blocks, 256, 0, ctx->stream>>>(
+        k_surf_brick<false><<<blocks, kBrickThreads, 0, ctx->stream>>>(
             D.jobs, D.brick_b, nj, ctx->rec, S.brick_off, S.brick_hist, S.blist,
             ctx->timing ? S.stats : nullptr, S.blist_order, S.n_list, S.hlist, S.hsub, S.n_heavy,
             S.skip, S.next, cycles);
@@ -1311,8 +1311,8 @@ vox_status vox_create(int device, vox_ctx **out) {
     }
     if (hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, device) !=
             hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->surf_blocks_per_cu, k_surf_brick<false>, 256,
-                                                     0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->surf_blocks_per_cu, k_surf_brick<false>,
+                                                     kBrickThreads, 0) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->erode_blocks_per_cu, k_erode, 256, 0) !=
             hipSuccess) {
         vox_destroy(ctx);

@@ -63,6 +63,10 @@ __host__ __device__ __forceinline__ uint32_t plane_chunks(uint32_t W, uint32_t Y
 constexpr int kCartBX = 128, kCartBY = 4, kCartBZ = 8;
 constexpr int kFccBX = 64, kFccBY = 4, kFccBZ = 4;
 constexpr int kMaxBrickVox = 4096;
+// Brick pass: waves that voxelize, and one that prepares their next triangles.
+constexpr uint32_t kBrickWaves = 3, kBrickThreads = (kBrickWaves + 1) * kWave;
+// Counters the brick pass draws list entries from, and the words between them.
+constexpr uint32_t kBrickLists = 8, kBrickListPitch = 32;
 
 // Brick geometry as the node passes need it: bricks per row/column and the
 // log2 of the brick's words per row (x), rows (y) and planes (z).

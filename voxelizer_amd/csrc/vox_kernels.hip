@@ -798,18 +798,16 @@ __device__ __forceinline__ F3 rotate_axes(const F3 &p, int a) {  // (u, v, a) up
     return a == AX_X ? F3{p.y, p.z, p.x} : a == AX_Y ? F3{p.z, p.x, p.y} : p;
 }
 
-// Sets up triangle t for the brick whose alloc-coordinate box starts at
+// Sets up a triangle (its record r0..r2, mesh-local index lt) for the brick whose alloc-coordinate box starts at
 // (ext coordinates) (blx, bly, blz), restricted to its z layers [z0, z1)
 // (a sub-brick); returns its work items there: voxels along the axis for 1D,
 // dominant-plane columns for 2D/3D.
 __device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p, bool fdiv,
-                                                   const SplitTable &spl,
-                                                   const float4 *__restrict__ tri_rec, uint32_t t,
-                                                   uint32_t tri_base, bool embed,
-                                                   int32_t blx, int32_t bly, int32_t blz,
-                                                   int32_t z0, int32_t z1, SurfTri &st) {
-    const float4 r0 = tri_rec[3 * (size_t)t], r1 = tri_rec[3 * (size_t)t + 1],
-                 r2 = tri_rec[3 * (size_t)t + 2];
+                                                   const SplitTable &spl, const float4 &r0,
+                                                   const float4 &r1, const float4 &r2,
+                                                   uint32_t lt, bool embed, int32_t blx,
+                                                   int32_t bly, int32_t blz, int32_t z0,
+                                                   int32_t z1, SurfTri &st) {
     const F3 tri[3] = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, {r1.z, r1.w, r2.x}};
     const uint32_t info = __float_as_uint(r2.y);
     F3 mn, mx;
@@ -841,7 +839,7 @@ __device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p, bool fdi
     }
     const uint32_t wu = (uint32_t)(hi[0] - lo[0] + 1), wa = (uint32_t)(hi[2] - lo[2] + 1);
     st.ext = wu | wa << 16;
-    st.key = winner_key((uint32_t)bb, t - tri_base, __float_as_uint(r2.z), embed);
+    st.key = winner_key((uint32_t)bb, lt, __float_as_uint(r2.z), embed);
     st.pk = pk |= base;
     if (bb == BB_1D) return wa;
     st.lu = (float)lo[0] - 0.5f;
@@ -1034,25 +1032,47 @@ __device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable
 }
 
 // Persistent workgroups over a list of non-empty bricks (`order`: brick ids
-// in index order for the plain schedule, or sorted by predicted cost).  Each
-// workgroup takes runs of list entries from a global counter (the grab for
-// the following run is issued while the last brick of the current one is
-// processed), so bricks of uneven cost balance over the GPU.  Per brick: its triangles are
-// taken 64 at a time, each set up once into LDS, and all (triangle, column)
-// items of the chunk are spread over the 256 threads; winners accumulate in
-// LDS (ds_max of bbType<<30 | triangle).  Only rows of the brick that
-// received a key are visited afterwards: one ballot per 64 voxels gives the
-// surface bit words, one lane per surface voxel fetches its winner's material
-// into the brick's block of the material grid (one byte per voxel, brick
-// order), and the rows' keys are cleared for the next brick.  Surface bits
-// are ORed into the solid grid.  With `stats`, surface voxels are counted;
-// with `cycles`, each brick's duration (s_memtime) is recorded.  The kKeys
-// variant also stores the winner keys of jobs with a keygrid (PartialNode).
-// DPP controls of the epilogue's 8-lane OR (all lanes active).
+// in index order), before it the heavy bricks of the learned schedule
+// (`hlist`).  A workgroup is kBrickWaves waves that voxelize and one that
+// prepares: while the others work on a chunk of up to 64 triangles of a brick,
+// it takes the next list entry, loads the next chunk's triangle ids and
+// records, and, while the others write the finished brick, sets the chunk's
+// triangles up in LDS (a lane per triangle).  So neither the chain entry ->
+// brick -> ids -> records -> setup nor a global load stands in the voxelizing
+// waves' way: they work from LDS and only store.
+//
+// All (triangle, column) items of the chunk are spread over the voxelizing
+// threads; winners accumulate in LDS (ds_max of winner_key).  Rows that
+// received a key are visited when the brick's last chunk is done: each lane
+// takes four voxels, a word's eight lanes OR their bits into the solid grid,
+// and the words that hold a surface voxel have their winners' materials
+// stored in the brick's block of the material grid.  With `stats`, surface
+// voxels are counted; with `cycles`, each brick's duration from its first
+// item to its last store (s_memtime) is recorded.  The kKeys variant also
+// stores surface words and winner keys for jobs with a keygrid (PartialNode).
+//
+// Before the split every brick paid that chain and its setup in series, and one
+// counter handed out the list.  Together (fifteen voxelizing waves a CU and
+// five preparing; with four and one a workgroup's registers allow four
+// workgroups a CU, and the hall took 2050 instead of 1800 us as a whole):
+// hall (1536x1024x768, 1.4 M triangles) 849 -> 650 us, room 512x403x303
+// 198 -> 168 us, LongFCC room 640x255x384 417 -> 316 us, 64-mesh batch
+// 1835 -> 1400 us, 132 large triangles over 672x515x387 278 -> 147 us,
+// sphere 128^3 24.4 -> 19.0 us.
 constexpr int kDppQuadSwap1 = 0xB1, kDppQuadSwap2 = 0x4E, kDppHalfMirror = 0x141;
 
+// What the voxelizing waves need to know of a chunk.
+struct BrickStep {
+    uint32_t valid;         // 0: the list is done
+    uint32_t ends;          // bit 0: the brick's first chunk, bit 1: its last
+    uint32_t job, brick;    // brick within the job
+    uint32_t bx, by, bz;    // its coordinates
+    uint32_t layers;        // z0 | z1 << 16
+    uint32_t total, ntri;   // work items, triangles with items
+};
+
 template <bool kKeys>
-__global__ __launch_bounds__(256, 5) void k_surf_brick(
+__global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
     const Job *__restrict__ jobs, const uint32_t *__restrict__ brick_bases, uint32_t njobs,
     const float4 *__restrict__ tri_rec, const uint32_t *__restrict__ brick_off,
     const uint32_t *__restrict__ brick_hist, const uint32_t *__restrict__ blist,
@@ -1063,234 +1083,317 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
     uint64_t *__restrict__ cycles) {
     __shared__ __align__(16) uint32_t keys[kMaxBrickVox];
     __shared__ SurfTri tris[kSurfChunk];
-    __shared__ uint32_t cstart[kSurfChunk], ctotal[2], smask[256 / kWave][2];
+    __shared__ uint32_t cstart[kSurfChunk], smask[kBrickWaves][2];
     __shared__ uint8_t cslot[kSurfChunk];
-    // Per wave the columns that await their depth part; in the epilogue the
-    // brick's surface words.
-    __shared__ uint32_t wqueue[256 / kWave][2 * kWave];
-    uint32_t *wsurf = &wqueue[0][0];
-    static_assert(sizeof(wqueue) >= kMaxBrickVox / 8, "surface words fit the queues");
-    __shared__ uint8_t touched[32];
-    __shared__ uint32_t s_q, s_qe;
+    __shared__ uint32_t wqueue[kBrickWaves][2 * kWave];  // columns that await their depth part
+    __shared__ uint8_t touched[2][32];  // rows with a key, of this brick and (cleared) the next
+    __shared__ BrickStep step;
     __shared__ SplitTable spl;
-    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-    for (int32_t i = tid; i < kMaxBrickVox; i += blockDim.x) keys[i] = 0u;
-    if (tid < 32u) touched[tid] = 0;
-    if (tid < 2u * (256u / kWave)) (&smask[0][0])[tid] = 0u;
-    // Entries: the heavy list first (learned order), then the plain list.
-    const uint32_t nh = hlist ? *n_heavy : 0u;
-    const uint32_t n_list = *n_order + nh;
-    // Guided grabs: a workgroup takes a run of list entries sized to the
-    // work left (remaining / (8 * workgroups), 1..32; heavy entries one at a
-    // time), so the shared counter sees a few grabs per workgroup rather
-    // than one per brick (one address bumped per brick serialises the pass),
-    // while the tail still goes one brick at a time.
-    auto grab = [&](uint32_t seen, uint32_t &qe) {
-        const uint32_t left = n_list > seen ? n_list - seen : 0u;
-        const uint32_t k = seen < nh ? 1u : min(max(left / (8u * gridDim.x), 1u), 32u);
-        const uint32_t q0 = atomicAdd(next, k);
-        qe = min(q0 + k, n_list);
-        return q0;
-    };
-    if (tid == 0) {
-        uint32_t qe;
-        s_q = grab(0u, qe);
-        s_qe = qe;
-    }
-    __syncthreads();
-    uint32_t q = s_q, qend = s_qe;
-    uint32_t cur_job = UINT32_MAX;  // job whose split table is in LDS
-    uint32_t nsurf = 0u;            // surface voxels found by this lane
-    while (q < n_list) {  // q and qend are uniform over the block
-        uint32_t q_next = q + 1u, qe_next = qend;
-        if (tid == 0 && q + 1u >= qend) q_next = grab(qend, qe_next);  // next run, early
-        // The brick's header comes through uniform (scalar) loads, which do
-        // not wait behind the previous brick's outstanding vector stores.
-        const uint32_t qs = __builtin_amdgcn_readfirstlane(q);
-        const bool from_heavy = qs < nh;
-        const uint32_t gb =
-            __builtin_amdgcn_readfirstlane(from_heavy ? hlist[qs] : order[qs - nh]);
-        // A plain entry already taken from the heavy list is passed over
-        // (its flag byte read as part of an aligned dword, uniformly).
-        const bool skipped =
-            !from_heavy && hlist &&
-            ((__builtin_amdgcn_readfirstlane(
-                  ((const uint32_t *)skip)[(qs - nh) >> 2]) >> (8u * ((qs - nh) & 3u))) & 0xFFu);
-        // Layer range of the entry: a heavy entry may be a sub-brick.
-        const uint32_t sub =
-            from_heavy ? __builtin_amdgcn_readfirstlane(hsub[qs]) : 0xFFFF0000u;
-        if (!skipped) {
-            const uint32_t cnt = __builtin_amdgcn_readfirstlane(brick_hist[gb]);
-            uint64_t t_start = 0;
-            if (cycles && tid == 0) t_start = __builtin_amdgcn_s_memtime();
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    for (uint32_t i = tid; i < (uint32_t)kMaxBrickVox; i += kBrickThreads) keys[i] = 0u;
+    if (tid < 64u) (&touched[0][0])[tid] = 0;
+    if (tid < 2u * kBrickWaves) (&smask[0][0])[tid] = 0u;
+
+    if (wave == kBrickWaves) {
+        // ---- the preparing wave ----
+        const uint32_t nh = hlist ? *n_heavy : 0u;
+        const uint32_t n_list = *n_order + nh;  // heavy entries first, then the plain list
+        // Every workgroup starts with the entry of its own number; the rest
+        // lies in kBrickLists parts, each with a counter that a workgroup
+        // draws its next entry or two from: its own part's first (part and
+        // XCD have the same number), then the others' when that is used up.
+        // One counter bound the pass at 14-18 ns a draw (room 195 us against
+        // 166 with eight), which longer runs only trade for imbalance: runs
+        // of up to 16, 8, 4, 2 and 1 took 866, 658, 644, 640 and 660 us on
+        // the hall, 16 and 32 counters no less than eight.
+        const uint32_t dealt = min(gridDim.x, n_list);
+        const uint32_t part = (n_list - dealt + kBrickLists - 1u) / kBrickLists;
+        uint32_t list = blockIdx.x % kBrickLists, tried = 0u;
+        // The run in hand, an entry per lane: brick, pairs, first pair, layers.
+        uint32_t gb = 0u, cnt = 0u, off = 0u, sub = 0u;
+        uint32_t rn = 0u, ri = 0u;
+        // The next run on its way: its first entry (pending 1: being drawn),
+        // its bricks (2: being read).
+        uint32_t q0 = blockIdx.x, qk = 1u, qend = n_list, pending = 1u;
+        uint32_t ngb = 0u, nsub = 0u;
+        bool nskip = false;
+        auto draw = [&](uint32_t seen) {  // seen: entries of the list before this were drawn
+            const uint32_t lo = min(dealt + list * part, n_list);
+            qend = min(dealt + (list + 1u) * part, n_list);
+            const uint32_t left = qend - min(max(seen, lo), qend);
+            qk = left * kBrickLists / (32u * gridDim.x) > 1u ? 2u : 1u;
+            if (lane == 0u) q0 = lo + atomicAdd(next + list * kBrickListPitch, qk);
+            pending = 1u;
+        };
+        auto bricks_of_run = [&]() {  // pending 1 -> 2
+            q0 = __builtin_amdgcn_readfirstlane(q0);
+            while (q0 >= qend && tried < kBrickLists) {
+                list = list + 1u < kBrickLists ? list + 1u : 0u;
+                tried++;
+                draw(0u);
+                q0 = __builtin_amdgcn_readfirstlane(q0);
+            }
+            qk = q0 < qend ? min(qk, qend - q0) : 0u;
+            const uint32_t q = q0 + lane;
+            ngb = 0u;
+            nsub = 0xFFFF0000u;
+            nskip = lane >= qk;
+            if (!nskip) {
+                if (q < nh) {
+                    ngb = hlist[q];
+                    nsub = hsub[q];
+                } else {
+                    ngb = order[q - nh];
+                    // A plain entry already taken from the heavy list is passed over.
+                    if (hlist) nskip = skip[q - nh] != 0;
+                }
+            }
+            pending = 2u;
+        };
+        // The chunk in preparation.
+        uint32_t cb = 0u, ccnt = 0u, coff = 0u, csub = 0u, c0 = 0u;
+        bool more = true, first = false;
+        uint32_t cjob = 0u, spl_job = UINT32_MAX;
+        float4 r0, r1, r2;
+        uint32_t t = 0u;
+        auto fetch = [&]() {  // the next chunk's triangles
+            first = false;
+            if (c0 + kSurfChunk < ccnt) {
+                c0 += kSurfChunk;
+            } else {
+                ccnt = 0u;
+                while (ccnt == 0u) {
+                    if (ri == rn) {
+                        if (pending == 1u) bricks_of_run();
+                        rn = qk;
+                        ri = 0u;
+                        if (rn == 0u) {
+                            more = false;
+                            return;
+                        }
+                        gb = ngb;
+                        sub = nsub;
+                        cnt = nskip ? 0u : brick_hist[gb];
+                        off = nskip ? 0u : brick_off[gb];
+                        pending = 0u;
+                    }
+                    cb = (uint32_t)__builtin_amdgcn_readlane((int)gb, (int)ri);
+                    ccnt = (uint32_t)__builtin_amdgcn_readlane((int)cnt, (int)ri);
+                    coff = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)ri);
+                    csub = (uint32_t)__builtin_amdgcn_readlane((int)sub, (int)ri);
+                    ri++;
+                    if (ri == rn) draw(q0 + rn);  // the next run, early
+                }
+                c0 = 0u;
+                first = true;
+            }
+            if (c0 + lane < ccnt) {
+                t = blist[coff + c0 + lane];
+                r0 = tri_rec[3 * (size_t)t];
+                r1 = tri_rec[3 * (size_t)t + 1];
+                r2 = tri_rec[3 * (size_t)t + 2];
+            }
+        };
+        auto publish = [&]() {
+            if (!more) {
+                if (lane == 0u) step.valid = 0u;
+                return;
+            }
             // Consecutive entries mostly share a job: its range is tested
             // before a search.
-            const uint32_t j =
-                njobs > 1u && cur_job != UINT32_MAX && gb >= brick_bases[cur_job] &&
-                        gb < brick_bases[cur_job + 1u]
-                    ? cur_job
-                    : job_of(brick_bases, njobs, gb);
-            const Job &J = jobs[j];
-            if (j != cur_job) {  // uniform: the job's matSplitRes table into LDS
-                __syncthreads();
+            if (njobs > 1u && !(spl_job != UINT32_MAX && cb >= brick_bases[cjob] &&
+                                cb < brick_bases[cjob + 1u]))
+                cjob = job_of(brick_bases, njobs, cb);
+            const Job &J = jobs[cjob];
+            if (cjob != spl_job) {  // the job's matSplitRes table into LDS
                 const VK_G uint32_t *src = (const VK_G uint32_t *)gptr(J.splits);
                 uint32_t *dst = (uint32_t *)&spl;
-                for (uint32_t i = tid; i < sizeof(SplitTable) / 4; i += blockDim.x) dst[i] = src[i];
-                cur_job = j;
+                for (uint32_t i = lane; i < sizeof(SplitTable) / 4; i += kWave) dst[i] = src[i];
+                spl_job = cjob;
+                wave_lds_sync();
             }
             const SurfParams p = surf_params(J);
-            const VK_G uint8_t *__restrict__ materials = gptr(J.mats);
-            const bool embed = J.embed != 0;
-            const uint32_t b = gb - J.brick_base;  // brick within the job
-            const int32_t bd0 = p.bdim[0], bd1 = p.bdim[1], bd2 = p.bdim[2];
-            const int32_t nvox = bd0 * bd1 * bd2;
-            const int32_t z0 = (int32_t)(sub & 0xFFFFu), z1 = min((int32_t)(sub >> 16), bd2);
-            const int32_t wpr = bd0 / 32;     // words per row
-            const int32_t row_shift = 31 - __clz(bd0);
-            const uint32_t bxi = b % p.nb[0], byi = (b / p.nb[0]) % p.nb[1],
-                           bzi = b / (p.nb[0] * p.nb[1]);
+            const uint32_t b = cb - J.brick_base;
+            const uint32_t bx = b % p.nb[0], by = (b / p.nb[0]) % p.nb[1],
+                           bz = b / (p.nb[0] * p.nb[1]);
+            const uint32_t z0 = csub & 0xFFFFu, z1 = min(csub >> 16, (uint32_t)p.bdim[2]);
             // Bricks are laid over alloc coordinates; ext = alloc - off.
-            const int32_t blx = (int32_t)(bxi * bd0) - p.off[0],
-                          bly = (int32_t)(byi * bd1) - p.off[1],
-                          blz = (int32_t)(bzi * bd2) - p.off[2];
-            const int32_t nwords = nvox / 32;
-            // This thread's brick word (for the OR into the solid grid), early;
-            // a sub-brick owns the words of its layers only.
-            size_t gi = 0;
-            bool gword = false;
-            uint32_t bw = 0u;
-            if ((int32_t)tid < nwords) {
-                const int32_t wx = (int32_t)tid % wpr, ly = ((int32_t)tid / wpr) % bd1,
-                              lz = (int32_t)tid / (wpr * bd1);
-                const uint32_t aw = bxi * (uint32_t)wpr + (uint32_t)wx;
-                const uint32_t ay = byi * (uint32_t)bd1 + (uint32_t)ly;
-                const uint32_t az = bzi * (uint32_t)bd2 + (uint32_t)lz;
-                gword = lz >= z0 && lz < z1 && aw < p.alloc[0] / 32u && ay < p.alloc[1] &&
-                        az < p.alloc[2];
-                if (gword) {
-                    gi = ((size_t)az * p.alloc[1] + ay) * (p.alloc[0] / 32u) + aw;
-                    bw = gptr(J.bits)[gi];
-                }
+            uint32_t items = 0u;
+            if (c0 + lane < ccnt)
+                items = surf_tri_setup(p, J.fdiv != 0, spl, r0, r1, r2, t - J.tri_base,
+                                       J.embed != 0, (int32_t)(bx * p.bdim[0]) - p.off[0],
+                                       (int32_t)(by * p.bdim[1]) - p.off[1],
+                                       (int32_t)(bz * p.bdim[2]) - p.off[2], (int32_t)z0,
+                                       (int32_t)z1, tris[lane]);
+            static_assert(kSurfChunk == kWave, "one wave sets up a chunk");
+            const uint32_t incl = wave_incl_scan(items);
+            // The triangles with items, in order: first item and LDS slot.
+            const unsigned long long nz = __ballot(items != 0u);
+            if (items) {
+                const uint32_t r = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(nz >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)nz, 0u));
+                cstart[r] = incl - items;
+                cslot[r] = (uint8_t)lane;
             }
-            const uint32_t off = __builtin_amdgcn_readfirstlane(brick_off[gb]);
-            for (uint32_t c0 = 0; c0 < cnt; c0 += kSurfChunk) {
-                __syncthreads();
-                if (tid < (uint32_t)kSurfChunk) {
-                    uint32_t items = 0u;
-                    if (c0 + tid < cnt) {
-                        const uint32_t t = blist[off + c0 + tid];
-                        items = surf_tri_setup(p, J.fdiv != 0, spl, tri_rec, t, J.tri_base, embed,
-                                               blx, bly, blz, z0, z1, tris[tid]);
-                    }
-                    static_assert(kSurfChunk == kWave, "one wave sets up a chunk");
-                    const uint32_t incl = wave_incl_scan(items);
-                    // The triangles with items, in order: first item and LDS slot.
-                    const unsigned long long nz = __ballot(items != 0u);
-                    if (items) {
-                        const uint32_t r = __builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(nz >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)nz, 0u));
-                        cstart[r] = incl - items;
-                        cslot[r] = (uint8_t)tid;
-                    }
-                    if (tid == (uint32_t)kSurfChunk - 1u) {
-                        ctotal[0] = incl;
-                        ctotal[1] = (uint32_t)__popcll(nz);
-                    }
-                }
-                __syncthreads();
-                const uint32_t total = ctotal[0], ntri = ctotal[1];
-                // Lane j holds the first item of the j-th triangle with items
-                // (strictly increasing in j) and its slot.  A wave takes 64
-                // consecutive items at a time: the triangle of its first item
-                // is a ballot over the held starts, and each lane adds the
-                // triangles starting between the first item and its own, read
-                // from a 64-bit mask of start offsets that the starting lanes
-                // OR together in LDS.
-                const uint32_t cs = lane < ntri ? cstart[lane] : UINT32_MAX;
-                const uint32_t sl = lane < ntri ? (uint32_t)cslot[lane] : 0u;
-                uint32_t *sm = &smask[wave][0], *wq = wqueue[wave];
-                uint32_t nq = 0u;  // columns in the wave's queue (uniform)
-                auto depth = [&](uint32_t e) {
-                    surf_depth(p, spl, tris[e >> 24], e & 0xFFFu, (e >> 12) & 0xFFFu, keys, touched,
-                               (uint32_t)nvox, (uint32_t)row_shift);
-                };
-                for (uint32_t w0 = wave * kWave; w0 < total; w0 += blockDim.x) {  // uniform
-                    const uint32_t t0 = (uint32_t)__popcll(__ballot(cs <= w0)) - 1u;
-                    const uint32_t ps = cs - w0 - 1u;  // start offset - 1, in 0..62
-                    if (cs > w0 && ps < kWave - 1u) atomicOr(&sm[ps >> 5], 1u << (ps & 31u));
-                    const uint32_t m_lo = sm[0], m_hi = sm[1];
-                    if (lane == 0u) {
-                        sm[0] = 0u;
-                        sm[1] = 0u;
-                    }
-                    const uint32_t ti =
-                        t0 + __builtin_amdgcn_mbcnt_hi(m_hi, __builtin_amdgcn_mbcnt_lo(m_lo, 0u));
-                    const uint32_t slot = (uint32_t)__shfl((int)sl, (int)ti);
-                    const uint32_t first = (uint32_t)__shfl((int)cs, (int)ti);
-                    const uint32_t c = w0 + lane;
-                    uint32_t cu = 0u, cv = 0u;
-                    const bool deep =
-                        c < total && surf_column(p, tris[slot], c - first, keys, touched,
-                                                 (uint32_t)nvox, (uint32_t)row_shift, cu, cv);
-                    const unsigned long long dm = __ballot(deep);
-                    if (deep)
-                        wq[nq + __builtin_amdgcn_mbcnt_hi(
-                                    (uint32_t)(dm >> 32),
-                                    __builtin_amdgcn_mbcnt_lo((uint32_t)dm, 0u))] =
-                            slot << 24 | cv << 12 | cu;
-                    nq += (uint32_t)__popcll(dm);
-                    wave_lds_sync();
-                    if (nq >= (uint32_t)kWave) {
-                        nq -= (uint32_t)kWave;
-                        depth(wq[nq + lane]);
-                        wave_lds_sync();
-                    }
-                }
-                if (lane < nq) depth(wq[lane]);
+            if (lane == kWave - 1u)
+                step = BrickStep{1u, (first ? 1u : 0u) | (c0 + kSurfChunk >= ccnt ? 2u : 0u),
+                                 cjob, b, bx, by, bz, z0 | z1 << 16, incl,
+                                 (uint32_t)__popcll(nz)};
+        };
+        fetch();
+        publish();
+        while (true) {
+            __syncthreads();  // the step is set up
+            if (!more) return;
+            fetch();
+            __syncthreads();  // its items are done
+            publish();
+            if (pending == 1u) bricks_of_run();
+        }
+    }
+
+    // ---- the voxelizing waves ----
+    uint32_t nsurf = 0u;  // surface voxels found by this lane
+    uint32_t par = 1u;
+    uint64_t t_start = 0;
+    while (true) {
+        __syncthreads();  // the step is set up
+        if (__builtin_amdgcn_readfirstlane(step.valid) == 0u) break;
+        const uint32_t ends = __builtin_amdgcn_readfirstlane(step.ends);
+        const uint32_t b = __builtin_amdgcn_readfirstlane(step.brick);
+        const uint32_t total = __builtin_amdgcn_readfirstlane(step.total),
+                       ntri = __builtin_amdgcn_readfirstlane(step.ntri);
+        const uint32_t bx = __builtin_amdgcn_readfirstlane(step.bx),
+                       by = __builtin_amdgcn_readfirstlane(step.by),
+                       bz = __builtin_amdgcn_readfirstlane(step.bz),
+                       layers = __builtin_amdgcn_readfirstlane(step.layers);
+        const Job &J = jobs[__builtin_amdgcn_readfirstlane(step.job)];
+        const SurfParams p = surf_params(J);
+        const uint32_t nvox = (uint32_t)(p.bdim[0] * p.bdim[1] * p.bdim[2]);
+        const uint32_t row_shift = 31u - (uint32_t)__clz(p.bdim[0]);
+        if (ends & 1u) {
+            par ^= 1u;
+            if (tid < 32u) touched[par ^ 1u][tid] = 0;  // the previous brick's
+            if (cycles && tid == 0u) t_start = __builtin_amdgcn_s_memtime();
+        }
+        // Lane j holds the first item of the j-th triangle with items
+        // (strictly increasing in j) and its slot.  A wave takes 64
+        // consecutive items at a time: the triangle of its first item
+        // is a ballot over the held starts, and each lane adds the
+        // triangles starting between the first item and its own, read
+        // from a 64-bit mask of start offsets that the starting lanes
+        // OR together in LDS.
+        const uint32_t cs = lane < ntri ? cstart[lane] : UINT32_MAX;
+        const uint32_t sl = lane < ntri ? (uint32_t)cslot[lane] : 0u;
+        uint32_t *sm = &smask[wave][0], *wq = wqueue[wave];
+        uint8_t *rows = touched[par];
+        uint32_t nq = 0u;  // columns in the wave's queue (uniform)
+        auto depth = [&](uint32_t e) {
+            surf_depth(p, spl, tris[e >> 24], e & 0xFFFu, (e >> 12) & 0xFFFu, keys, rows, nvox,
+                       row_shift);
+        };
+        for (uint32_t w0 = wave * kWave; w0 < total; w0 += kBrickWaves * kWave) {  // uniform
+            const uint32_t t0 = (uint32_t)__popcll(__ballot(cs <= w0)) - 1u;
+            const uint32_t ps = cs - w0 - 1u;  // start offset - 1, in 0..62
+            if (cs > w0 && ps < kWave - 1u) atomicOr(&sm[ps >> 5], 1u << (ps & 31u));
+            const uint32_t m_lo = sm[0], m_hi = sm[1];
+            if (lane == 0u) {
+                sm[0] = 0u;
+                sm[1] = 0u;
             }
-            __syncthreads();
-            // Surface bit words and winner materials, 256 voxels per wave
-            // step: each lane takes 4 consecutive voxels (one 16-byte LDS
-            // read of their keys), the 8 lanes of a 32-voxel word OR their
-            // nibbles together, and each lane of a word holding a surface
-            // voxel writes its 4 material bytes as one dword of the brick's
-            // block in the material grid (the winner's material, 0 for the
-            // word's other voxels).  Steps whose rows received no key only
-            // zero their surface words.  Keys are cleared for the next brick.
-            // With materials in the keys the loop issues no global loads, so
-            // its stores never wait (a wait for a load also waits for earlier
-            // stores here).
-            VK_G uint32_t *__restrict__ mg =
-                (VK_G uint32_t *)(gptr(J.matgrid) + (size_t)b * (uint32_t)nvox);
-            VK_G u32x4 *__restrict__ kg =
-                kKeys && J.keygrid ? (VK_G u32x4 *)(gptr(J.keygrid) + (size_t)b * (uint32_t)nvox)
-                                   : nullptr;
-            const uint32_t tmask = (uint32_t)__ballot(lane < 32u && touched[lane & 31u] != 0);
-            const uint32_t rows_per_step = 256u >> row_shift;  // bd0 >= 64: 1, 2 or 4 rows
-            auto rows_out = [&](auto embed_c) {
-                constexpr bool kEmbedded = decltype(embed_c)::value;
-                for (int32_t v0 = (int32_t)wave * 256; v0 < nvox; v0 += 1024) {
-                    const uint32_t rmask = ((1u << rows_per_step) - 1u) << (v0 >> row_shift);
-                    if (!(tmask & rmask)) {
-                        if (lane < 8u) wsurf[(v0 >> 5) + (int32_t)lane] = 0u;
-                        continue;
-                    }
-                    uint4 *kp = (uint4 *)&keys[v0 + 4 * (int32_t)lane];
-                    const uint4 kv = *kp;
-                    const uint32_t nib = (kv.x ? 8u : 0u) | (kv.y ? 4u : 0u) | (kv.z ? 2u : 0u) |
-                                         (kv.w ? 1u : 0u);
-                    // OR over the word's 8 lanes in registers (DPP): the
-                    // quad swaps [1,0,3,2] and [2,3,0,1], then the half-row
-                    // mirror (lane i <-> 7 - i) joins the two quads.
-                    uint32_t w = nib << (28u - 4u * (lane & 7u));
-                    w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppQuadSwap1, 0xF, 0xF, false);
-                    w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppQuadSwap2, 0xF, 0xF, false);
-                    w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppHalfMirror, 0xF, 0xF, false);
-                    if ((lane & 7u) == 0u) wsurf[(v0 >> 5) + (int32_t)(lane >> 3)] = w;
-                    if (!w) continue;
+            const uint32_t ti =
+                t0 + __builtin_amdgcn_mbcnt_hi(m_hi, __builtin_amdgcn_mbcnt_lo(m_lo, 0u));
+            const uint32_t slot = (uint32_t)__shfl((int)sl, (int)ti);
+            const uint32_t start = (uint32_t)__shfl((int)cs, (int)ti);
+            const uint32_t c = w0 + lane;
+            uint32_t cu = 0u, cv = 0u;
+            const bool deep = c < total && surf_column(p, tris[slot], c - start, keys, rows, nvox,
+                                                       row_shift, cu, cv);
+            const unsigned long long dm = __ballot(deep);
+            if (deep)
+                wq[nq + __builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(dm >> 32),
+                            __builtin_amdgcn_mbcnt_lo((uint32_t)dm, 0u))] =
+                    slot << 24 | cv << 12 | cu;
+            nq += (uint32_t)__popcll(dm);
+            wave_lds_sync();
+            if (nq >= (uint32_t)kWave) {
+                nq -= (uint32_t)kWave;
+                depth(wq[nq + lane]);
+                wave_lds_sync();
+            }
+        }
+        if (lane < nq) depth(wq[lane]);
+        __syncthreads();  // the step's items are done
+        if (!(ends & 2u)) continue;
+        // The brick's rows, 256 voxels per wave step: each lane takes 4
+        // consecutive voxels (one 16-byte LDS read of their keys), the 8
+        // lanes of a 32-voxel word OR their nibbles together, and each lane
+        // of a word holding a surface voxel writes its 4 material bytes as
+        // one dword of the brick's block in the material grid (the winner's
+        // material, 0 for the word's other voxels).  Steps whose rows
+        // received no key are passed over.  Keys are cleared for the next
+        // brick.  With materials in the keys the loop issues no global loads,
+        // so its stores never wait (a wait for a load also waits for earlier
+        // stores here).
+        VK_G uint32_t *__restrict__ bits = gptr(J.bits);
+        VK_G uint32_t *__restrict__ mg =
+            (VK_G uint32_t *)(gptr(J.matgrid) + (size_t)b * nvox);
+        VK_G u32x4 *__restrict__ kg =
+            kKeys && J.keygrid ? (VK_G u32x4 *)(gptr(J.keygrid) + (size_t)b * nvox) : nullptr;
+        VK_G uint32_t *__restrict__ surf = kKeys ? gptr(J.surf) : nullptr;
+        const VK_G uint8_t *__restrict__ materials = gptr(J.mats);
+        const bool embed = J.embed != 0;
+        const uint32_t z0 = layers & 0xFFFFu, z1 = layers >> 16;
+        const uint32_t lwx = row_shift - 5u, lby = 31u - (uint32_t)__clz(p.bdim[1]);
+        const uint32_t aw0 = bx << lwx, ay0 = by << lby, az0 = bz * (uint32_t)p.bdim[2];
+        const uint32_t W = p.alloc[0] / 32u;
+        const bool whole = z0 == 0u && z1 == (uint32_t)p.bdim[2];
+        VK_G uint8_t *wm = (VK_G uint8_t *)gptr(J.wmask) + (size_t)b * 16u;
+        const uint32_t tmask = (uint32_t)__ballot(lane < 32u && rows[lane & 31u] != 0);
+        const uint32_t rows_per_step = 256u >> row_shift;  // bd0 >= 64: 1, 2 or 4 rows
+        for (uint32_t v0 = wave * 256u; v0 < nvox; v0 += kBrickWaves * 256u) {
+            const uint32_t rmask = (rows_per_step > 1u ? (1u << rows_per_step) - 1u : 1u)
+                                   << (v0 >> row_shift);
+            // This lane's word and its place in the grid.
+            const uint32_t wi = (v0 >> 5) + (lane >> 3);
+            const uint32_t aw = aw0 + (wi & ((1u << lwx) - 1u)),
+                           ay = ay0 + ((wi >> lwx) & ((1u << lby) - 1u)),
+                           lz = wi >> (lwx + lby), az = az0 + lz;
+            const size_t gi = ((size_t)az * p.alloc[1] + ay) * W + aw;
+            uint32_t w = 0u;
+            if (tmask & rmask) {  // uniform
+                uint4 *kp = (uint4 *)&keys[v0 + 4u * lane];
+                const uint4 kv = *kp;
+                const uint32_t nib = (kv.x ? 8u : 0u) | (kv.y ? 4u : 0u) | (kv.z ? 2u : 0u) |
+                                     (kv.w ? 1u : 0u);
+                // OR over the word's 8 lanes in registers (DPP): the
+                // quad swaps [1,0,3,2] and [2,3,0,1], then the half-row
+                // mirror (lane i <-> 7 - i) joins the two quads.
+                w = nib << (28u - 4u * (lane & 7u));
+                w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppQuadSwap1, 0xF, 0xF, false);
+                w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppQuadSwap2, 0xF, 0xF, false);
+                w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, kDppHalfMirror, 0xF, 0xF, false);
+                // The words with a surface voxel: bit 8 i of the ballot is
+                // word i of the step, gathered into its byte of the brick's
+                // word mask (cleared each call; a part of a cut brick shares it).
+                const unsigned long long wb = __ballot(w != 0u) & 0x0101010101010101ull;
+                const uint32_t byte = (uint32_t)((wb * 0x0102040810204080ull) >> 56);
+                if (lane == 0u && byte) {
+                    if (whole)
+                        wm[v0 >> 8] = (uint8_t)byte;
+                    else
+                        atomicOr((uint32_t *)(J.wmask + (size_t)b * 4u + (v0 >> 10)),
+                                 byte << ((v0 >> 5) & 24u));
+                }
+                if (w) {
+                    if ((lane & 7u) == 0u)
+                        __hip_atomic_fetch_or(bits + gi, w, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
                     nsurf += (uint32_t)__popc(nib);
                     uint32_t m;
-                    if (kEmbedded) {
+                    if (embed) {
                         m = (kv.x & 0xFFu) | (kv.y & 0xFFu) << 8 | (kv.z & 0xFFu) << 16 |
                             (kv.w & 0xFFu) << 24;
                     } else {
@@ -1300,39 +1403,16 @@ __global__ __launch_bounds__(256, 5) void k_surf_brick(
                         m = mat(kv.x) | mat(kv.y) << 8 | mat(kv.z) << 16 | mat(kv.w) << 24;
                     }
                     if (nib) *kp = make_uint4(0u, 0u, 0u, 0u);
-                    mg[(v0 >> 2) + (int32_t)lane] = m;
-                    if (kKeys && kg) kg[(v0 >> 2) + (int32_t)lane] = u32x4{kv.x, kv.y, kv.z, kv.w};
+                    mg[(v0 >> 2) + lane] = m;
+                    if (kKeys && kg) kg[(v0 >> 2) + lane] = u32x4{kv.x, kv.y, kv.z, kv.w};
                 }
-            };
-            if (embed)
-                rows_out(std::integral_constant<bool, true>{});
-            else
-                rows_out(std::integral_constant<bool, false>{});
-            __syncthreads();
-            const uint32_t sw = gword ? wsurf[tid] : 0u;
-            if (gword) {
-                if (J.surf) gptr(J.surf)[gi] = sw;
-                if (sw) gptr(J.bits)[gi] = bw | sw;
             }
-            // The brick's word mask (words of other layers belong to other
-            // parts of a cut brick, hence the OR into a cleared mask).
-            const unsigned long long hm = __ballot(sw != 0u);
-            if (wave < 2u && lane == 0u && hm) {
-                uint32_t *wm = J.wmask + (size_t)b * 4u + 2u * wave;
-                if ((uint32_t)hm) atomicOr(wm, (uint32_t)hm);
-                if ((uint32_t)(hm >> 32)) atomicOr(wm + 1, (uint32_t)(hm >> 32));
-            }
-            if (cycles && tid == 0) cycles[gb] = __builtin_amdgcn_s_memtime() - t_start;
-        }  // brick
-        __syncthreads();
-        if (tid < 32u) touched[tid] = 0;
-        if (tid == 0) {
-            s_q = q_next;
-            s_qe = qe_next;
+            if (kKeys && surf && (lane & 7u) == 0u && lz >= z0 && lz < z1 && aw < W &&
+                ay < p.alloc[1] && az < p.alloc[2])
+                surf[gi] = w;
         }
-        __syncthreads();
-        q = s_q;
-        qend = s_qe;
+        if (cycles && tid == 0u)
+            cycles[J.brick_base + b] = __builtin_amdgcn_s_memtime() - t_start;
     }
     // One atomic per wave at exit: a shared counter bumped per brick would
     // serialise every workgroup on one address.

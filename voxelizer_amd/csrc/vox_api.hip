@@ -140,17 +140,11 @@ struct vox_ctx {
     std::vector<float> rec_feats, rec_cycles;
     // worker contexts of batched runs (same device, own streams and buffers)
     std::vector<vox_ctx *> workers;
-    // per-triangle-slot vertex records and job ids of the current call
-    float4 *rec = nullptr;
-    uint32_t *tri_job = nullptr;
-    // pinned staging area of job-table uploads, and the event of the last one
+    // pinned staging area of job-table uploads; busy until the stream was
+    // waited for after the last one
     void *up = nullptr;
     size_t up_cap = 0;
-    hipEvent_t up_ev = nullptr;
-    // The surface stage's preparation (setup, binning, brick order) runs on
-    // `side` beside the solid stage; fork and join through these events.
-    hipStream_t side = nullptr, main_stream = nullptr;  // main_stream: `stream` as created
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    bool up_busy = false;
     // surface brick shapes (voxels along x, y, z)
     int cart_bdim[3] = {kCartBX, kCartBY, kCartBZ};
     // meshes with fewer triangles carry materials in the surface pass's
@@ -258,10 +252,8 @@ vox_status buf(vox_ctx *ctx, const char *name, size_t count, T **out) {
     }
     Buf &b = ctx->bufs[name];
     if (bytes > b.cap) {
-        if (b.p) {  // either stream may still use the old buffer
+        if (b.p) {  // the stream may still use the old buffer
             VOX_HIP(hipStreamSynchronize(ctx->stream));
-            if (ctx->side && ctx->side != ctx->stream) VOX_HIP(hipStreamSynchronize(ctx->side));
-            if (ctx->side && ctx->stream == ctx->side) VOX_HIP(hipStreamSynchronize(ctx->main_stream));
             VOX_HIP(hipFree(b.p));
             b.p = nullptr;
             b.cap = 0;
@@ -295,79 +287,71 @@ vox_status fill(vox_ctx *ctx, uint32_t *p, size_t n, uint32_t v) {
     return VOX_OK;
 }
 
-// Several fills in one launch (each launch on the stream costs a few
-// microseconds whatever its size).
 struct FillSeg {
     uint32_t *p;
     size_t n;
     uint32_t v;
 };
-constexpr int kMaxFillSegs = 6;
-struct FillSegs {
-    uint32_t *p[kMaxFillSegs];
-    size_t n[kMaxFillSegs];
-    uint32_t v[kMaxFillSegs];
-    int count;
-};
-__global__ void k_fill_many(FillSegs s) {
-    for (int k = 0; k < s.count; k++)
-        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < s.n[k];
-             i += (size_t)gridDim.x * blockDim.x)
-            s.p[k][i] = s.v[k];
+__global__ void k_fill_many(FillSegs s) { fill_segs(s, blockIdx.x, gridDim.x); }
+// The table of the segments that hold anything; returns the longest's length.
+size_t fill_table(const FillSeg *segs, size_t n, FillSegs &s) {
+    s.count = 0;
+    size_t most = 0;
+    for (size_t k = 0; k < n && s.count < kMaxFillSegs; k++) {
+        if (segs[k].n == 0 || !segs[k].p) continue;
+        s.p[s.count] = segs[k].p;
+        s.n[s.count] = segs[k].n;
+        s.v[s.count] = segs[k].v;
+        s.count++;
+        most = std::max(most, segs[k].n);
+    }
+    return most;
 }
 vox_status fill_many(vox_ctx *ctx, std::initializer_list<FillSeg> segs) {
     FillSegs s;
-    s.count = 0;
-    size_t most = 0;
-    for (const FillSeg &f : segs) {
-        if (f.n == 0 || !f.p) continue;
-        if (s.count == kMaxFillSegs) return fail(ctx, VOX_ERR_INVALID, "too many fill segments");
-        s.p[s.count] = f.p;
-        s.n[s.count] = f.n;
-        s.v[s.count] = f.v;
-        s.count++;
-        most = std::max(most, f.n);
-    }
+    const size_t most = fill_table(segs.begin(), segs.size(), s);
     if (s.count == 0) return VOX_OK;
     k_fill_many<<<grid_for(most, 256, 4096), 256, 0, ctx->stream>>>(s);
     VOX_HIP(hipGetLastError());
     return VOX_OK;
 }
 
-// Exclusive scan of in[0,n) into out[0,n+1]: out[n] is the total mod 2^32,
-// out[n+1] is 1 if the true total reached 2^32 (see k_scan_down).
-vox_status scan(vox_ctx *ctx, const uint32_t *in, uint32_t *out, uint32_t n, int depth = 0) {
-    const uint32_t nblocks = n / kScanTile + 1;
-    char name[32];
-    const char *tag = ctx->stream == ctx->side ? "b" : "";  // one set per stream
-    std::snprintf(name, sizeof(name), "scan%s_part%d", tag, depth);
-    uint32_t *part;
-    VOX_TRY(buf(ctx, name, 2 * (size_t)nblocks + 1, &part));
-    if (nblocks <= kScanDirectTiles) {
-        if (nblocks > 1) {
-            k_scan_reduce<<<nblocks, kScanThreads, 0, ctx->stream>>>(in, n, part);
-            VOX_HIP(hipGetLastError());
+// Exclusive scans of one or two arrays (see ScanSeg); a segment without partial
+// sums gets its tile sums here.
+vox_status scan(vox_ctx *ctx, ScanSeg *seg, uint32_t nseg) {
+    uint32_t tiles = 0, up_tiles = 0, n_up = 0;
+    ScanSegs down{}, up{};
+    for (uint32_t k = 0; k < nseg; k++) {
+        ScanSeg &S = seg[k];
+        const uint32_t t = S.n / kScanTile + 1;
+        tiles = std::max(tiles, t);
+        if (!S.part && (t > kScanSmallTiles || S.in == S.out)) {
+            VOX_TRY(buf(ctx, k ? "scan_part1" : "scan_part0", 3 * (size_t)t, &S.part));
+            S.npart = t;
+            S.per_tile = 1;
+            up.s[n_up++] = S;
+            up_tiles = std::max(up_tiles, t);
         }
-        k_scan_down<<<nblocks, kScanThreads, 0, ctx->stream>>>(in, out, n, part);
-        VOX_HIP(hipGetLastError());
-        return VOX_OK;
+        down.s[k] = S;
     }
-    k_scan_blocks<<<nblocks, kScanThreads, 0, ctx->stream>>>(in, out, n, part);
+    if (n_up) {
+        k_scan_reduce<<<dim3(up_tiles, n_up), kScanThreads, 0, ctx->stream>>>(up);
+        VOX_HIP(hipGetLastError());
+    }
+    k_scan_down<<<dim3(tiles, nseg), kScanThreads, 0, ctx->stream>>>(down);
     VOX_HIP(hipGetLastError());
-    if (nblocks > 1) {
-        std::snprintf(name, sizeof(name), "scan%s_psum%d", tag, depth);
-        uint32_t *psum;
-        VOX_TRY(buf(ctx, name, nblocks + 2, &psum));
-        VOX_TRY(scan(ctx, part, psum, nblocks, depth + 1));
-        k_scan_add<<<nblocks, kScanThreads, 0, ctx->stream>>>(out, n, part, psum);
-        VOX_HIP(hipGetLastError());
-    }
     return VOX_OK;
 }
 
+// Device words to the host, through the pinned area: a kernel stores them there,
+// which costs less than a copy.
+__global__ void k_publish(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint32_t n) {
+    if (threadIdx.x < n) out[threadIdx.x] = in[threadIdx.x];
+}
 vox_status read_u32(vox_ctx *ctx, const uint32_t *dev, size_t n, uint32_t *host) {
-    if (n * 4 > kPinnedBytes) return fail(ctx, VOX_ERR_INVALID, "read_u32: read exceeds staging");
-    VOX_HIP(hipMemcpyAsync(ctx->pinned, dev, n * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (n > kWave) return fail(ctx, VOX_ERR_INVALID, "read_u32: too many words");
+    k_publish<<<1, kWave, 0, ctx->stream>>>(dev, ctx->pinned, (uint32_t)n);
+    VOX_HIP(hipGetLastError());
     VOX_HIP(hipStreamSynchronize(ctx->stream));
     std::memcpy(host, ctx->pinned, n * 4);
     return VOX_OK;
@@ -551,7 +535,8 @@ vox_status add_job(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, uin
     J.tile_base = P.tile_b.back();
     P.tile_b.push_back(J.tile_base + J.tilesY * J.tilesZ);
     J.pad_base = P.pad_b.back();
-    P.pad_b.push_back(J.pad_base + (pad_words(W, L.alloc[1], L.alloc[2]) + 255u) / 256u);
+    P.pad_b.push_back(J.pad_base +
+                      (pad_words(W, L.alloc[1], L.alloc[2]) + kPadBlock - 1u) / kPadBlock);
     J.m = F3{(float)J.em[0], (float)J.em[1], (float)J.em[2]};
     J.fd = (float)g.voxel_length;
     J.frd = 1.0f / J.fd;
@@ -640,28 +625,44 @@ vox_status add_mesh(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, ui
     return VOX_OK;
 }
 
-// Host-to-device upload through the context's pinned staging area; waits
-// for the previous upload to leave the area first.
+// A wait for the stream, after which the staging area is free again.
+vox_status wait_stream(vox_ctx *ctx) {
+    VOX_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->up_busy = false;
+    return VOX_OK;
+}
+
+__global__ void k_copy16(const uint4 *__restrict__ in, uint4 *__restrict__ out, uint32_t n) {
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) out[i] = in[i];
+}
+
+// Host-to-device upload through the context's pinned staging area, which the
+// GPU reads itself (a copy command costs several microseconds more); waits for
+// the previous upload to leave the area first.  dst holds bytes rounded up to
+// 16 (upload_size).
+size_t upload_size(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 vox_status upload(vox_ctx *ctx, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return VOX_OK;
-    if (bytes > ctx->up_cap && ctx->arena)
+    const size_t room = upload_size(bytes);
+    if (room > ctx->up_cap && ctx->arena)
         return fail(ctx, VOX_ERR_UNSUPPORTED,
                     "no-allocation call: job table larger than the staging area");
-    if (bytes > ctx->up_cap) {
+    if (ctx->up_busy) VOX_TRY(wait_stream(ctx));
+    if (room > ctx->up_cap) {
         if (ctx->up) {
-            VOX_HIP(hipEventSynchronize(ctx->up_ev));
             VOX_HIP(hipHostFree(ctx->up));
             ctx->up = nullptr;
+            ctx->up_cap = 0;
         }
-        const size_t want = (bytes + bytes / 2 + 4095) & ~(size_t)4095;
+        const size_t want = (room + room / 2 + 4095) & ~(size_t)4095;
         VOX_HIP(hipHostMalloc(&ctx->up, want, hipHostMallocDefault));
         ctx->up_cap = want;
-    } else {
-        VOX_HIP(hipEventSynchronize(ctx->up_ev));
     }
     std::memcpy(ctx->up, src, bytes);
-    VOX_HIP(hipMemcpyAsync(dst, ctx->up, bytes, hipMemcpyHostToDevice, ctx->stream));
-    VOX_HIP(hipEventRecord(ctx->up_ev, ctx->stream));
+    k_copy16<<<grid_for(room / 16, 256, 64), 256, 0, ctx->stream>>>(
+        (const uint4 *)ctx->up, (uint4 *)dst, (uint32_t)(room / 16));
+    VOX_HIP(hipGetLastError());
+    ctx->up_busy = true;
     return VOX_OK;
 }
 
@@ -726,7 +727,7 @@ vox_status plan_upload(vox_ctx *ctx, Plan &P, PlanDev &D, uint32_t splitY, uint3
     const size_t jb = al(sizeof(Job) * nj), sb = al(sizeof(SplitTable) * nj);
     const size_t bb = al(bases.size() * 4);
     uint8_t *dev;
-    VOX_TRY(buf(ctx, "j_table", jb + sb + bb + starts.size(), &dev));
+    VOX_TRY(buf(ctx, "j_table", upload_size(jb + sb + bb + starts.size()), &dev));
     const SplitTable *dsplit = (const SplitTable *)(dev + jb);
     for (uint32_t k = 0; k < nj; k++) {
         Job &J = P.jobs[k];
@@ -775,102 +776,216 @@ void record(vox_ctx *ctx, int i) {
 }
 
 // ---------------------------------------------------------------------------
-// Solid stage over all jobs: per-triangle records, candidate tiles, counting
-// sort by tile, fill.  Every grid is filled in one pass; with several
-// voxSplitRes y/z subspaces each (triangle, tile) pair carries the tile rows
-// whose subspace queues it, as the reference's per-subspace queues decide.
+// Preparation of the solid and the surface stage over all jobs: triangle setup,
+// then two counting sorts side by side in the same launches, of (triangle, tile)
+// pairs by tile and of (triangle, brick) pairs by brick.  Every grid is filled in
+// one pass; with several voxSplitRes y/z subspaces each (triangle, tile) pair
+// carries the tile rows whose subspace queues it, as the reference's
+// per-subspace queues decide.
+//
+// Launches and waits bound small meshes (about 4 us a launch with the gap before
+// it, 15 us a wait), so the two sorts share every launch, the candidate totals of
+// both come back with one wait, and one launch clears what the call counts into.
+// With the sorts on two streams, 12 launches and a wait each, a counting pass
+// again as the placing pass and the bricks' list by a scan of its own (calls):
+// bits of a sphere 62^3 104 -> 64 us, sphere 128^3 221 -> 141 us, room
+// 512x403x303 486 -> 375 us, LongFCC room 640x255x384 651 -> 555 us, 64-mesh
+// batch 3191 -> 3045 us, hall 1712 -> 1561 us (as a graph 1659 -> 1562 us).
 // ---------------------------------------------------------------------------
-// Triangle records (vertices, class word, material) and slot jobs, read by
-// both the solid and the surface stage; with fixed sizes the overflow flag
-// is cleared here, before either stage can raise it.
-vox_status records_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D) {
-    const uint32_t nj = (uint32_t)P.jobs.size();
-    const uint32_t nslots = P.tri_b.back();
-    VOX_TRY(buf(ctx, "tri_rec", (size_t)std::max<uint32_t>(nslots, 1) * 3, &ctx->rec));
-    VOX_TRY(buf(ctx, "tri_job", nslots, &ctx->tri_job));
-    if (ctx->fixed) VOX_TRY(fill(ctx, ctx->ovf, 1, 0u));
-    if (nslots > 0) {
-        k_tri_records<<<grid_for(nslots, 256), 256, 0, ctx->stream>>>(D.jobs, D.tri_b, nj, nslots,
-                                                                       ctx->rec, ctx->tri_job);
-        VOX_HIP(hipGetLastError());
-    }
-    return VOX_OK;
-}
+struct Prep {
+    float4 *rec = nullptr;  // per-triangle-slot vertex records
+    uint32_t *tri_job = nullptr;
+    SolidPairs solid{};
+    SurfPairs surf{};
+    uint32_t *wmask = nullptr, *stats = nullptr, *next = nullptr, *cnt = nullptr;
+    uint4 *tri_info = nullptr, *tri_ext = nullptr;
+    uint32_t *order = nullptr, *n_list = nullptr;  // non-empty bricks in index order
+    bool learned = false;
+};
 
-vox_status solid_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D) {
+// Buffers and clears of the erosion's first launch group.
+struct ErodeBufs {
+    uint32_t *changes = nullptr, *totals = nullptr, *stamp = nullptr, *notconv = nullptr;
+};
+constexpr uint32_t kErodeBatch = 4;  // passes per launch group and read-back
+
+vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, ErodeBufs &E) {
     const uint32_t nj = (uint32_t)P.jobs.size();
-    const uint32_t nslots = P.tri_b.back(), nTiles = P.tile_b.back();
-    uint32_t *tri_job = ctx->tri_job, *cand_count, *cand_off, *tile_hist, *tile_off, *tile_cursor,
-             *list;
-    uint2 *pairs;
-    uint4 *cbox;
-    VOX_TRY(buf(ctx, "s_cand_count", nslots, &cand_count));
-    VOX_TRY(buf(ctx, "s_cand_off", nslots + 2, &cand_off));
-    VOX_TRY(buf(ctx, "s_cbox", nslots, &cbox));
+    const uint32_t nslots = P.tri_b.back(), nTiles = P.tile_b.back(), nbt = P.brick_b.back();
+    const uint32_t tri_blocks = nslots / 256u, ne = P.erode_b.back();
+    const bool surf = P.any_mats;
+    const bool fine = nslots / kScanTile < kScanFineTiles;  // 256-slot sums for the scans
+    TriSetup T{};
+    uint32_t *tile_hist, *tile_off, *brick_hist = nullptr, *brick_off = nullptr;
+    VOX_TRY(buf(ctx, "tri_rec", (size_t)std::max<uint32_t>(nslots, 1) * 3, &R.rec));
+    if (nj > 1) VOX_TRY(buf(ctx, "tri_job", nslots, &R.tri_job));
+    VOX_TRY(buf(ctx, "s_cand_off", (size_t)nslots + 2, &T.off_s));
+    VOX_TRY(buf(ctx, "s_cbox", nslots, &T.cbox));
+    VOX_TRY(buf(ctx, "s_part", 2 * (size_t)tri_blocks, &T.part_s));
     VOX_TRY(buf(ctx, "s_tile_hist", nTiles, &tile_hist));
-    VOX_TRY(buf(ctx, "s_tile_off", nTiles + 2, &tile_off));
-    VOX_TRY(buf(ctx, "s_tile_cursor", nTiles, &tile_cursor));
-    if (nslots > 0) {
-        k_solid_setup<<<grid_for(nslots, 256), 256, 0, ctx->stream>>>(D.jobs, D.tri_b, nj, nslots,
-                                                                       ctx->rec, cand_count, cbox);
-        VOX_HIP(hipGetLastError());
+    VOX_TRY(buf(ctx, "s_tile_off", (size_t)nTiles + 2, &tile_off));
+    if (surf) {
+        // The model is consulted only when there are more bricks than resident
+        // brick-pass workgroups: with fewer, every brick starts at once and the
+        // order cannot matter.
+        R.learned = ctx->schedule == VOX_SCHEDULE_LEARNED && ctx->cost_ready &&
+                    nbt > (uint32_t)(ctx->n_cu * ctx->surf_blocks_per_cu);
+        if (ctx->timing) ctx->times.learned_schedule = R.learned ? 1u : 0u;
+        VOX_TRY(buf(ctx, "f_tri_info", nslots, &R.tri_info));
+        if (R.learned || ctx->record) VOX_TRY(buf(ctx, "f_tri_ext", nslots, &R.tri_ext));
+        VOX_TRY(buf(ctx, "f_cand_off", (size_t)nslots + 2, &T.off_f));
+        VOX_TRY(buf(ctx, "f_part", 2 * (size_t)tri_blocks, &T.part_f));
+        VOX_TRY(buf(ctx, "f_brick_hist", nbt, &brick_hist));
+        VOX_TRY(buf(ctx, "f_brick_off", (size_t)nbt + 2, &brick_off));
+        VOX_TRY(buf(ctx, "f_order", nbt, &R.order));
+        VOX_TRY(buf(ctx, "f_n_list", 1, &R.n_list));
+        VOX_TRY(buf(ctx, "f_stats", 1, &R.stats));
+        VOX_TRY(buf(ctx, "f_wmask", (size_t)nbt * 4u, &R.wmask));
+        VOX_TRY(buf(ctx, "f_next", kBrickLists * kBrickListPitch, &R.next));
+        if (R.learned && !ctx->record) VOX_TRY(buf(ctx, "f_cnt", 2, &R.cnt));
     }
-    VOX_TRY(scan(ctx, cand_count, cand_off, nslots));
-    uint32_t total = 0;
-    if (ctx->fixed) {
-        total = ctx->cap_solid;
-    } else {
-        uint32_t h[2];
-        VOX_TRY(read_u32(ctx, cand_off + nslots, 2, h));
+    const uint32_t npass = ctx->fixed ? ctx->n_passes : kErodeBatch;
+    if (ne > 0) {
+        VOX_TRY(buf(ctx, "e_changes", (size_t)npass * nj, &E.changes));
+        VOX_TRY(buf(ctx, "e_totals", npass, &E.totals));
+        VOX_TRY(buf(ctx, "e_stamp", ne, &E.stamp));
+        if (ctx->fixed) VOX_TRY(buf(ctx, "e_notconv", 1, &E.notconv));
+    }
+    T.rec = R.rec;
+    T.tri_job = R.tri_job;
+    T.tri_info = R.tri_info;
+    T.tri_ext = R.tri_ext;
+    // Everything the call counts into starts at zero (with fixed sizes the
+    // overflow flag too).
+    const FillSeg zero[] = {{ctx->fixed ? ctx->ovf : nullptr, 1, 0u},
+                            {tile_hist, nTiles, 0u},
+                            {brick_hist, nbt, 0u},
+                            {R.wmask, (size_t)nbt * 4u, 0u},
+                            {R.stats, 1, 0u},
+                            {R.next, kBrickLists * kBrickListPitch, 0u},
+                            {R.cnt, 2, 0u},
+                            {E.changes, (size_t)npass * nj, 0u},
+                            {E.totals, npass, 0u},
+                            {E.stamp, ne, 0u},
+                            {E.notconv, 1, 0u}};
+    static_assert(sizeof(zero) / sizeof(zero[0]) <= kMaxFillSegs, "fill table");
+    FillSegs clear;
+    const size_t most = fill_table(zero, sizeof(zero) / sizeof(zero[0]), clear);
+    k_tri_setup<<<tri_blocks + grid_for(most, 1024, 1024), 256, 0, ctx->stream>>>(
+        D.jobs, D.tri_b, nj, tri_blocks, T, clear);
+    VOX_HIP(hipGetLastError());
+    // Candidate offsets; their totals go straight to the host.
+    uint32_t *host = ctx->fixed ? nullptr : ctx->pinned;
+    ScanSeg seg[2] = {};
+    seg[0].in = seg[0].out = T.off_s;
+    seg[0].n = nslots;
+    seg[0].host = host;
+    if (fine) {
+        seg[0].part = T.part_s;
+        seg[0].npart = tri_blocks;
+        seg[0].per_tile = kScanTile / 256;
+    }
+    if (surf) {
+        seg[1] = seg[0];
+        seg[1].in = seg[1].out = T.off_f;
+        if (fine) seg[1].part = T.part_f;
+        seg[1].host = host ? host + 2 : nullptr;
+    }
+    VOX_TRY(scan(ctx, seg, surf ? 2 : 1));
+    uint32_t total_s = ctx->cap_solid, total_f = surf ? ctx->cap_surf : 0u;
+    if (!ctx->fixed) {
+        VOX_TRY(wait_stream(ctx));
+        uint32_t h[4] = {0u, 0u, 0u, 0u};
+        std::memcpy(h, ctx->pinned, surf ? 16 : 8);
         if (h[1])
             return fail(ctx, VOX_ERR_UNSUPPORTED,
                         "2^32 or more (triangle, tile) candidates in one call");
-        total = h[0];
-        ctx->last_solid = total;
+        if (h[3])
+            return fail(ctx, VOX_ERR_UNSUPPORTED,
+                        "2^32 or more (triangle, brick) candidates in one call");
+        total_s = h[0];
+        total_f = h[2];
+        ctx->last_solid = total_s;
+        if (surf) ctx->last_surf = total_f;
     }
-    uint32_t *ovf = ctx->fixed ? ctx->ovf : nullptr;
-    uint32_t *first;
-    uint16_t *pmask = nullptr, *list_mask = nullptr;
-    VOX_TRY(buf(ctx, "s_pairs", total, &pairs));
-    VOX_TRY(buf(ctx, "s_list", total, &list));
+    SolidPairs &A = R.solid;
+    SurfPairs &B = R.surf;
+    uint32_t *first_s, *first_f = nullptr;
+    VOX_TRY(buf(ctx, "s_pairs", total_s, &A.pairs));
+    VOX_TRY(buf(ctx, "s_list", total_s, &A.list));
     if (D.solid_split) {
-        VOX_TRY(buf(ctx, "s_pmask", total, &pmask));
-        VOX_TRY(buf(ctx, "s_list_mask", total, &list_mask));
+        VOX_TRY(buf(ctx, "s_pmask", total_s, &A.pmask));
+        VOX_TRY(buf(ctx, "s_list_mask", total_s, &A.list_mask));
     }
-    VOX_TRY(buf(ctx, "s_first", block_starts_size(total), &first));
-    if (total > 0 && nslots > 0) {
-        k_block_starts<<<grid_for(nslots, 256), 256, 0, ctx->stream>>>(cand_off, nslots, total,
-                                                                        first);
+    VOX_TRY(buf(ctx, "s_first", block_starts_size(total_s), &first_s));
+    A.rec = R.rec;
+    A.off = T.off_s;
+    A.first = first_s;
+    A.cbox = T.cbox;
+    A.hist = tile_hist;
+    A.bin_off = tile_off;
+    A.cap = total_s;
+    A.ovf = ctx->fixed ? ctx->ovf : nullptr;
+    if (surf) {
+        VOX_TRY(buf(ctx, "f_place", total_f, &B.place));
+        VOX_TRY(buf(ctx, "f_blist", total_f, &B.list));
+        VOX_TRY(buf(ctx, "f_first", block_starts_size(total_f), &first_f));
+        B.off = T.off_f;
+        B.first = first_f;
+        B.tri_info = R.tri_info;
+        B.hist = brick_hist;
+        B.bin_off = brick_off;
+        B.cap = total_f;
+        B.ovf = A.ovf;
+    }
+    const uint32_t bs = total_s ? grid_for(total_s, 256) : 0u;
+    const uint32_t bf = total_f ? grid_for(total_f, 256) : 0u;
+    const bool pairs = nslots > 0 && bs + bf > 0;
+    if (pairs) {
+        k_block_starts<<<dim3(grid_for(nslots, 256), bf ? 2 : 1), 256, 0, ctx->stream>>>(
+            BlockStarts{A.off, A.cap, first_s}, BlockStarts{B.off, B.cap, first_f}, nslots);
         VOX_HIP(hipGetLastError());
-    }
-    VOX_TRY(fill_many(ctx, {{tile_hist, nTiles, 0u}, {tile_cursor, nTiles, 0u}}));
-    if (total > 0) {
         if (nj > 1)
-            k_solid_candidates<true><<<grid_for(total, 256), 256, 0, ctx->stream>>>(
-                D.jobs, tri_job, nslots, ctx->rec, cand_off, cand_off + nslots, first, cbox,
-                pairs, pmask, tile_hist, total, ovf);
+            k_pairs_count<true><<<bs + bf, 256, 0, ctx->stream>>>(D.jobs, R.tri_job, nslots, A, B,
+                                                                  bs);
         else
-            k_solid_candidates<false><<<grid_for(total, 256), 256, 0, ctx->stream>>>(
-                D.jobs, tri_job, nslots, ctx->rec, cand_off, cand_off + nslots, first, cbox,
-                pairs, pmask, tile_hist, total, ovf);
+            k_pairs_count<false><<<bs + bf, 256, 0, ctx->stream>>>(D.jobs, R.tri_job, nslots, A, B,
+                                                                   bs);
         VOX_HIP(hipGetLastError());
     }
-    VOX_TRY(scan(ctx, tile_hist, tile_off, nTiles));
-    if (total > 0) {
-        k_solid_scatter<<<grid_for(total, 256), 256, 0, ctx->stream>>>(
-            pairs, pmask, cand_off + nslots, tile_off, tile_cursor, list, list_mask, total);
+    ScanSeg bins[2] = {};
+    bins[0].in = tile_hist;
+    bins[0].out = tile_off;
+    bins[0].n = nTiles;
+    if (surf) {
+        bins[1].in = brick_hist;
+        bins[1].out = brick_off;
+        bins[1].n = nbt;
+        bins[1].list = R.order;
+        bins[1].n_list = R.n_list;
+    }
+    VOX_TRY(scan(ctx, bins, surf ? 2 : 1));
+    if (pairs) {
+        if (nj > 1)
+            k_pairs_place<true><<<bs + bf, 256, 0, ctx->stream>>>(D.jobs, R.tri_job, nslots, A, B,
+                                                                  bs);
+        else
+            k_pairs_place<false><<<bs + bf, 256, 0, ctx->stream>>>(D.jobs, R.tri_job, nslots, A, B,
+                                                                   bs);
         VOX_HIP(hipGetLastError());
     }
-    if (nTiles > 0) {
-        k_solid_fill<<<nTiles, kWave, 16 * std::min(P.maxW, kFillSegWords) * 4, ctx->stream>>>(
-            D.jobs, D.tile_b, nj, ctx->rec, tile_off, tile_hist, list, list_mask);
-        VOX_HIP(hipGetLastError());
-    }
-    if (P.pad_b.back() > 0) {
-        k_zero_pad_rows<<<P.pad_b.back(), 256, 0, ctx->stream>>>(D.jobs, D.pad_b, nj);
-        VOX_HIP(hipGetLastError());
-    }
-    ctx->times.solid_pairs += total;  // candidate (triangle, tile) pairs
+    ctx->times.solid_pairs += total_s;  // candidate pairs
+    if (ctx->timing) ctx->times.surface_pairs += total_f;
+    return VOX_OK;
+}
+
+vox_status solid_fill(vox_ctx *ctx, const Plan &P, const PlanDev &D, const Prep &R) {
+    const uint32_t blocks = P.tile_b.back() + P.pad_b.back();
+    if (blocks == 0) return VOX_OK;
+    k_solid_fill<<<blocks, kWave, 16 * std::min(P.maxW, kFillSegWords) * 4, ctx->stream>>>(
+        D.jobs, D.tile_b, D.pad_b, (uint32_t)P.jobs.size(), R.rec, R.solid.bin_off, R.solid.hist,
+        R.solid.list, R.solid.list_mask);
+    VOX_HIP(hipGetLastError());
     return VOX_OK;
 }
 
@@ -895,130 +1010,31 @@ vox_status record_samples(vox_ctx *ctx, const uint32_t *list, const uint32_t *n_
 }
 
 // ---------------------------------------------------------------------------
-// Surface stage over the jobs that want materials: triangle classes and
-// brick boxes, counting sort of (triangle, brick) pairs by brick, the brick
-// order (plain or learned), the persistent brick pass, which leaves the
-// surface words and the material grid the node passes read.
+// Surface stage over the jobs that want materials (after the solid stage: it
+// ORs surface bits into the solid grid): for the learned schedule the heavy
+// bricks of the list, then the persistent brick pass, which leaves the surface
+// words and the material grid the node passes read.
 // ---------------------------------------------------------------------------
-// Triangle slots from which the surface preparation runs on its own stream.
-constexpr uint32_t kForkMinSlots = 16384;
-
-// What the brick pass needs from the surface stage's preparation.
-struct SurfPass {
-    uint32_t *brick_off = nullptr, *brick_hist = nullptr, *blist = nullptr, *stats = nullptr;
-    uint32_t *blist_order = nullptr, *next = nullptr;
-    const uint32_t *n_list = nullptr, *hlist = nullptr, *hsub = nullptr, *n_heavy = nullptr;
-    const uint8_t *skip = nullptr;
-    float *feats = nullptr;
-};
-
-// Surface stage up to the brick pass: triangle setup, (triangle, brick)
-// pairs binned by brick, the brick list and, for the learned schedule, its
-// heavy bricks.  It only reads the triangle records, so it can run beside
-// the solid stage.
-vox_status surface_prep(vox_ctx *ctx, const Plan &P, const PlanDev &D, SurfPass &S) {
+vox_status surface_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, const Prep &R) {
     const uint32_t nj = (uint32_t)P.jobs.size();
     const uint32_t nslots = P.tri_b.back(), nbt = P.brick_b.back();
-    uint4 *tri_info, *tri_ext = nullptr;
-    uint32_t *cand, *cand_off, *brick_hist, *brick_off, *brick_cursor, *blist, *stats;
-    // The model is consulted only when there are more bricks than resident
-    // brick-pass workgroups: with fewer, every brick starts at once and the
-    // order cannot matter.
-    const bool learned = ctx->schedule == VOX_SCHEDULE_LEARNED && ctx->cost_ready &&
-                         nbt > (uint32_t)(ctx->n_cu * ctx->surf_blocks_per_cu);
-    const bool features = learned || ctx->record;
-    if (ctx->timing) ctx->times.learned_schedule = learned ? 1u : 0u;
-    VOX_TRY(buf(ctx, "f_tri_info", nslots, &tri_info));
-    if (features) VOX_TRY(buf(ctx, "f_tri_ext", nslots, &tri_ext));
-    float4 *tri_rec = ctx->rec;
-    VOX_TRY(buf(ctx, "f_cand", nslots, &cand));
-    VOX_TRY(buf(ctx, "f_cand_off", nslots + 2, &cand_off));
-    VOX_TRY(buf(ctx, "f_brick_hist", nbt, &brick_hist));
-    VOX_TRY(buf(ctx, "f_brick_off", nbt + 2, &brick_off));
-    VOX_TRY(buf(ctx, "f_brick_cursor", nbt, &brick_cursor));
-    VOX_TRY(buf(ctx, "f_stats", 1, &stats));
-    if (nslots > 0) {
-        k_surf_setup<<<grid_for(nslots, 256), 256, 0, ctx->stream>>>(D.jobs, D.tri_b, nj, nslots,
-                                                                      tri_info, cand, tri_ext,
-                                                                      tri_rec);
-        VOX_HIP(hipGetLastError());
-    }
-    VOX_TRY(scan(ctx, cand, cand_off, nslots));
-    uint32_t total = 0;
-    if (ctx->fixed) {
-        total = ctx->cap_surf;
-    } else {
-        uint32_t h[2];
-        VOX_TRY(read_u32(ctx, cand_off + nslots, 2, h));
-        if (h[1])
-            return fail(ctx, VOX_ERR_UNSUPPORTED,
-                        "2^32 or more (triangle, brick) candidates in one call");
-        total = h[0];
-        ctx->last_surf = total;
-    }
-    uint32_t *ovf = ctx->fixed ? ctx->ovf : nullptr;
-    uint32_t *first;
-    VOX_TRY(buf(ctx, "f_blist", total, &blist));
-    VOX_TRY(buf(ctx, "f_first", block_starts_size(total), &first));
-    if (total > 0 && nslots > 0) {
-        k_block_starts<<<grid_for(nslots, 256), 256, 0, ctx->stream>>>(cand_off, nslots, total,
-                                                                        first);
-        VOX_HIP(hipGetLastError());
-    }
-    // Everything this stage and the brick pass count into starts at zero.
-    uint32_t *wmask, *next, *cnt = nullptr;
-    VOX_TRY(buf(ctx, "f_wmask", (size_t)nbt * 4u, &wmask));
-    VOX_TRY(buf(ctx, "f_next", kBrickLists * kBrickListPitch, &next));
-    if (learned && !ctx->record) VOX_TRY(buf(ctx, "f_cnt", 2, &cnt));
-    VOX_TRY(fill_many(ctx, {{brick_hist, nbt, 0u},
-                            {brick_cursor, nbt, 0u},
-                            {wmask, (size_t)nbt * 4u, 0u},
-                            {stats, 1, 0u},
-                            {next, kBrickLists * kBrickListPitch, 0u},
-                            {cnt, cnt ? 2u : 0u, 0u}}));
-    auto bin = [&](int scatter) -> vox_status {
-        if (total == 0) return VOX_OK;
-        if (nj > 1)
-            k_surf_bin<true><<<grid_for(total, 256), 256, 0, ctx->stream>>>(
-                D.jobs, ctx->tri_job, nslots, cand_off, cand_off + nslots, first, tri_info,
-                brick_hist, brick_off, brick_cursor, blist, scatter, total, ovf);
-        else
-            k_surf_bin<false><<<grid_for(total, 256), 256, 0, ctx->stream>>>(
-                D.jobs, ctx->tri_job, nslots, cand_off, cand_off + nslots, first, tri_info,
-                brick_hist, brick_off, brick_cursor, blist, scatter, total, ovf);
-        VOX_HIP(hipGetLastError());
-        return VOX_OK;
-    };
-    VOX_TRY(bin(0));
-    VOX_TRY(scan(ctx, brick_hist, brick_off, nbt));
-    // Non-empty bricks in index order (the plain schedule of the brick pass).
-    uint32_t *flags, *blist_order, *blist_order_off;
-    VOX_TRY(buf(ctx, "f_flags", nbt, &flags));
-    VOX_TRY(buf(ctx, "f_order", nbt, &blist_order));
-    VOX_TRY(buf(ctx, "f_order_off", nbt + 2, &blist_order_off));
-    k_nonzero_flags<<<grid_for(nbt, 256), 256, 0, ctx->stream>>>(brick_hist, flags, nbt);
-    VOX_HIP(hipGetLastError());
-    VOX_TRY(scan(ctx, flags, blist_order_off, nbt));
-    k_nonzero_list<<<grid_for(nbt, 256), 256, 0, ctx->stream>>>(brick_hist, blist_order_off,
-                                                                blist_order, nbt);
-    VOX_HIP(hipGetLastError());
-    VOX_TRY(bin(1));
-    if (ctx->timing) ctx->times.surface_pairs += total;
-    // Learned schedule: the listed bricks screened by pair count, their cost
-    // predicted by the MLP, the heavy ones on a list the brick pass takes
-    // first (see vox_cost.hip).
-    const uint32_t *n_list = blist_order_off + nbt;
+    const uint32_t *brick_hist = R.surf.hist, *brick_off = R.surf.bin_off, *blist = R.surf.list;
+    const uint32_t *cand_total = R.surf.off + nslots;
     const uint32_t *hlist = nullptr, *hsubs = nullptr, *n_heavy = nullptr;
     const uint8_t *skip = nullptr;
     float *feats = nullptr;
     uint64_t *cycles = nullptr;
-    if (ctx->record) VOX_TRY(buf(ctx, "f_feats", (size_t)nbt * kCostFeatures, &feats));
     if (ctx->record) {  // training samples: features of every listed brick
+        VOX_TRY(buf(ctx, "f_feats", (size_t)nbt * kCostFeatures, &feats));
+        VOX_TRY(buf(ctx, "f_cycles", nbt, &cycles));
         k_brick_features<<<grid_for(nbt, 4, 65535), 256, 0, ctx->stream>>>(
-            blist_order, nullptr, n_list, brick_hist, brick_off, blist, tri_info, tri_ext, D.jobs,
-            D.brick_b, nj, feats);
+            R.order, nullptr, R.n_list, brick_hist, brick_off, blist, R.tri_info, R.tri_ext,
+            D.jobs, D.brick_b, nj, feats);
         VOX_HIP(hipGetLastError());
-    } else if (learned) {
+    } else if (R.learned) {
+        // The listed bricks screened by pair count, their cost predicted by the
+        // MLP, the heavy ones on a list the brick pass takes first (see
+        // vox_cost.hip).
         uint32_t *lcand, *heavy, *hsub;
         uint8_t *skipf;
         VOX_TRY(buf(ctx, "f_lcand", nbt, &lcand));
@@ -1026,9 +1042,8 @@ vox_status surface_prep(vox_ctx *ctx, const Plan &P, const PlanDev &D, SurfPass 
         VOX_TRY(buf(ctx, "f_hsub", (size_t)kMaxSplitParts * nbt, &hsub));
         VOX_TRY(buf(ctx, "f_skip", nbt, &skipf));
         const uint32_t g256 = grid_for(nbt, 256, 1024);
-        k_cost_screen<<<g256, 256, 0, ctx->stream>>>(blist_order, n_list, brick_hist,
-                                                     cand_off + nslots, ctx->screen_ratio, lcand,
-                                                     cnt, skipf);
+        k_cost_screen<<<g256, 256, 0, ctx->stream>>>(R.order, R.n_list, brick_hist, cand_total,
+                                                     ctx->screen_ratio, lcand, R.cnt, skipf);
         VOX_HIP(hipGetLastError());
         // Cutting a brick repeats its triangle setup in every part; it pays
         // only where one long brick can end the pass last, i.e. when there
@@ -1038,83 +1053,51 @@ vox_status surface_prep(vox_ctx *ctx, const Plan &P, const PlanDev &D, SurfPass 
         const uint32_t max_parts =
             ctx->split_parts ? ctx->split_parts : per_wg >= 16u ? 1u : per_wg >= 4u ? 2u : 4u;
         k_cost_predict<<<grid_for(nbt, 4, (uint32_t)ctx->n_cu * 8u), 256, 0, ctx->stream>>>(
-            ctx->cost_params, blist_order, lcand, cnt, ctx->heavy_cost, max_parts, brick_hist,
-            brick_off, blist, tri_info, tri_ext, D.jobs, D.brick_b, nj, heavy, hsub, skipf);
+            ctx->cost_params, R.order, lcand, R.cnt, ctx->heavy_cost, max_parts, brick_hist,
+            brick_off, blist, R.tri_info, R.tri_ext, D.jobs, D.brick_b, nj, heavy, hsub, skipf);
         VOX_HIP(hipGetLastError());
         hlist = heavy;
         hsubs = hsub;
-        n_heavy = cnt + 1;
+        n_heavy = R.cnt + 1;
         skip = skipf;
     }
-    (void)cycles;
-    S.brick_off = brick_off;
-    S.brick_hist = brick_hist;
-    S.blist = blist;
-    S.stats = stats;
-    S.blist_order = blist_order;
-    S.next = next;
-    S.n_list = n_list;
-    S.hlist = hlist;
-    S.hsub = hsubs;
-    S.n_heavy = n_heavy;
-    S.skip = skip;
-    S.feats = feats;
-    return VOX_OK;
-}
-
-// The brick pass (after the solid stage: it ORs surface bits into the solid
-// grid).
-vox_status surface_brick(vox_ctx *ctx, const Plan &P, const PlanDev &D, const SurfPass &S) {
-    const uint32_t nj = (uint32_t)P.jobs.size(), nbt = P.brick_b.back();
-    uint64_t *cycles = nullptr;
-    if (ctx->record) VOX_TRY(buf(ctx, "f_cycles", nbt, &cycles));
     const uint32_t blocks = std::min<uint32_t>(nbt, (uint32_t)(ctx->n_cu * ctx->surf_blocks_per_cu));
+    uint32_t *stats = ctx->timing ? R.stats : nullptr;
     if (P.any_partial)
         k_surf_brick<true><<<blocks, kBrickThreads, 0, ctx->stream>>>(
-            D.jobs, D.brick_b, nj, ctx->rec, S.brick_off, S.brick_hist, S.blist,
-            ctx->timing ? S.stats : nullptr, S.blist_order, S.n_list, S.hlist, S.hsub, S.n_heavy,
-            S.skip, S.next, cycles);
+            D.jobs, D.brick_b, nj, R.rec, brick_off, brick_hist, blist, stats, R.order, R.n_list,
+            hlist, hsubs, n_heavy, skip, R.next, cycles);
     else
         k_surf_brick<false><<<blocks, kBrickThreads, 0, ctx->stream>>>(
-            D.jobs, D.brick_b, nj, ctx->rec, S.brick_off, S.brick_hist, S.blist,
-            ctx->timing ? S.stats : nullptr, S.blist_order, S.n_list, S.hlist, S.hsub, S.n_heavy,
-            S.skip, S.next, cycles);
+            D.jobs, D.brick_b, nj, R.rec, brick_off, brick_hist, blist, stats, R.order, R.n_list,
+            hlist, hsubs, n_heavy, skip, R.next, cycles);
     VOX_HIP(hipGetLastError());
     if (ctx->timing) {
         uint32_t vox = 0;
-        VOX_TRY(read_u32(ctx, S.stats, 1, &vox));
+        VOX_TRY(read_u32(ctx, R.stats, 1, &vox));
         ctx->times.surface_voxels += vox;
     }
-    if (ctx->record)
-        VOX_TRY(record_samples(ctx, S.blist_order, S.n_list, S.feats, cycles, nbt));
+    if (ctx->record) VOX_TRY(record_samples(ctx, R.order, R.n_list, feats, cycles, nbt));
     return VOX_OK;
 }
 
 // Erosion to the fixed point over every Cartesian job, in place.  A single
 // job may have several alloc y/z subspaces, eroded one after another in the
 // reference's order; jobs of a batch have one each.  Passes are launched
-// kBatch at a time; a job's pass after one that changed nothing in it exits
+// kErodeBatch at a time; a job's pass after one that changed nothing in it exits
 // at once, so one host read per batch of passes suffices.  With fixed sizes
 // (graph capture) each subspace gets ctx->n_passes passes and no read-back;
 // the last pass of every subspace raises the not-converged flag if it still
 // changed something.
-vox_status erode_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, uint32_t splitY,
-                       uint32_t splitZ) {
-    constexpr uint32_t kBatch = 4;
+vox_status erode_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, const ErodeBufs &E,
+                       uint32_t splitY, uint32_t splitZ) {
     const uint32_t nj = (uint32_t)P.jobs.size();
     const uint32_t nblocks = P.erode_b.back();
     ctx->last_changed = nullptr;
     if (nblocks == 0) return VOX_OK;
-    uint32_t *changes, *totals, *stamp, *notconv = nullptr;
-    const uint32_t nbuf = ctx->fixed ? ctx->n_passes : kBatch;  // passes per launch group
-    VOX_TRY(buf(ctx, "e_changes", (size_t)nbuf * nj, &changes));
-    VOX_TRY(buf(ctx, "e_totals", nbuf, &totals));
-    VOX_TRY(buf(ctx, "e_stamp", nblocks, &stamp));
-    if (ctx->fixed) {
-        VOX_TRY(buf(ctx, "e_notconv", 1, &notconv));
-        ctx->last_changed = notconv;
-    }
-    bool cleared = false;  // stamp and notconv go with the first group's flags
+    const uint32_t nbuf = ctx->fixed ? ctx->n_passes : kErodeBatch;  // passes per launch group
+    if (ctx->fixed) ctx->last_changed = E.notconv;
+    bool cleared = true;  // the first group's flags, by the triangle setup
     std::vector<Span> ys{{0u, UINT32_MAX}}, zs{{0u, UINT32_MAX}};
     if (nj == 1) {
         ys = split_axis_max(P.jobs[0].gd.Y, splitY);
@@ -1129,15 +1112,15 @@ vox_status erode_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, uint32_t s
             bool first = true;
             uint32_t sub = 0;  // passes this subspace needed
             for (int guard = 0; guard < 1000000; guard++) {
-                VOX_TRY(fill_many(ctx, {{changes, (size_t)nbuf * nj, 0u},
-                                        {totals, nbuf, 0u},
-                                        {cleared ? nullptr : stamp, nblocks, 0u},
-                                        {cleared ? nullptr : notconv, 1, 0u}}));
-                cleared = true;
+                if (!cleared)
+                    VOX_TRY(fill_many(ctx, {{E.changes, (size_t)nbuf * nj, 0u},
+                                            {E.totals, nbuf, 0u}}));
+                cleared = false;
                 for (uint32_t k = 0; k < nbuf; k++) {
                     k_erode<<<grid, 256, 0, ctx->stream>>>(
-                        D.jobs, D.erode_b, nj, ysp.min, ysp.max, zsp.min, zsp.max, stamp,
-                        changes, totals, k == nbuf - 1 ? notconv : nullptr, k, gpass + k,
+                        D.jobs, D.erode_b, nj, ysp.min, ysp.max, zsp.min, zsp.max,
+                        E.stamp, E.changes, E.totals, k == nbuf - 1 ? E.notconv : nullptr, k,
+                        gpass + k,
                         (first && k == 0) ? 1 : 0);
                     VOX_HIP(hipGetLastError());
                 }
@@ -1147,19 +1130,19 @@ vox_status erode_stage(vox_ctx *ctx, const Plan &P, const PlanDev &D, uint32_t s
                     sub = nbuf;
                     break;
                 }
-                uint32_t h[kBatch];
-                VOX_TRY(read_u32(ctx, totals, kBatch, h));
-                uint32_t k0 = kBatch;
-                for (uint32_t k = 0; k < kBatch; k++)
+                uint32_t h[kErodeBatch];
+                VOX_TRY(read_u32(ctx, E.totals, kErodeBatch, h));
+                uint32_t k0 = kErodeBatch;
+                for (uint32_t k = 0; k < kErodeBatch; k++)
                     if (h[k] == 0u) {
                         k0 = k;
                         break;
                     }
-                if (k0 < kBatch) {
+                if (k0 < kErodeBatch) {
                     sub += k0 + 1;
                     break;
                 }
-                sub += kBatch;
+                sub += kErodeBatch;
             }
             passes += sub;
             most = std::max(most, sub);
@@ -1215,33 +1198,12 @@ vox_status run_plan(vox_ctx *ctx, Plan &P, uint32_t splitY, uint32_t splitZ) {
 // The stages after the job-table upload (what a graph captures).
 vox_status run_stages(vox_ctx *ctx, Plan &P, const PlanDev &D, uint32_t splitY,
                       uint32_t splitZ) {
-    VOX_TRY(records_stage(ctx, P, D));
-    // Fork: the surface preparation on the side stream, the solid stage on
-    // the main one; they join before the brick pass.  (Inside a graph
-    // capture the side stream joins the capture through the fork event.)
-    SurfPass S;
-    // Small meshes (a few thousand triangles) have too little of either
-    // stage to overlap; the fork's extra dependencies would cost more.
-    const bool fork = P.any_mats && P.tri_b.back() >= kForkMinSlots;
-    if (fork) {
-        VOX_HIP(hipEventRecord(ctx->ev_fork, ctx->stream));
-        VOX_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-        hipStream_t main = ctx->stream;
-        ctx->stream = ctx->side;
-        const vox_status st = surface_prep(ctx, P, D, S);
-        ctx->stream = main;
-        VOX_TRY(st);
-        VOX_HIP(hipEventRecord(ctx->ev_join, ctx->side));
-    }
-    VOX_TRY(solid_stage(ctx, P, D));
+    Prep R;
+    ErodeBufs E;
+    VOX_TRY(prepare(ctx, P, D, R, E));
+    VOX_TRY(solid_fill(ctx, P, D, R));
     record(ctx, 1);
-    if (fork) {
-        VOX_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
-        VOX_TRY(surface_brick(ctx, P, D, S));
-    } else if (P.any_mats) {
-        VOX_TRY(surface_prep(ctx, P, D, S));
-        VOX_TRY(surface_brick(ctx, P, D, S));
-    }
+    if (P.any_mats) VOX_TRY(surface_stage(ctx, P, D, R));
     record(ctx, 2);
     if (D.pre) {
         const Job &J = P.jobs[0];
@@ -1254,10 +1216,36 @@ vox_status run_stages(vox_ctx *ctx, Plan &P, const PlanDev &D, uint32_t splitY,
         if (J.pbits)
             VOX_HIP(hipMemcpyAsync(J.pbits, J.bits, (size_t)J.gd.W * J.gd.Y * J.gd.Z * 4,
                                    hipMemcpyDeviceToDevice, ctx->stream));
-    VOX_TRY(erode_stage(ctx, P, D, splitY, splitZ));
+    VOX_TRY(erode_stage(ctx, P, D, E, splitY, splitZ));
     record(ctx, 3);
     VOX_TRY(node_stage(ctx, P, D, D.pre, D.ystart, D.zstart));
     record(ctx, 4);
+    return VOX_OK;
+}
+
+// Bounding box of nv device vertices (calculateBoundingBox).  The blocks leave
+// theirs in the pinned area.
+vox_status device_bbox(vox_ctx *ctx, const float *V, uint32_t nv, double mn[3], double mx[3]) {
+    constexpr uint32_t kBlocks = 256;
+    static_assert(kBlocks * 24 <= kPinnedBytes, "a block's six keys");
+    const uint32_t blocks = grid_for(nv, 256, kBlocks);
+    k_bbox<<<blocks, 256, 0, ctx->stream>>>(V, nv, ctx->pinned);
+    VOX_HIP(hipGetLastError());
+    VOX_HIP(hipStreamSynchronize(ctx->stream));
+    for (int c = 0; c < 3; c++) {
+        uint32_t a = UINT32_MAX, b = 0u;
+        for (uint32_t k = 0; k < blocks; k++) {
+            a = std::min(a, ctx->pinned[6 * k + c]);
+            b = std::max(b, ctx->pinned[6 * k + 3 + c]);
+        }
+        uint32_t ua = (a & 0x80000000u) ? (a & 0x7FFFFFFFu) : ~a;
+        uint32_t ub = (b & 0x80000000u) ? (b & 0x7FFFFFFFu) : ~b;
+        float fa, fb;
+        std::memcpy(&fa, &ua, 4);
+        std::memcpy(&fb, &ub, 4);
+        mn[c] = fa;
+        mx[c] = fb;
+    }
     return VOX_OK;
 }
 
@@ -1296,19 +1284,11 @@ vox_status vox_create(int device, vox_ctx **out) {
     vox_ctx *ctx = new vox_ctx();
     ctx->dev = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&ctx->stream) != hipSuccess ||
-        (ctx->main_stream = ctx->stream, false) ||
         hipHostMalloc((void **)&ctx->pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
         delete ctx;
         return VOX_ERR_HIP;
     }
     for (auto &e : ctx->ev) (void)hipEventCreate(&e);
-    if (hipEventCreateWithFlags(&ctx->up_ev, hipEventDisableTiming) != hipSuccess ||
-        hipStreamCreate(&ctx->side) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) {
-        vox_destroy(ctx);
-        return VOX_ERR_HIP;
-    }
     if (hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, device) !=
             hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&ctx->surf_blocks_per_cu, k_surf_brick<false>,
@@ -1360,7 +1340,6 @@ void vox_destroy(vox_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->dev);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     for (auto &kv : ctx->bufs)
         if (kv.second.p) (void)hipFree(kv.second.p);
     if (ctx->own_mesh) {
@@ -1374,11 +1353,7 @@ void vox_destroy(vox_ctx *ctx) {
     ctx->workers.clear();
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->up) (void)hipHostFree(ctx->up);
-    if (ctx->up_ev) (void)hipEventDestroy(ctx->up_ev);
-    if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
-    if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->cost_params) (void)hipFree(ctx->cost_params);
-    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -1578,24 +1553,8 @@ vox_status vox_plan_grid(vox_ctx *ctx, vox_plan_mode mode, double param, uint32_
                     mode == VOX_PLAN_MAX_DIMENSION ? "maxDimension must be >= 2"
                                                    : "cubeLength must be > 0");
     VOX_HIP(hipSetDevice(ctx->dev));
-    uint32_t *bb;
-    VOX_TRY(buf(ctx, "p_bbox", 6, &bb));
-    VOX_TRY(fill_many(ctx, {{bb, 3, UINT32_MAX}, {bb + 3, 3, 0u}}));
-    k_bbox<<<grid_for(ctx->nv, 256, 256), 256, 0, ctx->stream>>>(ctx->V, ctx->nv, bb);
-    VOX_HIP(hipGetLastError());
-    uint32_t h[6];
-    VOX_TRY(read_u32(ctx, bb, 6, h));
     double mn[3], mx[3];
-    for (int c = 0; c < 3; c++) {
-        uint32_t a = h[c], b = h[3 + c];
-        uint32_t ua = (a & 0x80000000u) ? (a & 0x7FFFFFFFu) : ~a;
-        uint32_t ub = (b & 0x80000000u) ? (b & 0x7FFFFFFFu) : ~b;
-        float fa, fb;
-        std::memcpy(&fa, &ua, 4);
-        std::memcpy(&fb, &ub, 4);
-        mn[c] = fa;
-        mx[c] = fb;
-    }
+    VOX_TRY(device_bbox(ctx, ctx->V, ctx->nv, mn, mx));
     plan_from_bbox(mn, mx, mode, param, vsx, g);
     return VOX_OK;
 }
@@ -1664,8 +1623,10 @@ vox_status vox_solid_bits(vox_ctx *ctx, const vox_grid *g, const double shift[3]
     PlanDev D;
     record(ctx, 0);
     VOX_TRY(plan_upload(ctx, P, D, sy, sz));
-    VOX_TRY(records_stage(ctx, P, D));
-    VOX_TRY(solid_stage(ctx, P, D));
+    Prep R;
+    ErodeBufs E;
+    VOX_TRY(prepare(ctx, P, D, R, E));
+    VOX_TRY(solid_fill(ctx, P, D, R));
     record(ctx, 1);
     if (ctx->timing) {
         VOX_HIP(hipEventSynchronize(ctx->ev[1]));
@@ -1761,27 +1722,6 @@ __global__ void k_unrotate_nodes(const uint8_t *__restrict__ in, uint8_t *__rest
     }
 }
 
-// Bounding box of n device vertices (calculateBoundingBox).
-vox_status device_bbox(vox_ctx *ctx, const float *V, uint32_t nv, double mn[3], double mx[3]) {
-    uint32_t *bb;
-    VOX_TRY(buf(ctx, "p_bbox", 6, &bb));
-    VOX_TRY(fill_many(ctx, {{bb, 3, UINT32_MAX}, {bb + 3, 3, 0u}}));
-    k_bbox<<<grid_for(nv, 256, 256), 256, 0, ctx->stream>>>(V, nv, bb);
-    VOX_HIP(hipGetLastError());
-    uint32_t h[6];
-    VOX_TRY(read_u32(ctx, bb, 6, h));
-    for (int c = 0; c < 3; c++) {
-        uint32_t a = h[c], b = h[3 + c];
-        uint32_t ua = (a & 0x80000000u) ? (a & 0x7FFFFFFFu) : ~a;
-        uint32_t ub = (b & 0x80000000u) ? (b & 0x7FFFFFFFu) : ~b;
-        float fa, fb;
-        std::memcpy(&fa, &ua, 4);
-        std::memcpy(&fb, &ub, 4);
-        mn[c] = fa;
-        mx[c] = fb;
-    }
-    return VOX_OK;
-}
 }  // namespace
 
 vox_status vox_voxelize_partition(vox_ctx *ctx, const vox_grid *g, vox_node_kind kind,
@@ -1833,8 +1773,10 @@ vox_status vox_solid_bits_partition(vox_ctx *ctx, const vox_grid *g, const uint3
     PlanDev D;
     record(ctx, 0);
     VOX_TRY(plan_upload(ctx, P, D, sy, sz));
-    VOX_TRY(records_stage(ctx, P, D));
-    VOX_TRY(solid_stage(ctx, P, D));
+    Prep R;
+    ErodeBufs E;
+    VOX_TRY(prepare(ctx, P, D, R, E));
+    VOX_TRY(solid_fill(ctx, P, D, R));
     record(ctx, 1);
     if (ctx->timing) {
         VOX_HIP(hipEventSynchronize(ctx->ev[1]));
@@ -2189,6 +2131,7 @@ vox_status graph_capture(vox_graph *g) {
     VOX_TRY(buf(w, "s_pmask", w->cap_solid, &u16));
     VOX_TRY(buf(w, "s_list_mask", w->cap_solid, &u16));
     VOX_TRY(buf(w, "f_blist", w->cap_surf, &u));
+    VOX_TRY(buf(w, "f_place", w->cap_surf, &u));
     VOX_TRY(buf(w, "s_first", block_starts_size(w->cap_solid), &u));
     VOX_TRY(buf(w, "f_first", block_starts_size(w->cap_surf), &u));
     VOX_TRY(buf(w, "e_changes", (size_t)w->n_passes * nj, &u));

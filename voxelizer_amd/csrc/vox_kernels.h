@@ -1,10 +1,11 @@
 // vox_kernels.h -- HIP kernels of the voxelizer hot path (gfx950, wave64).
 //
-// Solid stage:   k_solid_setup -> scan -> k_block_starts -> k_solid_candidates -> scan ->
-//                k_solid_scatter -> k_solid_fill (LDS-staged crossings +
-//                per-row prefix XOR, one coalesced write per bit word).
-// Surface stage: k_surf_setup -> scan -> k_block_starts -> k_surf_bin (count) -> scan ->
-//                k_surf_bin (scatter) -> k_surf_brick (LDS atomicMax winners).
+// Preparation:   k_tri_setup -> scan -> k_block_starts -> k_pairs_count -> scan ->
+//                k_pairs_place: the (triangle, tile) pairs of the solid stage and
+//                the (triangle, brick) pairs of the surface stage, sorted.
+// Solid stage:   k_solid_fill (LDS-staged crossings + per-row prefix XOR, one
+//                coalesced write per bit word).
+// Surface stage: k_surf_brick (LDS atomicMax winners).
 // Nodes:         k_erode (bitwise 6-neighbour erosion passes) ->
 //                k_nodes_cart / k_nodes_fcc (bid/mask + material, node write).
 #pragma once
@@ -237,6 +238,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
     return v;
 }
 
+// Inclusive maximum over the wave's lanes, the same way.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return v;
+}
+
 // Wave-aggregated atomic bump: one global atomic per wave.
 __device__ __forceinline__ uint32_t wave_bump(uint32_t *counter, bool pred) {
     unsigned long long mask = __ballot(pred);
@@ -252,7 +264,7 @@ __device__ __forceinline__ uint32_t wave_bump(uint32_t *counter, bool pred) {
 
 // Block-level grouping of keys in an LDS hash table (256-thread blocks):
 // candidates that land in the same bin share one global atomic per block.
-constexpr uint32_t kAggSlots = 1024;
+constexpr uint32_t kAggSlots = 512;
 constexpr uint32_t kAggEmpty = 0xFFFFFFFFu;
 struct AggTable {
     uint32_t key[kAggSlots];
@@ -268,7 +280,7 @@ __device__ __forceinline__ void agg_clear(AggTable &T) {
 // Inserts key; returns its slot and, in rank, its 0-based order among the
 // block's items with the same key.
 __device__ __forceinline__ uint32_t agg_insert(AggTable &T, uint32_t key, uint32_t &rank) {
-    uint32_t h = (key * 2654435761u) >> 22;  // 10 bits
+    uint32_t h = (key * 2654435761u) >> 23;  // 9 bits
     while (true) {
         const uint32_t prev = atomicCAS(&T.key[h], kAggEmpty, key);
         if (prev == kAggEmpty || prev == key) break;
@@ -278,54 +290,76 @@ __device__ __forceinline__ uint32_t agg_insert(AggTable &T, uint32_t key, uint32
     return h;
 }
 
-__device__ __forceinline__ uint32_t upper_bound_u32(const uint32_t *__restrict__ a, uint32_t n,
-                                                    uint32_t key) {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] <= key)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
+// LDS of the candidate passes.
+struct CandLds {
+    AggTable agg;
+    uint32_t own[256], wmax[256 / kWave];
+};
 
 // ---------------------------------------------------------------------------
-// Scan (exclusive, uint32), 256 threads x 16 items per tile.  Up to
-// kScanDirectTiles tiles: k_scan_reduce (tile sums) then k_scan_down (each
-// tile adds the sums before it and scans itself); more: tiles scanned with
-// k_scan_blocks, their sums scanned recursively, then k_scan_add.  The
-// output has n + 2 entries: out[n] is the total mod 2^32 and out[n + 1] is 1
-// when the true total reached 2^32 (the offsets wrapped), else 0.  partials
-// holds 2 * tiles + 1 words (tile sums' low words, then their high words).
+// Scan (exclusive, uint32), 256 threads x 16 items per tile, of up to two arrays
+// at once: k_scan_reduce (tile sums) then k_scan_down (each tile adds the sums
+// before it and scans itself).  The candidate counts' sums come from their
+// producer, and a few tiles need none.  The output has n + 2 entries: out[n] is
+// the total mod 2^32 and out[n + 1] is 1 when the true total reached 2^32 (the
+// offsets wrapped), else 0.
 // ---------------------------------------------------------------------------
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;
-constexpr uint32_t kScanDirectTiles = 4096;
+// Tiles up to which k_scan_down adds 256-element sums (16 per tile).
+constexpr uint32_t kScanFineTiles = 4096;
+// A tile of few sums the values before it itself, which costs less than the
+// launch of k_scan_reduce.
+constexpr uint32_t kScanSmallTiles = 4;
 
-__global__ void k_scan_reduce(const uint32_t *__restrict__ in, uint32_t n,
-                              uint32_t *__restrict__ partials);
-__global__ void k_scan_down(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-                            uint32_t n, const uint32_t *__restrict__ partials);
+struct ScanSeg {
+    const uint32_t *in;
+    uint32_t *out;
+    uint32_t n;
+    uint32_t *part;     // partial sums: npart low words, npart high words (, npart nonzero counts)
+    uint32_t npart;
+    uint32_t per_tile;  // partial sums per tile; 0: none
+    uint32_t *host;     // pinned host words for the total and the wrap flag, or null
+    uint32_t *list;     // indices of the nonzero entries, or null
+    uint32_t *n_list;
+};
+struct ScanSegs {
+    ScanSeg s[2];
+};
+__global__ void k_scan_reduce(ScanSegs segs);
+__global__ void k_scan_down(ScanSegs segs);
 
-__global__ void k_scan_blocks(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-                              uint32_t n, uint32_t *__restrict__ partials);
-__global__ void k_scan_add(uint32_t *__restrict__ out, uint32_t n,
-                           const uint32_t *__restrict__ partials,
-                           const uint32_t *__restrict__ psum);
+// ---------------------------------------------------------------------------
+// Fills
+// ---------------------------------------------------------------------------
+// Several fills in one launch (each launch on the stream costs a few
+// microseconds whatever its size).
+constexpr int kMaxFillSegs = 16;
+struct FillSegs {
+    uint32_t *p[kMaxFillSegs];
+    size_t n[kMaxFillSegs];
+    uint32_t v[kMaxFillSegs];
+    int count;
+};
+__device__ __forceinline__ void fill_segs(const FillSegs &s, uint32_t block, uint32_t blocks) {
+    for (int k = 0; k < s.count; k++)
+        for (size_t i = (size_t)block * blockDim.x + threadIdx.x; i < s.n[k];
+             i += (size_t)blocks * blockDim.x)
+            s.p[k][i] = s.v[k];
+}
 
 // ---------------------------------------------------------------------------
 // Grid planning
 // ---------------------------------------------------------------------------
-__global__ void k_bbox(const float *__restrict__ V, uint32_t nv, uint32_t *__restrict__ out6);
+// out: six keys per block (minimum x, y, z, maximum x, y, z).
+__global__ void k_bbox(const float *__restrict__ V, uint32_t nv, uint32_t *__restrict__ out);
 
 // ---------------------------------------------------------------------------
 // Solid
 // ---------------------------------------------------------------------------
 struct SolidParams {
-    const float4 *rec;  // per-triangle vertex records (k_tri_records)
+    const float4 *rec;  // per-triangle vertex records (k_tri_setup)
     double emx, emy, emz, d;
     uint32_t smin[2], smax[2];  // y/z extent of the centres, ext coords
     uint32_t tilesY;            // (ext y + 3) / 4
@@ -352,56 +386,75 @@ __device__ __forceinline__ SolidParams solid_params(const Job &J, const float4 *
     return p;
 }
 
-// The (triangle, tile) and (triangle, brick) pair passes take the first
-// min(total, cap) candidates; a total above cap sets *ovf (a replayed graph
-// sized by an earlier run reports that its lists were too short).
-// Per-triangle records: vertices v0, v1, v2 in 48 contiguous bytes
+// Triangle setup.  Records: vertices v0, v1, v2 in 48 contiguous bytes
 // (rec[3t] = v0.xyz v1.x, rec[3t+1] = v1.yz v2.xy, rec[3t+2] = v2.z, class
-// word (surface stage), 0, 0), one per triangle slot of every job; tri_job
-// holds each slot's job.  nslots is a multiple of 256 and the per-triangle
-// kernels run 256-thread blocks.
-__global__ void k_tri_records(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_bases,
-                              uint32_t njobs, uint32_t nslots, float4 *__restrict__ rec,
-                              uint32_t *__restrict__ tri_job);
-__global__ void k_solid_setup(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_bases,
-                              uint32_t njobs, uint32_t nslots, const float4 *__restrict__ rec,
-                              uint32_t *__restrict__ cand_count, uint4 *__restrict__ cbox);
-// first[b] = the triangle holding candidate 256*b of a candidate pass (cand_off:
-// exclusive offsets, nslots + 1 entries); candidates at or past cap are skipped.
-__global__ void k_block_starts(const uint32_t *__restrict__ cand_off, uint32_t nslots,
-                               uint32_t cap, uint32_t *__restrict__ first);
+// word (surface stage), material, 0), one per triangle slot of every job;
+// tri_job holds each slot's job (null for one job).  tri_blocks = slots / 256.
+struct TriSetup {
+    float4 *rec;
+    uint32_t *tri_job;
+    uint32_t *off_s;   // candidate tiles per slot (scanned in place afterwards)
+    uint4 *cbox;
+    uint32_t *part_s;  // 256-slot sums: tri_blocks low words, tri_blocks high words
+    uint32_t *off_f;   // candidate bricks per slot; null: no surface stage
+    uint4 *tri_info, *tri_ext;
+    uint32_t *part_f;
+};
+__global__ void k_tri_setup(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_bases,
+                            uint32_t njobs, uint32_t tri_blocks, TriSetup o, FillSegs clear);
+// first[b] = the triangle holding candidate 256*b of a candidate pass (off:
+// exclusive offsets, nslots + 2 entries); candidates at or past cap are skipped.
+struct BlockStarts {
+    const uint32_t *off;
+    uint32_t cap;
+    uint32_t *first;
+};
+__global__ void k_block_starts(BlockStarts a, BlockStarts b, uint32_t nslots);
 inline size_t block_starts_size(uint32_t total) { return (size_t)(total + 255u) / 256u + 1u; }
-// With pmask (jobs with several y/z subspaces), pmask[c] receives the rows of
-// the candidate's tile whose subspace queues the triangle (bit r = centre row
-// r of the tile, y fastest); the scatter pass carries it into list_mask and
-// the fill applies a triangle's crossings only on those rows.
+// The pair passes take the first min(total, cap) candidates; a total above cap
+// sets *ovf (a replayed graph sized by an earlier run reports that its lists
+// were too short).  With pmask (jobs with several y/z subspaces), pmask[c]
+// receives the rows of the candidate's tile whose subspace queues the triangle
+// (bit r = centre row r of the tile, y fastest); the placing pass carries it into
+// list_mask and the fill applies a triangle's crossings only on those rows.
+struct SolidPairs {
+    const float4 *rec;
+    const uint32_t *off, *first;
+    const uint4 *cbox;
+    uint2 *pairs;       // (tile, place in the tile's list) per candidate
+    uint16_t *pmask;
+    uint32_t *hist;     // pairs per tile
+    const uint32_t *bin_off;
+    uint32_t *list;
+    uint16_t *list_mask;
+    uint32_t cap;
+    uint32_t *ovf;
+};
+struct SurfPairs {
+    const uint32_t *off, *first;
+    const uint4 *tri_info;
+    uint32_t *place;    // place in the brick's list per candidate
+    uint32_t *hist;     // pairs per brick
+    const uint32_t *bin_off;
+    uint32_t *list;
+    uint32_t cap;
+    uint32_t *ovf;
+};
 template <bool kMulti>
-__global__ void k_solid_candidates(const Job *__restrict__ jobs,
-                                   const uint32_t *__restrict__ tri_job, uint32_t nslots,
-                                   const float4 *__restrict__ rec,
-                                   const uint32_t *__restrict__ cand_off,
-                                   const uint32_t *__restrict__ cand_total,
-                                   const uint32_t *__restrict__ first,
-                                   const uint4 *__restrict__ cbox, uint2 *__restrict__ pairs,
-                                   uint16_t *__restrict__ pmask,
-                                   uint32_t *__restrict__ tile_hist, uint32_t cap,
-                                   uint32_t *__restrict__ ovf);
-__global__ void k_solid_scatter(const uint2 *__restrict__ pairs,
-                                const uint16_t *__restrict__ pmask,
-                                const uint32_t *__restrict__ cand_total,
-                                const uint32_t *__restrict__ tile_off,
-                                uint32_t *__restrict__ tile_cursor, uint32_t *__restrict__ list,
-                                uint16_t *__restrict__ list_mask, uint32_t cap);
-// One workgroup per tile of every job (grid = all tiles).
+__global__ void k_pairs_count(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_job,
+                              uint32_t nslots, SolidPairs a, SurfPairs b, uint32_t solid_blocks);
+template <bool kMulti>
+__global__ void k_pairs_place(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_job,
+                              uint32_t nslots, SolidPairs a, SurfPairs b, uint32_t solid_blocks);
+// One workgroup per tile of every job, then one per kPadBlock words of pad rows.
 __global__ void k_solid_fill(const Job *__restrict__ jobs, const uint32_t *__restrict__ tile_bases,
-                             uint32_t njobs, const float4 *__restrict__ rec,
+                             const uint32_t *__restrict__ pad_bases, uint32_t njobs,
+                             const float4 *__restrict__ rec,
                              const uint32_t *__restrict__ tile_off,
                              const uint32_t *__restrict__ tile_hist,
                              const uint32_t *__restrict__ list,
                              const uint16_t *__restrict__ list_mask);
-// Zeroes the pad rows (y or z at the alloc border); grid = all jobs' blocks.
-__global__ void k_zero_pad_rows(const Job *__restrict__ jobs,
-                                const uint32_t *__restrict__ pad_bases, uint32_t njobs);
+constexpr uint32_t kPadBlock = 512;
 __host__ __device__ __forceinline__ uint32_t pad_words(uint32_t W, uint32_t rowsY,
                                                     uint32_t rowsZ) {
     return (2u * rowsZ + 2u * rowsY) * W;
@@ -410,19 +463,6 @@ __host__ __device__ __forceinline__ uint32_t pad_words(uint32_t W, uint32_t rows
 // ---------------------------------------------------------------------------
 // Surface
 // ---------------------------------------------------------------------------
-__global__ void k_surf_setup(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_bases,
-                             uint32_t njobs, uint32_t nslots, uint4 *__restrict__ tri_info,
-                             uint32_t *__restrict__ cand_count, uint4 *__restrict__ tri_ext,
-                             float4 *__restrict__ tri_rec);
-template <bool kMulti>
-__global__ void k_surf_bin(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_job,
-                           uint32_t nslots, const uint32_t *__restrict__ cand_off,
-                           const uint32_t *__restrict__ cand_total,
-                           const uint32_t *__restrict__ first,
-                           const uint4 *__restrict__ tri_info,
-                           uint32_t *__restrict__ brick_hist, const uint32_t *__restrict__ brick_off,
-                           uint32_t *__restrict__ brick_cursor, uint32_t *__restrict__ blist,
-                           int scatter, uint32_t cap, uint32_t *__restrict__ ovf);
 // kKeys: jobs with a keygrid also get their winner keys there (PartialNode).
 template <bool kKeys>
 __global__ void k_surf_brick(const Job *__restrict__ jobs, const uint32_t *__restrict__ brick_bases,
@@ -437,10 +477,6 @@ __global__ void k_surf_brick(const Job *__restrict__ jobs, const uint32_t *__res
                              const uint32_t *__restrict__ n_heavy,
                              const uint8_t *__restrict__ skip, uint32_t *__restrict__ next,
                              uint64_t *__restrict__ cycles);
-__global__ void k_nonzero_flags(const uint32_t *__restrict__ hist, uint32_t *__restrict__ flags,
-                                uint32_t n);
-__global__ void k_nonzero_list(const uint32_t *__restrict__ hist, const uint32_t *__restrict__ off,
-                               uint32_t *__restrict__ list, uint32_t n);
 
 // ---------------------------------------------------------------------------
 // Nodes

@@ -13,8 +13,7 @@ namespace vk {
 // ---------------------------------------------------------------------------
 // Every scan writes out[0, n] (exclusive prefix, out[n] = total mod 2^32) and
 // out[n + 1] = 1 if the true total reached 2^32 (the 32-bit offsets wrapped),
-// else 0.  Tile sums are kept in 64 bits for that: partials[b] holds tile b's
-// low word and partials[ntiles + b] its high word.
+// else 0; partial sums are kept in 64 bits for that.
 
 // Sum of one value per thread over a 256-thread block, in 64 bits.
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t s) {
@@ -32,50 +31,6 @@ __device__ __forceinline__ uint64_t block_sum_u64(uint64_t s) {
     for (uint32_t w = 0; w < kScanThreads / kWave; w++) t += wsum64[w];
     __syncthreads();  // wsum64 may be reused by the caller's next call
     return t;
-}
-
-// Exclusive scan of in[0, n) into out[0, n] (out[n] = total); one block scans
-// kScanTile elements and leaves its sum in partials[block] (low word) and
-// partials[nblocks + block] (high word).  The last block clears the wrap flag
-// out[n + 1]; k_scan_add sets it.
-__global__ __launch_bounds__(kScanThreads) void k_scan_blocks(const uint32_t *__restrict__ in,
-                                                              uint32_t *__restrict__ out,
-                                                              uint32_t n,
-                                                              uint32_t *__restrict__ partials) {
-    __shared__ uint32_t sh[kScanThreads];
-    const uint32_t tid = threadIdx.x;
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)tid * kScanItems;
-    uint32_t v[kScanItems];
-    uint32_t s = 0;
-    uint64_t s64 = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        uint64_t idx = base + k;
-        v[k] = idx < n ? in[idx] : 0u;
-        s += v[k];
-        s64 += v[k];
-    }
-    const uint64_t tile64 = block_sum_u64(s64);
-    sh[tid] = s;
-    __syncthreads();
-    for (uint32_t off = 1; off < kScanThreads; off <<= 1) {
-        uint32_t t = tid >= off ? sh[tid - off] : 0u;
-        __syncthreads();
-        sh[tid] += t;
-        __syncthreads();
-    }
-    uint32_t excl = tid ? sh[tid - 1] : 0u;
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        uint64_t idx = base + k;
-        if (idx <= n) out[idx] = excl;
-        excl += v[k];
-    }
-    if (tid == kScanThreads - 1) {
-        partials[blockIdx.x] = sh[tid];
-        partials[gridDim.x + blockIdx.x] = (uint32_t)(tile64 >> 32);
-    }
-    if (tid == 0 && blockIdx.x == gridDim.x - 1u) out[(uint64_t)n + 1u] = 0u;
 }
 
 // Block-wide sum and exclusive prefix of one value per thread: a wave scan
@@ -96,89 +51,147 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t s, uint32_t &total)
     return before + incl - s;
 }
 
-// Tile sums of in[0, n) (direct path): low words in partials[0, nblocks),
-// high words in partials[nblocks, 2 * nblocks).
-__global__ __launch_bounds__(kScanThreads) void k_scan_reduce(const uint32_t *__restrict__ in,
-                                                              uint32_t n,
-                                                              uint32_t *__restrict__ partials) {
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-    uint64_t s = 0u;
+// Sum over a 256-thread block of up to 2^32 / 256 per thread.
+__device__ __forceinline__ uint32_t block_sum_u32(uint32_t s) {
+    uint32_t total;
+    block_excl_scan(s, total);
+    __syncthreads();  // its LDS may be reused
+    return total;
+}
+
+// A thread's 16 consecutive values of a tile (0 past n), in 16-byte loads.
+__device__ __forceinline__ void scan_load(const uint32_t *in, uint32_t n, uint64_t base,
+                                          uint32_t v[kScanItems]) {
+    if (base + kScanItems <= n) {
 #pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        const uint64_t idx = base + k;
-        s += idx < n ? in[idx] : 0u;
-    }
-    const uint64_t total = block_sum_u64(s);
-    if (threadIdx.x == 0) {
-        partials[blockIdx.x] = (uint32_t)total;
-        partials[gridDim.x + blockIdx.x] = (uint32_t)(total >> 32);
+        for (int q = 0; q < kScanItems / 4; q++) {
+            const uint4 x = reinterpret_cast<const uint4 *>(in + base)[q];
+            v[4 * q] = x.x;
+            v[4 * q + 1] = x.y;
+            v[4 * q + 2] = x.z;
+            v[4 * q + 3] = x.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) v[k] = base + k < n ? in[base + k] : 0u;
     }
 }
 
-// Exclusive scan of in[0, n) into out[0, n] (out[n] = total), direct path:
-// the tile first sums the tile sums before it (at most kScanDirectTiles).
-// The last tile also adds them in 64 bits and writes the wrap flag.
-__global__ __launch_bounds__(kScanThreads) void k_scan_down(const uint32_t *__restrict__ in,
-                                                            uint32_t *__restrict__ out,
-                                                            uint32_t n,
-                                                            const uint32_t *__restrict__ partials) {
-    __shared__ uint32_t s_off;
-    const bool last = blockIdx.x == gridDim.x - 1u;
-    uint32_t p = 0u;
-    uint64_t p64 = 0u;
-    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) {
-        p += partials[i];
-        if (last) p64 += ((uint64_t)partials[gridDim.x + i] << 32) | partials[i];
-    }
-    uint32_t ptotal;
-    block_excl_scan(p, ptotal);
-    if (threadIdx.x == 0) s_off = ptotal;
-    __syncthreads();  // also orders the two uses of block_excl_scan's LDS
-    const uint32_t off = s_off;
+// Tile sums of each segment's in[0, n) (blockIdx.y: the segment):
+// low words in part[0, npart), high words in part[npart, 2 * npart) and, with a
+// list, the nonzero entries in part[2 * npart, 3 * npart).
+__global__ __launch_bounds__(kScanThreads) void k_scan_reduce(ScanSegs segs) {
+    const ScanSeg &S = segs.s[blockIdx.y];
+    if (blockIdx.x >= S.npart) return;  // uniform
     const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
-    uint32_t s = 0u;
+    scan_load(S.in, S.n, base, v);
+    uint64_t s = 0u;
+    uint32_t nz = 0u;
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
-        const uint64_t idx = base + k;
-        v[k] = idx < n ? in[idx] : 0u;
         s += v[k];
+        nz += v[k] != 0u ? 1u : 0u;
+    }
+    const uint64_t total = block_sum_u64(s);
+    if (S.list) nz = block_sum_u32(nz);
+    if (threadIdx.x == 0) {
+        S.part[blockIdx.x] = (uint32_t)total;
+        S.part[S.npart + blockIdx.x] = (uint32_t)(total >> 32);
+        if (S.list) S.part[2u * S.npart + blockIdx.x] = nz;
+    }
+}
+
+// Exclusive scan of each segment's in[0, n) into out[0, n] (out[n] = total):
+// a tile first adds the sums before it: those in part, each of
+// 1 / per_tile of a tile, or with per_tile = 0 (at most kScanSmallTiles tiles)
+// the values themselves.  The last tile also adds them in 64 bits and writes
+// the wrap flag, and both to `host` if given.  in may be out.  With a list, the
+// indices of the nonzero entries go there in order, their number to *n_list.
+__global__ __launch_bounds__(kScanThreads) void k_scan_down(ScanSegs segs) {
+    const ScanSeg &S = segs.s[blockIdx.y];
+    const uint32_t n = S.n, tiles = n / kScanTile + 1u;
+    if (blockIdx.x >= tiles) return;  // uniform
+    const bool last = blockIdx.x == tiles - 1u, listed = S.list != nullptr;
+    uint32_t p = 0u, pz = 0u;
+    uint64_t p64 = 0u;
+    if (S.per_tile) {
+        const uint32_t before = min(blockIdx.x * S.per_tile, S.npart);
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < before; i += kScanThreads) {
+            const uint32_t v = S.part[i];
+            p += v;
+            if (last) p64 += ((uint64_t)S.part[S.npart + i] << 32) | v;
+            if (listed) pz += S.part[2u * S.npart + i];
+        }
+    } else {
+        for (uint32_t b = 0; b < blockIdx.x; b++) {
+            uint32_t v[kScanItems];
+            scan_load(S.in, n, (uint64_t)b * kScanTile + threadIdx.x * kScanItems, v);
+#pragma unroll
+            for (int k = 0; k < kScanItems; k++) {
+                p += v[k];
+                if (last) p64 += v[k];
+                pz += v[k] != 0u ? 1u : 0u;
+            }
+        }
+    }
+    const uint32_t off = block_sum_u32(p);
+    const uint32_t zoff = listed ? block_sum_u32(pz) : 0u;
+    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
+    uint32_t v[kScanItems];
+    scan_load(S.in, n, base, v);
+    uint32_t s = 0u, nz = 0u;
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) {
+        s += v[k];
+        nz += v[k] != 0u ? 1u : 0u;
         if (last) p64 += v[k];
     }
     uint32_t total;
     uint32_t excl = off + block_excl_scan(s, total);
+    uint32_t e[kScanItems];
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
-        const uint64_t idx = base + k;
-        if (idx <= n) out[idx] = excl;
+        e[k] = excl;
         excl += v[k];
+    }
+    if (base + kScanItems <= n) {
+#pragma unroll
+        for (int q = 0; q < kScanItems / 4; q++)
+            reinterpret_cast<uint4 *>(S.out + base)[q] =
+                make_uint4(e[4 * q], e[4 * q + 1], e[4 * q + 2], e[4 * q + 3]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++)
+            if (base + k <= n) S.out[base + k] = e[k];
+    }
+    if (listed) {
+        __syncthreads();  // block_excl_scan's LDS
+        uint32_t ztotal;
+        uint32_t at = zoff + block_excl_scan(nz, ztotal);
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++)
+            if (v[k] != 0u) S.list[at++] = (uint32_t)base + (uint32_t)k;
+        if (last && threadIdx.x == 0) *S.n_list = zoff + ztotal;
     }
     if (last) {  // uniform
         const uint64_t all = block_sum_u64(p64);
-        if (threadIdx.x == 0) out[(uint64_t)n + 1u] = (all >> 32) != 0u ? 1u : 0u;
+        if (threadIdx.x == 0) {
+            const uint32_t wrap = (all >> 32) != 0u ? 1u : 0u;
+            S.out[(uint64_t)n + 1u] = wrap;
+            if (S.host) {
+                S.host[0] = (uint32_t)all;
+                S.host[1] = wrap;
+            }
+        }
     }
-}
-
-// Adds the scanned tile sums (recursive path) and sets the wrap flag when a
-// tile's sum or the sum of the tile sums reached 2^32 (psum[nblocks + 1] is
-// the recursive scan's own flag).
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(uint32_t *__restrict__ out,
-                                                           uint32_t n,
-                                                           const uint32_t *__restrict__ partials,
-                                                           const uint32_t *__restrict__ psum) {
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile;
-    const uint32_t add = psum[blockIdx.x];
-    for (uint32_t k = threadIdx.x; k < (uint32_t)kScanTile; k += kScanThreads) {
-        uint64_t idx = base + k;
-        if (idx <= n) out[idx] += add;
-    }
-    if (threadIdx.x == 0 &&
-        (partials[gridDim.x + blockIdx.x] != 0u || (blockIdx.x == 0 && psum[gridDim.x + 1u] != 0u)))
-        out[(uint64_t)n + 1u] = 1u;
 }
 
 // ---------------------------------------------------------------------------
-// Bounding box: order-preserving uint keys of the float coordinates.
+// Bounding box: order-preserving uint keys of the float coordinates, six per
+// block, left to the host to join (in its own memory: no clear, no atomics, no
+// copy back).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t fkey(float f) {
     uint32_t u = __float_as_uint(f);
@@ -186,7 +199,7 @@ __device__ __forceinline__ uint32_t fkey(float f) {
 }
 
 __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ V, uint32_t nv,
-                                              uint32_t *__restrict__ out6) {
+                                              uint32_t *__restrict__ out) {
     uint32_t mn[3] = {UINT32_MAX, UINT32_MAX, UINT32_MAX}, mx[3] = {0u, 0u, 0u};
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += gridDim.x * blockDim.x) {
 #pragma unroll
@@ -203,7 +216,7 @@ __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ V, uint3
             mx[c] = max(mx[c], (uint32_t)__shfl_xor((int)mx[c], off));
         }
     }
-    // Block reduction through LDS, then one set of atomics per block.
+    // Block reduction through LDS.
     __shared__ uint32_t red[6][256 / kWave];
     const uint32_t wv = threadIdx.x / kWave;
     if (lane_id() == 0) {
@@ -219,38 +232,13 @@ __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ V, uint3
         uint32_t r = red[c][0];
         for (uint32_t k = 1; k < blockDim.x / kWave; k++)
             r = c < 3 ? min(r, red[c][k]) : max(r, red[c][k]);
-        if (c < 3)
-            atomicMin(&out6[c], r);
-        else
-            atomicMax(&out6[c], r);
+        out[6u * blockIdx.x + c] = r;
     }
 }
 
 // ---------------------------------------------------------------------------
 // Solid stage
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_tri_records(const Job *__restrict__ jobs,
-                                                     const uint32_t *__restrict__ tri_bases,
-                                                     uint32_t njobs, uint32_t nslots,
-                                                     float4 *__restrict__ rec,
-                                                     uint32_t *__restrict__ tri_job) {
-    for (uint32_t t0 = blockIdx.x * 256u; t0 < nslots; t0 += gridDim.x * 256u) {
-        const uint32_t j = job_of(tri_bases, njobs, t0);
-        const Job &J = jobs[j];
-        const uint32_t t = t0 + threadIdx.x, lt = t - J.tri_base;
-        tri_job[t] = j;
-        if (lt >= J.nt) continue;  // padding slot
-        const VK_G float *V = gptr(J.V);
-        const VK_G uint32_t *I = gptr(J.I);
-        const uint32_t a = I[3u * lt], b = I[3u * lt + 1u], c = I[3u * lt + 2u];
-        rec[3 * (size_t)t] = make_float4(V[3u * a], V[3u * a + 1u], V[3u * a + 2u], V[3u * b]);
-        rec[3 * (size_t)t + 1] =
-            make_float4(V[3u * b + 1u], V[3u * b + 2u], V[3u * c], V[3u * c + 1u]);
-        const uint32_t mat = J.mats ? (uint32_t)gptr(J.mats)[lt] : 0u;
-        rec[3 * (size_t)t + 2] = make_float4(V[3u * c + 2u], 0.0f, __uint_as_float(mat), 0.0f);
-    }
-}
-
 // The triangle's vertices widened to FP64 (fetchTriangleVertices,
 // src/voxelizer.cu:2242-2253), from its 48-byte record.
 __device__ __forceinline__ void load_tri_d(const SolidParams &p, uint32_t t, D3 v[3]) {
@@ -261,51 +249,48 @@ __device__ __forceinline__ void load_tri_d(const SolidParams &p, uint32_t t, D3 
     v[2] = {(double)r1.z, (double)r1.w, (double)r2.x};
 }
 
-// Candidate tiles of each triangle: its commonSpace tile rectangle; the
-// commonSpace box itself is kept so the candidate pass needs no divisions.
-__global__ __launch_bounds__(256) void k_solid_setup(const Job *__restrict__ jobs,
-                                                     const uint32_t *__restrict__ tri_bases,
-                                                     uint32_t njobs, uint32_t nslots,
-                                                     const float4 *__restrict__ rec,
-                                                     uint32_t *__restrict__ cand_count,
-                                                     uint4 *__restrict__ cbox) {
-    for (uint32_t t0 = blockIdx.x * 256u; t0 < nslots; t0 += gridDim.x * 256u) {
-        const Job &J = jobs[job_of(tri_bases, njobs, t0)];
-        const SolidParams p = solid_params(J, rec);
-        const uint32_t t = t0 + threadIdx.x;
-        uint32_t c = 0;
-        if (t - J.tri_base < J.nt) {
-            D3 v[3];
-            load_tri_d(p, t, v);
-            TileSetup ts;
-            if (tile_setup(v, p.emy, p.emz, p.d, p.smin[0], p.smin[1], p.smax[0], p.smax[1],
-                           ts)) {
-                c = (ts.tmax[0] - ts.tmin[0] + 1u) * (ts.tmax[1] - ts.tmin[1] + 1u);
-                cbox[t] = make_uint4(ts.cmin[0], ts.cmin[1], ts.cmax[0], ts.cmax[1]);
-            }
-        }
-        cand_count[t] = c;
-    }
-}
-
-// One thread per candidate (triangle, tile): the reference's per-tile queue
-// test, done in parallel instead of one thread walking all tiles of a
-// triangle.  The triangle of a candidate is found by a binary search narrowed
-// to the triangles the block's candidates span.  Queued pairs are counted per
-// tile (LDS-grouped atomics) for the counting sort.
-// Block starts of a candidate pass: first[b] = the triangle that holds
+// Block starts of the candidate passes: first[b] = the triangle that holds
 // candidate 256*b (the passes' blocks take 256 consecutive candidates), so a
 // block bounds its triangles with two loads instead of a binary search over
 // the whole offset array (about 21 dependent loads on the large hall).
-// Candidates at or past `cap` are not processed.
-__global__ __launch_bounds__(256) void k_block_starts(const uint32_t *__restrict__ cand_off,
-                                                      uint32_t nslots, uint32_t cap,
-                                                      uint32_t *__restrict__ first) {
-    const uint32_t total = cand_off[nslots + 1u] ? 0u : min(cand_off[nslots], cap);
+// Candidates at or past `cap` are not processed.  blockIdx.y: the pass.
+__global__ __launch_bounds__(256) void k_block_starts(BlockStarts a, BlockStarts b,
+                                                      uint32_t nslots) {
+    const BlockStarts &S = blockIdx.y ? b : a;
+    const uint32_t total = S.off[nslots + 1u] ? 0u : min(S.off[nslots], S.cap);
     for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < nslots; t += gridDim.x * 256u) {
-        const uint32_t lo = min(cand_off[t], total), hi = min(cand_off[t + 1u], total);
-        for (uint32_t b = (lo + 255u) / 256u; b * 256u < hi; b++) first[b] = t;
+        const uint32_t lo = min(S.off[t], total), hi = min(S.off[t + 1u], total);
+        for (uint32_t k = (lo + 255u) / 256u; k * 256u < hi; k++) S.first[k] = t;
     }
+}
+
+// The triangle of candidate base + threadIdx.x, for a 256-thread block: the
+// triangles that start among its candidates (few and consecutive) leave their
+// number where they start, and a running maximum over the block spreads them.
+// One coalesced load and one scan, where a binary search per thread took eight
+// or more dependent loads.  Triangles without candidates start where the next
+// one does and lose to its larger number.
+__device__ __forceinline__ uint32_t block_owner(const uint32_t *__restrict__ off,
+                                                const uint32_t *__restrict__ first,
+                                                uint32_t nslots, uint32_t base, uint32_t total,
+                                                CandLds &L) {
+    const uint32_t b = base / 256u;
+    const uint32_t t0 = first[b], t1 = base + 256u < total ? first[b + 1u] : nslots - 1u;
+    L.own[threadIdx.x] = threadIdx.x == 0u ? t0 : 0u;
+    __syncthreads();
+    for (uint32_t t = t0 + threadIdx.x; t <= t1; t += 256u) {
+        const uint32_t o = off[t] - base;
+        if (o < 256u) atomicMax(&L.own[o], t);
+    }
+    __syncthreads();
+    const uint32_t incl = wave_incl_max(L.own[threadIdx.x]);
+    const uint32_t wave = threadIdx.x / kWave;
+    if (lane_id() == kWave - 1u) L.wmax[wave] = incl;
+    __syncthreads();
+    uint32_t t = incl;
+#pragma unroll
+    for (uint32_t w = 0; w + 1u < 256u / kWave; w++) t = max(t, w < wave ? L.wmax[w] : 0u);
+    return t;
 }
 
 // Rows of tile (ty, tz) whose voxSplitRes subspace queues the triangle (bit
@@ -368,44 +353,45 @@ __device__ __forceinline__ uint32_t tile_split_mask(const TileSetup &ts, uint32_
     return mask;
 }
 
+// Counts the block's candidates per bin and returns this one's place in its
+// bin: its rank among the block's (LDS table), after those counted before (one
+// global atomic per distinct bin).
+__device__ __forceinline__ uint32_t bin_place(CandLds &L, bool live, uint32_t bin,
+                                              uint32_t *__restrict__ hist) {
+    uint32_t slot = 0u, rank = 0u;
+    if (live) slot = agg_insert(L.agg, bin, rank);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kAggSlots; i += 256u)
+        if (L.agg.key[i] != kAggEmpty) L.agg.base[i] = atomicAdd(&hist[L.agg.key[i]], L.agg.cnt[i]);
+    __syncthreads();
+    return L.agg.base[slot] + rank;
+}
+
+// The solid pass's candidates: the reference's per-tile queue test, a thread
+// per (triangle, tile) instead of one walking all tiles of a triangle.
 template <bool kMulti>
-__global__ __launch_bounds__(256) void k_solid_candidates(
-    const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_job, uint32_t nslots,
-    const float4 *__restrict__ rec, const uint32_t *__restrict__ cand_off,
-    const uint32_t *__restrict__ cand_total, const uint32_t *__restrict__ first,
-    const uint4 *__restrict__ cbox, uint2 *__restrict__ pairs, uint16_t *__restrict__ pmask,
-    uint32_t *__restrict__ tile_hist, uint32_t cap, uint32_t *__restrict__ ovf) {
-    __shared__ uint32_t trange[2];
-    __shared__ AggTable agg;
-    // cand_total[1]: the candidate count reached 2^32 (the offsets wrapped).
-    const uint32_t full = *cand_total, total = cand_total[1] ? 0u : min(full, cap);
-    if (ovf && (full > cap || cand_total[1]) && blockIdx.x == 0 && threadIdx.x == 0) *ovf = 1u;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += stride) {
+__device__ __forceinline__ void count_solid(const Job *__restrict__ jobs,
+                                            const uint32_t *__restrict__ tri_job, uint32_t nslots,
+                                            const SolidPairs &a, uint32_t block, uint32_t blocks,
+                                            CandLds &L) {
+    // off[nslots + 1]: the candidate count reached 2^32 (the offsets wrapped).
+    const uint32_t full = a.off[nslots], wrap = a.off[nslots + 1u];
+    const uint32_t total = wrap ? 0u : min(full, a.cap);
+    if (a.ovf && (full > a.cap || wrap) && block == 0u && threadIdx.x == 0) *a.ovf = 1u;
+    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
         __syncthreads();
-        agg_clear(agg);
-        if (threadIdx.x < 2) {  // the triangles of candidates base and base + 256 bound the block's
-            const uint32_t b = base / 256u + threadIdx.x;
-            trange[threadIdx.x] = threadIdx.x == 0 || base + 256u < total ? first[b] : nslots - 1u;
-        }
-        __syncthreads();
+        agg_clear(L.agg);
         const uint32_t c = base + threadIdx.x;
+        const uint32_t t = block_owner(a.off, a.first, nslots, base, total, L);
         bool hit = false;
-        uint32_t t = 0, tile = 0;
+        uint32_t tile = 0;
         if (c < total) {
-            uint32_t lo = trange[0], hi = trange[1] + 1u;
-            while (lo + 1u < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (cand_off[mid] <= c) lo = mid;
-                else hi = mid;
-            }
-            t = lo;
             const Job &J = jobs[kMulti ? tri_job[t] : 0u];
-            const SolidParams p = solid_params(J, rec);
+            const SolidParams p = solid_params(J, a.rec);
             D3 v[3];
             load_tri_d(p, t, v);
             TileSetup ts;
-            const uint4 cb = cbox[t];
+            const uint4 cb = a.cbox[t];
             ts.cmin[0] = cb.x;
             ts.cmin[1] = cb.y;
             ts.cmax[0] = cb.z;
@@ -413,70 +399,138 @@ __global__ __launch_bounds__(256) void k_solid_candidates(
             tile_edges(v, ts);
             const uint32_t tmin0 = cb.x / 4u, tmin1 = cb.y / 4u, tmax0 = (cb.z - 1u) / 4u;
             const uint32_t w = tmax0 - tmin0 + 1u;
-            const uint32_t local = c - cand_off[t];
+            const uint32_t local = c - a.off[t];
             const uint32_t ty = tmin0 + local % w, tz = tmin1 + local / w;
             if (J.sstart) {  // several y/z subspaces
                 const uint32_t m = tile_split_mask(ts, ty, tz, p.emy, p.emz, p.d, J.sstart,
                                                    (uint32_t)J.res[1], J.sstart + J.res[1],
                                                    (uint32_t)J.res[2]);
                 hit = m != 0u;
-                pmask[c] = (uint16_t)m;
+                a.pmask[c] = (uint16_t)m;
             } else {
                 hit = tile_hit(ts, ty, tz, p.emy, p.emz, p.d);
             }
             tile = J.tile_base + tz * p.tilesY + ty;
         }
-        // One slot per candidate (no global counter); misses are skipped
-        // by the scatter pass.
-        if (c < total) pairs[c] = make_uint2(t, hit ? tile : UINT32_MAX);
-        __syncthreads();
-        uint32_t rank;
-        if (hit) agg_insert(agg, tile, rank);
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < kAggSlots; i += blockDim.x)
-            if (agg.key[i] != kAggEmpty) atomicAdd(&tile_hist[agg.key[i]], agg.cnt[i]);
+        const uint32_t place = bin_place(L, hit, tile, a.hist);
+        // One slot per candidate (no global counter); misses are skipped by
+        // the placing pass.
+        if (c < total) a.pairs[c] = make_uint2(hit ? tile : UINT32_MAX, place);
     }
 }
-template __global__ void k_solid_candidates<false>(const Job *, const uint32_t *, uint32_t,
-                                                   const float4 *, const uint32_t *,
-                                                   const uint32_t *, const uint32_t *,
-                                                   const uint4 *, uint2 *, uint16_t *,
-                                                   uint32_t *, uint32_t, uint32_t *);
-template __global__ void k_solid_candidates<true>(const Job *, const uint32_t *, uint32_t,
-                                                  const float4 *, const uint32_t *,
-                                                  const uint32_t *, const uint32_t *,
-                                                  const uint4 *, uint2 *, uint16_t *,
-                                                  uint32_t *, uint32_t, uint32_t *);
 
-__global__ __launch_bounds__(256) void k_solid_scatter(const uint2 *__restrict__ pairs,
-                                                       const uint16_t *__restrict__ pmask,
-                                                       const uint32_t *__restrict__ cand_total,
-                                                       const uint32_t *__restrict__ tile_off,
-                                                       uint32_t *__restrict__ tile_cursor,
-                                                       uint32_t *__restrict__ list,
-                                                       uint16_t *__restrict__ list_mask,
-                                                       uint32_t cap) {
-    __shared__ AggTable agg;
-    const uint32_t n = cand_total[1] ? 0u : min(*cand_total, cap);
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+// Brick of candidate c (of triangle t) of the surface pass.
+template <bool kMulti>
+__device__ __forceinline__ uint32_t cand_brick(const Job *__restrict__ jobs,
+                                               const uint32_t *__restrict__ tri_job,
+                                               const SurfPairs &a, uint32_t t, uint32_t c) {
+    const Job &J = jobs[kMulti ? tri_job[t] : 0u];
+    const uint4 ti = a.tri_info[t];
+    const uint32_t bx0 = ti.y & 0xFFFFu, by0 = ti.y >> 16, bz0 = ti.z & 0xFFFFu;
+    const uint32_t w0 = ti.z >> 16, w1 = ti.w & 0xFFFFu;
+    const uint32_t local = c - a.off[t];
+    const uint32_t bx = bx0 + local % w0;
+    const uint32_t by = by0 + (local / w0) % w1;
+    const uint32_t bz = bz0 + local / (w0 * w1);
+    return J.brick_base + (bz * J.nb[1] + by) * J.nb[0] + bx;
+}
+
+template <bool kMulti>
+__device__ __forceinline__ void count_surf(const Job *__restrict__ jobs,
+                                           const uint32_t *__restrict__ tri_job, uint32_t nslots,
+                                           const SurfPairs &a, uint32_t block, uint32_t blocks,
+                                           CandLds &L) {
+    const uint32_t full = a.off[nslots], wrap = a.off[nslots + 1u];
+    const uint32_t total = wrap ? 0u : min(full, a.cap);
+    if (a.ovf && (full > a.cap || wrap) && block == 0u && threadIdx.x == 0) *a.ovf = 1u;
+    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
         __syncthreads();
-        agg_clear(agg);
+        agg_clear(L.agg);
+        const uint32_t c = base + threadIdx.x;
+        const uint32_t t = block_owner(a.off, a.first, nslots, base, total, L);
+        const bool live = c < total;
+        const uint32_t b = live ? cand_brick<kMulti>(jobs, tri_job, a, t, c) : 0u;
+        const uint32_t place = bin_place(L, live, b, a.hist);
+        if (live) a.place[c] = place;
+    }
+}
+
+// The counting sorts of (triangle, tile) and (triangle, brick) pairs by tile and
+// by brick: this pass counts the pairs of each bin and keeps every pair's place
+// in its bin, so the placing pass needs no counters of its own.  Both sorts
+// share a launch: blocks [0, solid_blocks) take the first, the rest the second.
+template <bool kMulti>
+__global__ __launch_bounds__(256) void k_pairs_count(const Job *__restrict__ jobs,
+                                                     const uint32_t *__restrict__ tri_job,
+                                                     uint32_t nslots, SolidPairs a, SurfPairs b,
+                                                     uint32_t solid_blocks) {
+    __shared__ CandLds L;
+    if (blockIdx.x < solid_blocks)
+        count_solid<kMulti>(jobs, tri_job, nslots, a, blockIdx.x, solid_blocks, L);
+    else
+        count_surf<kMulti>(jobs, tri_job, nslots, b, blockIdx.x - solid_blocks,
+                           gridDim.x - solid_blocks, L);
+}
+
+template <bool kMulti>
+__global__ __launch_bounds__(256) void k_pairs_place(const Job *__restrict__ jobs,
+                                                     const uint32_t *__restrict__ tri_job,
+                                                     uint32_t nslots, SolidPairs a, SurfPairs b,
+                                                     uint32_t solid_blocks) {
+    __shared__ CandLds L;
+    const bool solid = blockIdx.x < solid_blocks;
+    const uint32_t block = solid ? blockIdx.x : blockIdx.x - solid_blocks;
+    const uint32_t blocks = solid ? solid_blocks : gridDim.x - solid_blocks;
+    const uint32_t *off = solid ? a.off : b.off, *first = solid ? a.first : b.first;
+    const uint32_t total = off[nslots + 1u] ? 0u : min(off[nslots], solid ? a.cap : b.cap);
+    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
         __syncthreads();
-        const uint32_t i = base + threadIdx.x;
-        uint2 pr = make_uint2(0u, UINT32_MAX);
-        uint32_t slot = 0, rank = 0;
-        if (i < n) pr = pairs[i];
-        const bool live = pr.y != UINT32_MAX;
-        if (live) slot = agg_insert(agg, pr.y, rank);
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < kAggSlots; k += blockDim.x)
-            if (agg.key[k] != kAggEmpty) agg.base[k] = atomicAdd(&tile_cursor[agg.key[k]], agg.cnt[k]);
-        __syncthreads();
-        if (live) {
-            const uint32_t pos = tile_off[pr.y] + agg.base[slot] + rank;
-            list[pos] = pr.x;
-            if (list_mask) list_mask[pos] = pmask[i];
+        const uint32_t c = base + threadIdx.x;
+        const uint32_t t = block_owner(off, first, nslots, base, total, L);
+        if (c >= total) continue;  // the last trip
+        if (solid) {
+            const uint2 pr = a.pairs[c];
+            if (pr.x == UINT32_MAX) continue;
+            const uint32_t pos = a.bin_off[pr.x] + pr.y;
+            a.list[pos] = t;
+            if (a.list_mask) a.list_mask[pos] = a.pmask[c];
+        } else {
+            b.list[b.bin_off[cand_brick<kMulti>(jobs, tri_job, b, t, c)] + b.place[c]] = t;
         }
+    }
+}
+template __global__ void k_pairs_count<false>(const Job *, const uint32_t *, uint32_t, SolidPairs,
+                                              SurfPairs, uint32_t);
+template __global__ void k_pairs_count<true>(const Job *, const uint32_t *, uint32_t, SolidPairs,
+                                             SurfPairs, uint32_t);
+template __global__ void k_pairs_place<false>(const Job *, const uint32_t *, uint32_t, SolidPairs,
+                                              SurfPairs, uint32_t);
+template __global__ void k_pairs_place<true>(const Job *, const uint32_t *, uint32_t, SolidPairs,
+                                             SurfPairs, uint32_t);
+
+// Zeroes kPadBlock words of the pad rows (y or z at the alloc border).
+__device__ __forceinline__ void zero_pad_rows(const Job *__restrict__ jobs,
+                                              const uint32_t *__restrict__ pad_bases,
+                                              uint32_t njobs, uint32_t block) {
+    const Job &J = jobs[job_of(pad_bases, njobs, block)];
+    const uint32_t W = J.gd.W, rowsY = J.gd.Y, rowsZ = J.gd.Z;
+    const uint32_t i0 = (block - J.pad_base) * kPadBlock, n = pad_words(W, rowsY, rowsZ);
+    for (uint32_t i = i0 + threadIdx.x; i < min(i0 + kPadBlock, n); i += kWave) {
+        const uint32_t r = i / W, w = i % W;
+        uint32_t y, z, bit;
+        if (r < 2u * rowsZ) {
+            z = r >> 1;
+            y = (r & 1u) ? rowsY - 1u : 0u;
+            bit = (r & 1u) ? 2u : 1u;
+        } else {
+            const uint32_t q = r - 2u * rowsZ;
+            y = q >> 1;
+            z = (q & 1u) ? rowsZ - 1u : 0u;
+            bit = (q & 1u) ? 8u : 4u;
+        }
+        // Rows and planes that are a neighbouring partition's overlap hold
+        // voxelized data (written by the fill) instead of padding.
+        if (J.padmask & bit) gptr(J.bits)[((size_t)z * rowsY + y) * W + w] = 0u;
     }
 }
 
@@ -484,9 +538,11 @@ __global__ __launch_bounds__(256) void k_solid_scatter(const uint2 *__restrict__
 // crossings toggle one bit each in an LDS copy of the tile's 16 rows
 // (ds_xor); a per-row prefix XOR then turns crossings into solid runs
 // (the suffix flips of src/voxelizer.cu:1487-1616) and each bit word is
-// written to HBM once, coalesced, with no global atomics.
+// written to HBM once, coalesced, with no global atomics.  The workgroups past
+// the tiles clear the pad rows.
 __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jobs,
                                                       const uint32_t *__restrict__ tile_bases,
+                                                      const uint32_t *__restrict__ pad_bases,
                                                       uint32_t njobs,
                                                       const float4 *__restrict__ rec,
                                                       const uint32_t *__restrict__ tile_off,
@@ -494,6 +550,11 @@ __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jo
                                                       const uint32_t *__restrict__ list,
                                                       const uint16_t *__restrict__ list_mask) {
     extern __shared__ __align__(16) uint32_t cross[];  // [16][SW]
+    const uint32_t n_tiles = tile_bases[njobs];
+    if (blockIdx.x >= n_tiles) {
+        zero_pad_rows(jobs, pad_bases, njobs, blockIdx.x - n_tiles);
+        return;
+    }
     const Job &J = jobs[job_of(tile_bases, njobs, blockIdx.x)];
     const SolidParams p = solid_params(J, rec);
     VK_G uint32_t *__restrict__ bits = gptr(J.bits);
@@ -576,30 +637,6 @@ __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jo
     }
 }
 
-__global__ __launch_bounds__(256) void k_zero_pad_rows(const Job *__restrict__ jobs,
-                                                       const uint32_t *__restrict__ pad_bases,
-                                                       uint32_t njobs) {
-    const Job &J = jobs[job_of(pad_bases, njobs, blockIdx.x)];
-    const uint32_t W = J.gd.W, rowsY = J.gd.Y, rowsZ = J.gd.Z;
-    const uint32_t i = (blockIdx.x - J.pad_base) * 256u + threadIdx.x;
-    if (i >= pad_words(W, rowsY, rowsZ)) return;
-    const uint32_t r = i / W, w = i % W;
-    uint32_t y, z, bit;
-    if (r < 2u * rowsZ) {
-        z = r >> 1;
-        y = (r & 1u) ? rowsY - 1u : 0u;
-        bit = (r & 1u) ? 2u : 1u;
-    } else {
-        const uint32_t q = r - 2u * rowsZ;
-        y = q >> 1;
-        z = (q & 1u) ? rowsZ - 1u : 0u;
-        bit = (q & 1u) ? 8u : 4u;
-    }
-    // Rows and planes that are a neighbouring partition's overlap hold
-    // voxelized data (written by the fill) instead of padding.
-    if (J.padmask & bit) gptr(J.bits)[((size_t)z * rowsY + y) * W + w] = 0u;
-}
-
 // ---------------------------------------------------------------------------
 // Surface stage
 // ---------------------------------------------------------------------------
@@ -633,125 +670,96 @@ __device__ __forceinline__ void brick_range(const SurfParams &p, const VoxBB &vb
     hi[2] = (uint32_t)(vb.max.z + p.off[2]) / (uint32_t)p.bdim[2];
 }
 
-// Per triangle: class and dominant axis (classifyTriangles), and the box of
-// bricks its clipped voxel range touches, packed as
-// {info, lo.x | lo.y<<16, lo.z | w.x<<16, w.y | w.z<<16}.  With tri_ext,
-// also its clipped voxel extents along (u, v, a) and its work items (voxels
-// for 1D, dominant-plane columns otherwise), the cost model's inputs.
-__global__ __launch_bounds__(256) void k_surf_setup(const Job *__restrict__ jobs,
-                                                    const uint32_t *__restrict__ tri_bases,
-                                                    uint32_t njobs, uint32_t nslots,
-                                                    uint4 *__restrict__ tri_info,
-                                                    uint32_t *__restrict__ cand_count,
-                                                    uint4 *__restrict__ tri_ext,
-                                                    float4 *__restrict__ tri_rec) {
-    for (uint32_t t0 = blockIdx.x * 256u; t0 < nslots; t0 += gridDim.x * 256u) {
-        const Job &J = jobs[job_of(tri_bases, njobs, t0)];
-        const uint32_t t = t0 + threadIdx.x;
-        if (t - J.tri_base >= J.nt || !J.use_mats) {  // padding, or no surface wanted
-            cand_count[t] = 0u;
-            continue;
+// Per triangle, from one read of its vertices: the 48-byte record, the solid
+// pass's candidate tiles (its commonSpace tile rectangle; the box itself is kept
+// so the candidate pass needs no divisions) and, for jobs with a surface stage,
+// its class and dominant axis (classifyTriangles) and the box of bricks its
+// clipped voxel range touches, packed as
+// {info, lo.x | lo.y<<16, lo.z | w.x<<16, w.y | w.z<<16}.  With tri_ext, also
+// its clipped voxel extents along (u, v, a) and its work items (voxels for 1D,
+// dominant-plane columns otherwise), the cost model's inputs.  A block leaves
+// the sums of its candidate counts for the scans.  The blocks past the
+// triangles clear what the call counts into.
+__global__ __launch_bounds__(256) void k_tri_setup(const Job *__restrict__ jobs,
+                                                   const uint32_t *__restrict__ tri_bases,
+                                                   uint32_t njobs, uint32_t tri_blocks,
+                                                   TriSetup o, FillSegs clear) {
+    if (blockIdx.x >= tri_blocks) {
+        fill_segs(clear, blockIdx.x - tri_blocks, gridDim.x - tri_blocks);
+        return;
+    }
+    const uint32_t t0 = blockIdx.x * 256u, j = job_of(tri_bases, njobs, t0);
+    const Job &J = jobs[j];
+    const uint32_t t = t0 + threadIdx.x, lt = t - J.tri_base;
+    if (o.tri_job) o.tri_job[t] = j;
+    uint32_t cs = 0u, cf = 0u;
+    if (lt < J.nt) {  // not a padding slot
+        const VK_G float *V = gptr(J.V);
+        const VK_G uint32_t *I = gptr(J.I);
+        const uint32_t ia = I[3u * lt], ib = I[3u * lt + 1u], ic = I[3u * lt + 2u];
+        const F3 tri[3] = {{V[3u * ia], V[3u * ia + 1u], V[3u * ia + 2u]},
+                           {V[3u * ib], V[3u * ib + 1u], V[3u * ib + 2u]},
+                           {V[3u * ic], V[3u * ic + 1u], V[3u * ic + 2u]}};
+        const uint32_t mat = J.mats ? (uint32_t)gptr(J.mats)[lt] : 0u;
+        {
+            const SolidParams p = solid_params(J, nullptr);
+            D3 v[3];
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                v[k] = {(double)tri[k].x, (double)tri[k].y, (double)tri[k].z};
+            TileSetup ts;
+            if (tile_setup(v, p.emy, p.emz, p.d, p.smin[0], p.smin[1], p.smax[0], p.smax[1],
+                           ts)) {
+                cs = (ts.tmax[0] - ts.tmin[0] + 1u) * (ts.tmax[1] - ts.tmin[1] + 1u);
+                o.cbox[t] = make_uint4(ts.cmin[0], ts.cmin[1], ts.cmax[0], ts.cmax[1]);
+            }
         }
-        const SurfParams p = surf_params(J);
-        const float4 r0 = tri_rec[3 * (size_t)t], r1 = tri_rec[3 * (size_t)t + 1],
-                     r2 = tri_rec[3 * (size_t)t + 2];
-        const F3 tri[3] = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, {r1.z, r1.w, r2.x}};
-        // One voxel range for the class and for the brick box.
-        F3 mn, mx;
-        tri_bounds(tri, mn, mx);
-        VoxBB vb = voxel_bounds_half(mn, mx, p.m, p.d);
-        int bb, axis;
-        classify_vb(tri, vb, bb, axis);
-        uint32_t c = 0;
-        uint32_t lo[3] = {0, 0, 0}, w[3] = {0, 0, 0};
-        uint4 ext = make_uint4(0u, 0u, 0u, 0u);
-        if (bb != BB_DEGEN && surf_clip(p, vb)) {
-            uint32_t hi[3];
-            brick_range(p, vb, lo, hi);
-            for (int a = 0; a < 3; a++) w[a] = hi[a] - lo[a] + 1u;
-            c = w[0] * w[1] * w[2];
-            const uint32_t eu = (uint32_t)(pick3i(vb.max, axis_u(axis)) - pick3i(vb.min, axis_u(axis)) + 1);
-            const uint32_t ev = (uint32_t)(pick3i(vb.max, axis_v(axis)) - pick3i(vb.min, axis_v(axis)) + 1);
-            const uint32_t ea = (uint32_t)(pick3i(vb.max, axis) - pick3i(vb.min, axis) + 1);
-            ext = make_uint4(eu, ev, ea, bb == BB_1D ? ea : eu * ev);
+        uint32_t info = 0u;
+        if (o.off_f && J.use_mats) {
+            const SurfParams p = surf_params(J);
+            // One voxel range for the class and for the brick box.
+            F3 mn, mx;
+            tri_bounds(tri, mn, mx);
+            VoxBB vb = voxel_bounds_half(mn, mx, p.m, p.d);
+            int bb, axis;
+            classify_vb(tri, vb, bb, axis);
+            uint32_t lo[3] = {0, 0, 0}, w[3] = {0, 0, 0};
+            uint4 ext = make_uint4(0u, 0u, 0u, 0u);
+            if (bb != BB_DEGEN && surf_clip(p, vb)) {
+                uint32_t hi[3];
+                brick_range(p, vb, lo, hi);
+                for (int a = 0; a < 3; a++) w[a] = hi[a] - lo[a] + 1u;
+                cf = w[0] * w[1] * w[2];
+                const uint32_t eu = (uint32_t)(pick3i(vb.max, axis_u(axis)) - pick3i(vb.min, axis_u(axis)) + 1);
+                const uint32_t ev = (uint32_t)(pick3i(vb.max, axis_v(axis)) - pick3i(vb.min, axis_v(axis)) + 1);
+                const uint32_t ea = (uint32_t)(pick3i(vb.max, axis) - pick3i(vb.min, axis) + 1);
+                ext = make_uint4(eu, ev, ea, bb == BB_1D ? ea : eu * ev);
+            }
+            info = ((uint32_t)bb << 30) | ((uint32_t)axis << 28);
+            o.tri_info[t] = make_uint4(info, lo[0] | (lo[1] << 16), lo[2] | (w[0] << 16),
+                                       w[1] | (w[2] << 16));
+            if (o.tri_ext) o.tri_ext[t] = ext;
         }
-        const uint32_t info = ((uint32_t)bb << 30) | ((uint32_t)axis << 28);
-        tri_info[t] = make_uint4(info, lo[0] | (lo[1] << 16), lo[2] | (w[0] << 16),
-                                 w[1] | (w[2] << 16));
-        // The class word goes into the triangle's record for the brick pass.
-        reinterpret_cast<float *>(tri_rec)[12 * (size_t)t + 9] = __uint_as_float(info);
-        cand_count[t] = c;
-        if (tri_ext) tri_ext[t] = ext;
+        // The class word goes into the record for the brick pass.
+        o.rec[3 * (size_t)t] = make_float4(tri[0].x, tri[0].y, tri[0].z, tri[1].x);
+        o.rec[3 * (size_t)t + 1] = make_float4(tri[1].y, tri[1].z, tri[2].x, tri[2].y);
+        o.rec[3 * (size_t)t + 2] = make_float4(tri[2].z, __uint_as_float(info),
+                                               __uint_as_float(mat), 0.0f);
+    }
+    o.off_s[t] = cs;
+    const uint64_t ss = block_sum_u64(cs);
+    if (threadIdx.x == 0) {
+        o.part_s[blockIdx.x] = (uint32_t)ss;
+        o.part_s[tri_blocks + blockIdx.x] = (uint32_t)(ss >> 32);
+    }
+    if (!o.off_f) return;
+    o.off_f[t] = cf;
+    const uint64_t sf = block_sum_u64(cf);
+    if (threadIdx.x == 0) {
+        o.part_f[blockIdx.x] = (uint32_t)sf;
+        o.part_f[tri_blocks + blockIdx.x] = (uint32_t)(sf >> 32);
     }
 }
-
-// One thread per (triangle, brick) candidate: counting pass (scatter = 0)
-// or placement pass (scatter = 1) of the counting sort by brick.  The
-// triangle of candidate c is found by binary search in the candidate offsets,
-// narrowed per block to the triangles its 256 candidates span.
-template <bool kMulti>
-__global__ __launch_bounds__(256) void k_surf_bin(
-    const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_job, uint32_t nslots,
-    const uint32_t *__restrict__ cand_off, const uint32_t *__restrict__ cand_total,
-    const uint32_t *__restrict__ first, const uint4 *__restrict__ tri_info,
-    uint32_t *__restrict__ brick_hist,
-    const uint32_t *__restrict__ brick_off, uint32_t *__restrict__ brick_cursor,
-    uint32_t *__restrict__ blist, int scatter, uint32_t cap, uint32_t *__restrict__ ovf) {
-    __shared__ uint32_t trange[2];
-    __shared__ AggTable agg;
-    const uint32_t full = *cand_total, total = cand_total[1] ? 0u : min(full, cap);
-    if (ovf && (full > cap || cand_total[1]) && blockIdx.x == 0 && threadIdx.x == 0) *ovf = 1u;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += gridDim.x * blockDim.x) {
-        __syncthreads();
-        agg_clear(agg);
-        if (threadIdx.x < 2) {  // the triangles of candidates base and base + 256 bound the block's
-            const uint32_t b = base / 256u + threadIdx.x;
-            trange[threadIdx.x] = threadIdx.x == 0 || base + 256u < total ? first[b] : nslots - 1u;
-        }
-        __syncthreads();
-        const uint32_t c = base + threadIdx.x;
-        const bool live = c < total;
-        uint32_t lo = trange[0], hi = trange[1] + 1u;
-        if (!live) lo = hi = 0u;
-        while (lo + 1u < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (cand_off[mid] <= c) lo = mid;
-            else hi = mid;
-        }
-        const uint32_t t = lo;
-        uint32_t b = 0, slot = 0, rank = 0;
-        if (live) {
-            const Job &J = jobs[kMulti ? tri_job[t] : 0u];
-            const uint4 ti = tri_info[t];
-            const uint32_t bx0 = ti.y & 0xFFFFu, by0 = ti.y >> 16, bz0 = ti.z & 0xFFFFu;
-            const uint32_t w0 = ti.z >> 16, w1 = ti.w & 0xFFFFu;
-            const uint32_t local = c - cand_off[t];
-            const uint32_t bx = bx0 + local % w0;
-            const uint32_t by = by0 + (local / w0) % w1;
-            const uint32_t bz = bz0 + local / (w0 * w1);
-            b = J.brick_base + (bz * J.nb[1] + by) * J.nb[0] + bx;
-            slot = agg_insert(agg, b, rank);
-        }
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < kAggSlots; k += blockDim.x) {
-            if (agg.key[k] == kAggEmpty) continue;
-            if (!scatter)
-                atomicAdd(&brick_hist[agg.key[k]], agg.cnt[k]);
-            else
-                agg.base[k] = atomicAdd(&brick_cursor[agg.key[k]], agg.cnt[k]);
-        }
-        __syncthreads();
-        if (live && scatter) blist[brick_off[b] + agg.base[slot] + rank] = t;
-    }
-}
-template __global__ void k_surf_bin<false>(const Job *, const uint32_t *, uint32_t,
-                                           const uint32_t *, const uint32_t *, const uint32_t *,
-                                           const uint4 *, uint32_t *, const uint32_t *,
-                                           uint32_t *, uint32_t *, int, uint32_t, uint32_t *);
-template __global__ void k_surf_bin<true>(const Job *, const uint32_t *, uint32_t,
-                                          const uint32_t *, const uint32_t *, const uint32_t *,
-                                          const uint4 *, uint32_t *, const uint32_t *,
-                                          uint32_t *, uint32_t *, int, uint32_t, uint32_t *);
 
 // Winner key of a (triangle, voxel) hit; the largest key of a voxel wins
 // (bbType first, then the mesh-local triangle index, as the oracle's rule).
@@ -1433,20 +1441,6 @@ template __global__ void k_surf_brick<true>(const Job *, const uint32_t *, uint3
                                             const uint32_t *, const uint32_t *, const uint32_t *,
                                             const uint32_t *, const uint8_t *, uint32_t *,
                                             uint64_t *);
-
-// Non-empty bricks in index order: flags, then (after an exclusive scan of
-// the flags) the compacted list.
-__global__ __launch_bounds__(256) void k_nonzero_flags(const uint32_t *__restrict__ hist,
-                                                       uint32_t *__restrict__ flags, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        flags[i] = hist[i] != 0u ? 1u : 0u;
-}
-__global__ __launch_bounds__(256) void k_nonzero_list(const uint32_t *__restrict__ hist,
-                                                      const uint32_t *__restrict__ off,
-                                                      uint32_t *__restrict__ list, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        if (hist[i] != 0u) list[off[i]] = i;
-}
 
 // ---------------------------------------------------------------------------
 // Erosion: removal of solid voxels that lack a solid neighbour on some axis

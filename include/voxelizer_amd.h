@@ -291,10 +291,13 @@ vox_status vox_mlp_grad(vox_ctx *ctx, const float *params_dev, const float *x_de
 
 /* ---- surface brick shape and its autotuner (no counterpart in the
  * reference) -------------------------------------------------------------
- * The surface pass works on bricks of voxels (default 128x4x8 on Cartesian
- * grids, 64x4x4 on each FCC sub-grid).  Shapes are powers of two with x a
- * multiple of 64, y*z <= 32 rows and 256 to 4096 voxels; Cartesian shapes
- * need z a multiple of 4.  The shape changes speed only, never output. */
+ * The surface pass works on bricks of voxels.  Until a shape is set the grid
+ * decides: 32x8x16 (32x16x8 for at most 8 planes) or, where that pads too much,
+ * 128x4x8 on Cartesian grids and 64x4x4 on each FCC sub-grid.  Shapes to set are
+ * those two, or powers of two with x a multiple of 64, y*z <= 32 rows and 256 to
+ * 4096 voxels; Cartesian shapes need z a multiple of 4.  The shape changes speed
+ * only, never output.  vox_get_brick_dims returns the set shape (32x8x16 before
+ * one is set). */
 vox_status vox_set_brick_dims(vox_ctx *ctx, int fcc, const uint32_t dims[3]);
 vox_status vox_get_brick_dims(const vox_ctx *ctx, int fcc, uint32_t dims[3]);
 /* Times vox_voxelize_nodes (with materials) for this grid and node kind

@@ -45,3 +45,27 @@ def test_soups_match_oracle(gpu_ctx, oracle, n, empty, dim, kind):
     print(f"soup {n} empty {empty} dim {dim} kind {kind}", flush=True)
     got = gpu_ctx.voxelize_nodes(g, kind, True)
     assert np.array_equal(got, oracle.voxelize_nodes(m, og, kind, True))
+
+
+@pytest.mark.parametrize("ext", [(60, 60, 4), (60, 60, 5), (60, 60, 6), (29, 125, 13), (29, 126, 14),
+                                 (500, 3, 40), (3, 300, 3), (200, 140, 90)])
+@pytest.mark.parametrize("kind", [va.NODE_SHORT, va.NODE_SHORT_FCC, va.NODE_PARTIAL])
+def test_brick_choice_matches_oracle(gpu_ctx_auto, oracle, ext, kind):
+    """Grids on either side of the rules that pick the brick (8 planes, padding)."""
+    m = soup(300, 20, seed=sum(ext))
+    m.vertices = (m.vertices * np.array(ext)).astype(np.float32)
+    gpu_ctx_auto.set_mesh(m.vertices, m.indices)
+    gpu_ctx_auto.set_materials(m.materials, 8)
+    g = gpu_ctx_auto.plan_grid(va.PLAN_CUBE_LENGTH, 1.0)
+    og = oracle.plan_grid(m.vertices, va.PLAN_CUBE_LENGTH, 1.0)
+    assert g.same(og)
+    print(f"brick {ext} kind {kind}", flush=True)
+    ref = oracle.voxelize_nodes(m, og, kind, True)
+    assert np.array_equal(gpu_ctx_auto.voxelize_nodes(g, kind, True), ref)
+
+
+@pytest.fixture(scope="module")
+def gpu_ctx_auto():
+    ctx = va.Context(0)
+    yield ctx
+    ctx.close()

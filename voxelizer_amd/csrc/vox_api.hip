@@ -145,8 +145,11 @@ struct vox_ctx {
     void *up = nullptr;
     size_t up_cap = 0;
     bool up_busy = false;
-    // surface brick shapes (voxels along x, y, z)
-    int cart_bdim[3] = {kCartBX, kCartBY, kCartBZ};
+    // surface brick shapes (voxels along x, y, z) of Cartesian grids and of FCC
+    // sub-grids; with *_auto the grid decides (brick_shape)
+    int cart_bdim[3] = {kBrick[0], kBrick[1], kBrick[2]};
+    int fcc_bdim[3] = {kBrick[0], kBrick[1], kBrick[2]};
+    bool cart_auto = true, fcc_auto = true;
     // meshes with fewer triangles carry materials in the surface pass's
     // winner keys (at most 2^22; VOX_EMBED_TRIS lowers it, for tests of the
     // other path)
@@ -161,7 +164,6 @@ struct vox_ctx {
     uint32_t *ovf = nullptr;
     const uint32_t *last_changed = nullptr;
     uint32_t last_solid = 0, last_surf = 0, last_passes = 0;
-    int fcc_bdim[3] = {kFccBX, kFccBY, kFccBZ};
     // No-allocation mode (vox_voxelize_nodes_noalloc): buffers are carved
     // from this device's scratch array (scratch_dev, set up by vox_create)
     // instead of hipMalloc.
@@ -382,9 +384,34 @@ bool brick_ok(const uint32_t b[3], bool cart) {
     // The brick pass's epilogue gives each wave whole layers: a layer of at
     // most 256 voxels tiles its 256-voxel steps; a larger one needs bricks at
     // least 4 deep (each wave then takes a multiple of a layer's steps).
+    for (const int *d : {kBrick, kFlatBrick})
+        if (b[0] == (uint32_t)d[0] && b[1] == (uint32_t)d[1] && b[2] == (uint32_t)d[2]) return true;
     return b[0] >= 64 && b[1] * b[2] <= 32 && (b[0] / 32) * b[1] <= 32 &&
            (b[0] * b[1] <= 256 || b[2] >= 4) && nvox >= 256 && nvox <= (uint32_t)kMaxBrickVox &&
            (!cart || b[2] % kNodeZ == 0);
+}
+
+// The brick shape for a grid of the given alloc dims: the context's, or by the
+// grid (kBrick).  A no-allocation call takes the narrow shapes only where they
+// need no more scratch than the wide one.
+void brick_shape(const vox_ctx *ctx, bool fcc, const uint32_t alloc[3], int out[3]) {
+    const int *pick = fcc ? ctx->fcc_bdim : ctx->cart_bdim;
+    if (fcc ? ctx->fcc_auto : ctx->cart_auto) {
+        const int *wide = fcc ? kWideFcc : kWideCart;
+        pick = alloc[2] <= 8u ? kFlatBrick : kBrick;
+        auto bricks = [&](const int *b) {
+            uint64_t n = 1;
+            for (int a = 0; a < 3; a++) n *= (alloc[a] + (uint32_t)b[a] - 1u) / (uint32_t)b[a];
+            return n;
+        };
+        auto voxels = [](const int *b) { return (uint64_t)b[0] * b[1] * b[2]; };
+        const uint64_t n = bricks(pick), nw = bricks(wide);
+        const uint64_t v = n * voxels(pick), vw = nw * voxels(wide);
+        // A triangle's box of bricks has 16 bits per axis.
+        if (alloc[0] > 0xFFFFu * 32u || (ctx->arena ? v > vw || n > nw : v > vw + vw / 8u))
+            pick = wide;
+    }
+    for (int a = 0; a < 3; a++) out[a] = pick[a];
 }
 
 // ---------------------------------------------------------------------------
@@ -501,7 +528,7 @@ inline bool job_needs_surf(const Job &J) { return J.pnodes != nullptr; }
 // Cartesian).  cart: the job gets erosion and Cartesian node blocks.
 vox_status add_job(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, uint32_t nt,
                    const uint8_t *mats, const vox_grid &g, const Layout &L, const double shift[3],
-                   bool use_mats, const uint32_t ms[3], const int bdim[3], bool cart, void *nodes,
+                   bool use_mats, const uint32_t ms[3], bool fcc, bool cart, void *nodes,
                    int kind, uint32_t *ext_bits) {
     const uint32_t X = g.alloc[0], W = X / 32;
     if (W == 0) return fail(ctx, VOX_ERR_UNSUPPORTED, "empty x resolution");
@@ -511,6 +538,8 @@ vox_status add_job(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, uin
                     "word bitmask is undefined");
     if ((uint64_t)P.tri_b.back() + nt + 256 >= (1ull << 30))
         return fail(ctx, VOX_ERR_UNSUPPORTED, "more than 2^30 triangles in one call");
+    int bdim[3];
+    brick_shape(ctx, fcc, L.alloc, bdim);
     Job J;
     std::memset(&J, 0, sizeof(J));
     J.V = V;
@@ -610,7 +639,7 @@ vox_status add_mesh(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, ui
     const double zero[3] = {0.0, 0.0, 0.0};
     if (kind == VOX_NODE_SHORT || kind == VOX_NODE_LONG || kind == VOX_NODE_PARTIAL)
         return add_job(ctx, P, V, I, nt, mats, g, whole_layout(g), zero, use_mats, ms,
-                       ctx->cart_bdim, true, nodes, (int)kind, nullptr);
+                       false, true, nodes, (int)kind, nullptr);
     // fccWorker (src/host_side.cpp:1262-1698): four sub-grids shifted by
     // (0,0,0), (h,h,0), (0,h,h), (h,0,h), h = d/2 (1436-1463).
     const double h = g.voxel_length / 2.0;
@@ -618,7 +647,7 @@ vox_status add_mesh(vox_ctx *ctx, Plan &P, const float *V, const uint32_t *I, ui
     const uint32_t first = (uint32_t)P.jobs.size();
     for (int k = 0; k < 4; k++)
         VOX_TRY(add_job(ctx, P, V, I, nt, mats, g, whole_layout(g), shifts[k], use_mats, ms,
-                        ctx->fcc_bdim, false,
+                        true, false,
                         k == 0 ? nodes : nullptr, kind == VOX_NODE_SHORT_FCC ? 3 : 4, nullptr));
     P.fcc_first.push_back(first);
     P.fcc_b.push_back(P.fcc_b.back() + fcc_node_blocks(P.jobs[first].gd));
@@ -1619,7 +1648,7 @@ vox_status vox_solid_bits(vox_ctx *ctx, const vox_grid *g, const double shift[3]
     Plan P;
     VOX_TRY(add_job(ctx, P, ctx->V, ctx->I, ctx->nt, nullptr, *g, whole_layout(*g),
                     shift ? shift : zero, false, ms,
-                    ctx->cart_bdim, false, nullptr, 0, bits_dev));
+                    false, false, nullptr, 0, bits_dev));
     PlanDev D;
     record(ctx, 0);
     VOX_TRY(plan_upload(ctx, P, D, sy, sz));
@@ -1746,7 +1775,7 @@ vox_status vox_voxelize_partition(vox_ctx *ctx, const vox_grid *g, vox_node_kind
     const double zero[3] = {0.0, 0.0, 0.0};
     Plan P;
     VOX_TRY(add_job(ctx, P, ctx->V, ctx->I, ctx->nt, ctx->mats, *g, part_layout(*g, part_min, part_max),
-                    zero, use_materials != 0, ms, ctx->cart_bdim, true, nodes_dev,
+                    zero, use_materials != 0, ms, false, true, nodes_dev,
                     (int)kind, nullptr));
     VOX_TRY(run_plan(ctx, P, vs[1], vs[2]));
     return finish_times(ctx);
@@ -1768,7 +1797,7 @@ vox_status vox_solid_bits_partition(vox_ctx *ctx, const vox_grid *g, const uint3
     const uint32_t ms[3] = {512u, 512u, 512u};
     Plan P;
     VOX_TRY(add_job(ctx, P, ctx->V, ctx->I, ctx->nt, nullptr, *g,
-                    part_layout(*g, part_min, part_max), zero, false, ms, ctx->cart_bdim, false,
+                    part_layout(*g, part_min, part_max), zero, false, ms, false, false,
                     nullptr, 0, bits_dev));
     PlanDev D;
     record(ctx, 0);
@@ -1858,7 +1887,7 @@ vox_status vox_voxelize_slice(vox_ctx *ctx, vox_plan_mode mode, double param, vo
         uint8_t *rot;
         VOX_TRY(buf(ctx, "slice_rot_nodes", bytes, &rot));
         VOX_TRY(add_job(ctx, P, V, ctx->I, ctx->nt, ctx->mats, g, L, zero, use_materials != 0, ms,
-                        ctx->cart_bdim, true, rot, (int)kind, nullptr));
+                        false, true, rot, (int)kind, nullptr));
         // one erosion subspace across the rotated rows: vy >= X > the 3 rows
         VOX_TRY(run_plan(ctx, P, vy, vy));
         k_unrotate_nodes<<<grid_for(bytes / size, 256, 4096), 256, 0, ctx->stream>>>(
@@ -1866,7 +1895,7 @@ vox_status vox_voxelize_slice(vox_ctx *ctx, vox_plan_mode mode, double param, vo
         VOX_HIP(hipGetLastError());
     } else {
         VOX_TRY(add_job(ctx, P, V, ctx->I, ctx->nt, ctx->mats, g, L, zero, use_materials != 0, ms,
-                        ctx->cart_bdim, true, nodes_dev, (int)kind, nullptr));
+                        false, true, nodes_dev, (int)kind, nullptr));
         VOX_TRY(run_plan(ctx, P, vy, vy));
     }
     return finish_times(ctx);
@@ -1891,6 +1920,7 @@ vox_status vox_set_brick_dims(vox_ctx *ctx, int fcc, const uint32_t dims[3]) {
         return ctx ? fail(ctx, VOX_ERR_INVALID, "unsupported brick shape") : VOX_ERR_INVALID;
     int *d = fcc ? ctx->fcc_bdim : ctx->cart_bdim;
     for (int a = 0; a < 3; a++) d[a] = (int)dims[a];
+    (fcc ? ctx->fcc_auto : ctx->cart_auto) = false;
     return VOX_OK;
 }
 
@@ -1907,9 +1937,9 @@ vox_status vox_autotune_bricks(vox_ctx *ctx, const vox_grid *grid, vox_node_kind
                                float *best_ms) {
     if (!ctx || !grid || !nodes_dev || reps == 0) return VOX_ERR_INVALID;
     const bool fcc = kind == VOX_NODE_SHORT_FCC || kind == VOX_NODE_LONG_FCC;
-    static const uint32_t cart[][3] = {{128, 4, 8}, {64, 4, 8}, {128, 2, 8}, {128, 4, 4},
+    static const uint32_t cart[][3] = {{32, 8, 16}, {32, 16, 8}, {128, 4, 8}, {64, 4, 8}, {128, 2, 8}, {128, 4, 4},
                                        {256, 4, 4}, {256, 2, 8}, {64, 4, 4}, {128, 8, 4}};
-    static const uint32_t fccs[][3] = {{64, 4, 4}, {64, 4, 8}, {128, 4, 4}, {64, 8, 4},
+    static const uint32_t fccs[][3] = {{32, 8, 16}, {32, 16, 8}, {64, 4, 4}, {64, 4, 8}, {128, 4, 4}, {64, 8, 4},
                                        {128, 2, 4}, {64, 2, 8}};
     const uint32_t(*cand)[3] = fcc ? fccs : cart;
     const size_t ncand = fcc ? sizeof(fccs) / sizeof(fccs[0]) : sizeof(cart) / sizeof(cart[0]);
@@ -2034,6 +2064,8 @@ vox_status vox_voxelize_batch(vox_ctx *ctx, vox_batch_item *items, uint32_t n,
             w->cart_bdim[a] = ctx->cart_bdim[a];
             w->fcc_bdim[a] = ctx->fcc_bdim[a];
         }
+        w->cart_auto = ctx->cart_auto;
+        w->fcc_auto = ctx->fcc_auto;
         if (!params.empty()) VOX_TRY(vox_cost_set_params(w, params.data()));
     }
     // Longest estimated work first.
@@ -2189,6 +2221,8 @@ vox_status vox_graph_create(vox_ctx *ctx, const vox_batch_item *items, uint32_t 
         w->cart_bdim[a] = ctx->cart_bdim[a];
         w->fcc_bdim[a] = ctx->fcc_bdim[a];
     }
+    w->cart_auto = ctx->cart_auto;
+    w->fcc_auto = ctx->fcc_auto;
     if (ctx->cost_ready) {
         std::vector<float> params(kCostParams);
         st = vox_cost_get_params(ctx, params.data());

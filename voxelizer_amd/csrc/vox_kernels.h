@@ -57,12 +57,20 @@ __host__ __device__ __forceinline__ uint32_t plane_chunks(uint32_t W, uint32_t Y
     return (W * Y + kChunk - 1u) / kChunk;
 }
 
-// Surface bricks: default shapes of the Cartesian grid and of each FCC
-// sub-grid; the shape is a run-time choice (the autotuner picks among
-// power-of-two shapes with x a multiple of 64, at most 32 rows and 256 to
-// kMaxBrickVox voxels).
-constexpr int kCartBX = 128, kCartBY = 4, kCartBZ = 8;
-constexpr int kFccBX = 64, kFccBY = 4, kFccBZ = 4;
+// Surface bricks.  A (triangle, brick) pair costs a triangle setup, so bricks
+// are near cubes: one word (32 voxels) wide, 8 rows, 16 planes, or 16 rows and 8
+// planes for grids of at most 8 planes (a slice has three).  The wide shapes are
+// those in use before, taken where the others' padding would make the material
+// grid larger by more than an eighth (brick_shape).  Calls with (128, 4, 8), or on
+// FCC sub-grids (64, 4, 4), against this: room 512x403x303 368 -> 337 us, 132
+// large triangles over 672x515x387 343 -> 294 us, 64-mesh batch 3012 -> 2453 us,
+// hall 1531 -> 1475 us, x slice of the room 300 -> 275 us, LongFCC room
+// 640x255x384 547 -> 412 us; in between lie (64, 8, 8) 349, 310, 2607, 1503, 291
+// and 420 us; (32, 16, 8) takes 1561 us on the hall.
+// The shape is a run-time choice (the autotuner picks among powers of two with
+// 256 to kMaxBrickVox voxels).
+constexpr int kBrick[3] = {32, 8, 16}, kFlatBrick[3] = {32, 16, 8};
+constexpr int kWideCart[3] = {128, 4, 8}, kWideFcc[3] = {64, 4, 4};
 constexpr int kMaxBrickVox = 4096;
 // Brick pass: waves that voxelize, and one that prepares their next triangles.
 constexpr uint32_t kBrickWaves = 3, kBrickThreads = (kBrickWaves + 1) * kWave;
@@ -82,10 +90,11 @@ struct GridDims {
 // z planes per thread in the erosion pass (a block covers kChunk words of a
 // plane x kErodeZ planes).
 constexpr uint32_t kErodeZ = 8;
-// z planes per thread in the Cartesian node pass; divides kCartBZ so a
-// thread's planes share one surface brick.
+// z planes per thread in the Cartesian node pass; divides the depth of every
+// Cartesian brick so a thread's planes share one.
 constexpr uint32_t kNodeZ = 4;
-static_assert(kCartBZ % kNodeZ == 0, "node planes must not straddle a brick");  // z >= 4
+static_assert(kBrick[2] % kNodeZ == 0 && kFlatBrick[2] % kNodeZ == 0 && kWideCart[2] % kNodeZ == 0,
+              "node planes must not straddle a brick");
 // Cost model: features per brick, MLP parameters (16-64-64-1).
 constexpr int kCostFeatures = 16;
 constexpr int kCostParams = 64 * 16 + 64 + 64 * 64 + 64 + 64 + 1;  // 5313

@@ -908,10 +908,10 @@ __device__ __forceinline__ uint32_t surf_tri_setup(const SurfParams &p, bool fdi
 }
 
 __device__ __forceinline__ void key_write(uint32_t *keys, uint8_t *touched, uint32_t idx,
-                                          uint32_t nvox, uint32_t row_shift, uint32_t key) {
+                                          uint32_t nvox, uint32_t key) {
     if (idx >= nvox) return;  // unreachable: items lie in the brick
     atomicMax(&keys[idx], key);
-    touched[idx >> row_shift] = 1;
+    touched[idx >> 8] = 1;
 }
 
 // The dominant-plane half of work item k (a 1D triangle's voxel, or a column
@@ -920,11 +920,11 @@ __device__ __forceinline__ void key_write(uint32_t *keys, uint8_t *touched, uint
 // triangle's column that passes, whose depth part follows (surf_depth).
 __device__ __forceinline__ bool surf_column(const SurfParams &p, const SurfTri &st, uint32_t k,
                                             uint32_t *keys, uint8_t *touched, uint32_t nvox,
-                                            uint32_t row_shift, uint32_t &cu, uint32_t &cv) {
+                                            uint32_t &cu, uint32_t &cv) {
     const uint32_t pk = st.pk, base = pk & 0xFFFu;
     const uint32_t bb = (pk >> kPkClass) & 3u, a = (pk >> kPkAxis) & 3u;
     if (bb == BB_1D) {
-        key_write(keys, touched, base + (k << ((pk >> kPkA) & 15u)), nvox, row_shift, st.key);
+        key_write(keys, touched, base + (k << ((pk >> kPkA) & 15u)), nvox, st.key);
         return false;
     }
     // k = cv * wu + cu
@@ -944,7 +944,7 @@ __device__ __forceinline__ bool surf_column(const SurfParams &p, const SurfTri &
     if (in && bb != BB_3D)
         key_write(keys, touched,
                   base + (cu << ((pk >> kPkU) & 15u)) + (cv << ((pk >> kPkV) & 15u)), nvox,
-                  row_shift, st.key);
+                  st.key);
     return in && bb == BB_3D;
 }
 
@@ -960,8 +960,7 @@ __device__ __forceinline__ bool surf_column(const SurfParams &p, const SurfTri &
 // the interval along a that the voxel falls in.
 __device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable &spl,
                                            const SurfTri &st, uint32_t cu, uint32_t cv,
-                                           uint32_t *keys, uint8_t *touched, uint32_t nvox,
-                                           uint32_t row_shift) {
+                                           uint32_t *keys, uint8_t *touched, uint32_t nvox) {
     const uint32_t pk = st.pk, a = (pk >> kPkAxis) & 3u, sa = (pk >> kPkA) & 15u;
     const float mu = a == AX_X ? p.m.y : p.m.x, mv = a == AX_Z ? p.m.y : p.m.z;
     const float ma = a == AX_X ? p.m.x : a == AX_Y ? p.m.y : p.m.z;
@@ -1021,7 +1020,7 @@ __device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable
     if (!(pk & kManySplits)) {
         const bool single = max(lo, st.va) == min(hi, st.vb);
         for (int32_t i = ilo; i <= ihi; i++) {
-            if (single || inside()) key_write(keys, touched, idx, nvox, row_shift, key);
+            if (single || inside()) key_write(keys, touched, idx, nvox, key);
             fa += 1.0f;
             idx += 1u << sa;
         }
@@ -1033,7 +1032,7 @@ __device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable
         while (si + 1u < ns && (uint32_t)i >= spl.hi[a][si]) si++;
         const int32_t rl = max(lo, max(st.va, (int32_t)spl.lo[a][si]));
         const int32_t rh = min(hi, min(st.vb, (int32_t)spl.hi[a][si] - 1));
-        if (rl == rh || inside()) key_write(keys, touched, idx, nvox, row_shift, key);
+        if (rl == rh || inside()) key_write(keys, touched, idx, nvox, key);
         fa += 1.0f;
         idx += 1u << sa;
     }
@@ -1050,8 +1049,8 @@ __device__ __forceinline__ void surf_depth(const SurfParams &p, const SplitTable
 // waves' way: they work from LDS and only store.
 //
 // All (triangle, column) items of the chunk are spread over the voxelizing
-// threads; winners accumulate in LDS (ds_max of winner_key).  Rows that
-// received a key are visited when the brick's last chunk is done: each lane
+// threads; winners accumulate in LDS (ds_max of winner_key).  The 256-voxel steps
+// that received a key are visited when the brick's last chunk is done: each lane
 // takes four voxels, a word's eight lanes OR their bits into the solid grid,
 // and the words that hold a surface voxel have their winners' materials
 // stored in the brick's block of the material grid.  With `stats`, surface
@@ -1094,13 +1093,14 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
     __shared__ uint32_t cstart[kSurfChunk], smask[kBrickWaves][2];
     __shared__ uint8_t cslot[kSurfChunk];
     __shared__ uint32_t wqueue[kBrickWaves][2 * kWave];  // columns that await their depth part
-    __shared__ uint8_t touched[2][32];  // rows with a key, of this brick and (cleared) the next
+    // 256-voxel steps with a key, of this brick and (cleared) the next
+    __shared__ uint8_t touched[2][kMaxBrickVox / 256];
     __shared__ BrickStep step;
     __shared__ SplitTable spl;
     const uint32_t tid = threadIdx.x, lane = lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     for (uint32_t i = tid; i < (uint32_t)kMaxBrickVox; i += kBrickThreads) keys[i] = 0u;
-    if (tid < 64u) (&touched[0][0])[tid] = 0;
+    if (tid < sizeof(touched)) (&touched[0][0])[tid] = 0;
     if (tid < 2u * kBrickWaves) (&smask[0][0])[tid] = 0u;
 
     if (wave == kBrickWaves) {
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
         const uint32_t row_shift = 31u - (uint32_t)__clz(p.bdim[0]);
         if (ends & 1u) {
             par ^= 1u;
-            if (tid < 32u) touched[par ^ 1u][tid] = 0;  // the previous brick's
+            if (tid < sizeof(touched[0])) touched[par ^ 1u][tid] = 0;  // the previous brick's
             if (cycles && tid == 0u) t_start = __builtin_amdgcn_s_memtime();
         }
         // Lane j holds the first item of the j-th triangle with items
@@ -1295,11 +1295,11 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
         const uint32_t cs = lane < ntri ? cstart[lane] : UINT32_MAX;
         const uint32_t sl = lane < ntri ? (uint32_t)cslot[lane] : 0u;
         uint32_t *sm = &smask[wave][0], *wq = wqueue[wave];
-        uint8_t *rows = touched[par];
+        uint8_t *steps = touched[par];
         uint32_t nq = 0u;  // columns in the wave's queue (uniform)
         auto depth = [&](uint32_t e) {
-            surf_depth(p, spl, tris[e >> 24], e & 0xFFFu, (e >> 12) & 0xFFFu, keys, rows, nvox,
-                       row_shift);
+            surf_depth(p, spl, tris[e >> 24], e & 0xFFFu, (e >> 12) & 0xFFFu, keys, steps,
+                       nvox);
         };
         for (uint32_t w0 = wave * kWave; w0 < total; w0 += kBrickWaves * kWave) {  // uniform
             const uint32_t t0 = (uint32_t)__popcll(__ballot(cs <= w0)) - 1u;
@@ -1316,8 +1316,8 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
             const uint32_t start = (uint32_t)__shfl((int)cs, (int)ti);
             const uint32_t c = w0 + lane;
             uint32_t cu = 0u, cv = 0u;
-            const bool deep = c < total && surf_column(p, tris[slot], c - start, keys, rows, nvox,
-                                                       row_shift, cu, cv);
+            const bool deep = c < total && surf_column(p, tris[slot], c - start, keys, steps,
+                                                       nvox, cu, cv);
             const unsigned long long dm = __ballot(deep);
             if (deep)
                 wq[nq + __builtin_amdgcn_mbcnt_hi(
@@ -1340,8 +1340,8 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
         // lanes of a 32-voxel word OR their nibbles together, and each lane
         // of a word holding a surface voxel writes its 4 material bytes as
         // one dword of the brick's block in the material grid (the winner's
-        // material, 0 for the word's other voxels).  Steps whose rows
-        // received no key are passed over.  Keys are cleared for the next
+        // material, 0 for the word's other voxels).  Steps that received no
+        // key are passed over.  Keys are cleared for the next
         // brick.  With materials in the keys the loop issues no global loads,
         // so its stores never wait (a wait for a load also waits for earlier
         // stores here).
@@ -1359,11 +1359,10 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
         const uint32_t W = p.alloc[0] / 32u;
         const bool whole = z0 == 0u && z1 == (uint32_t)p.bdim[2];
         VK_G uint8_t *wm = (VK_G uint8_t *)gptr(J.wmask) + (size_t)b * 16u;
-        const uint32_t tmask = (uint32_t)__ballot(lane < 32u && rows[lane & 31u] != 0);
-        const uint32_t rows_per_step = 256u >> row_shift;  // bd0 >= 64: 1, 2 or 4 rows
+        constexpr uint32_t kSteps = kMaxBrickVox / 256;
+        const uint32_t tmask =
+            (uint32_t)__ballot(lane < kSteps && steps[lane & (kSteps - 1u)] != 0);
         for (uint32_t v0 = wave * 256u; v0 < nvox; v0 += kBrickWaves * 256u) {
-            const uint32_t rmask = (rows_per_step > 1u ? (1u << rows_per_step) - 1u : 1u)
-                                   << (v0 >> row_shift);
             // This lane's word and its place in the grid.
             const uint32_t wi = (v0 >> 5) + (lane >> 3);
             const uint32_t aw = aw0 + (wi & ((1u << lwx) - 1u)),
@@ -1371,7 +1370,7 @@ __global__ __launch_bounds__(kBrickThreads, 5) void k_surf_brick(
                            lz = wi >> (lwx + lby), az = az0 + lz;
             const size_t gi = ((size_t)az * p.alloc[1] + ay) * W + aw;
             uint32_t w = 0u;
-            if (tmask & rmask) {  // uniform
+            if ((tmask >> (v0 >> 8)) & 1u) {  // uniform
                 uint4 *kp = (uint4 *)&keys[v0 + 4u * lane];
                 const uint4 kv = *kp;
                 const uint32_t nib = (kv.x ? 8u : 0u) | (kv.y ? 4u : 0u) | (kv.z ? 2u : 0u) |

@@ -508,6 +508,15 @@ template __global__ void k_pairs_place<false>(const Job *, const uint32_t *, uin
 template __global__ void k_pairs_place<true>(const Job *, const uint32_t *, uint32_t, SolidPairs,
                                              SurfPairs, uint32_t);
 
+// Bit i: parity of the bits above and at i (MSB first: x%32 == 0 is bit 31).
+__device__ __forceinline__ uint32_t prefix_xor(uint32_t c) {
+    c ^= c >> 1;
+    c ^= c >> 2;
+    c ^= c >> 4;
+    c ^= c >> 8;
+    return c ^ (c >> 16);
+}
+
 // Zeroes kPadBlock words of the pad rows (y or z at the alloc border).
 __device__ __forceinline__ void zero_pad_rows(const Job *__restrict__ jobs,
                                               const uint32_t *__restrict__ pad_bases,
@@ -540,6 +549,15 @@ __device__ __forceinline__ void zero_pad_rows(const Job *__restrict__ jobs,
 // (the suffix flips of src/voxelizer.cu:1487-1616) and each bit word is
 // written to HBM once, coalesced, with no global atomics.  The workgroups past
 // the tiles clear the pad rows.
+//
+// Bound by FP64 and integer instructions.  A triangle's lanes test centres, and
+// the few that pass (their two divisions cost as much as the tests of four
+// centres) are queued in LDS and worked off by full waves; the rows' words are
+// taken 64 at a time whatever the row width.  With the divisions in line and a
+// step per row: hall (1536x1024x768) 145 -> 111 us, hall at 1100 98 -> 73 us,
+// 64-mesh batch 400 -> 210 us (225 with divisions in line), room 512x403x303
+// 33 -> 21 us, LongFCC room 640x255x384 55 -> 33 us, 132 large triangles over
+// 672x515x387 26 -> 19 us.
 __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jobs,
                                                       const uint32_t *__restrict__ tile_bases,
                                                       const uint32_t *__restrict__ pad_bases,
@@ -550,6 +568,8 @@ __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jo
                                                       const uint32_t *__restrict__ list,
                                                       const uint16_t *__restrict__ list_mask) {
     extern __shared__ __align__(16) uint32_t cross[];  // [16][SW]
+    __shared__ double tri[6][kWave];     // per lane: its triangle for fill_crossing
+    __shared__ uint16_t queue[2 * kWave];  // centres that await their crossing: lane, row
     const uint32_t n_tiles = tile_bases[njobs];
     if (blockIdx.x >= n_tiles) {
         zero_pad_rows(jobs, pad_bases, njobs, blockIdx.x - n_tiles);
@@ -578,51 +598,112 @@ __global__ __launch_bounds__(kWave) void k_solid_fill(const Job *__restrict__ jo
     while (lg < 4u && cnt <= (kWave >> (lg + 1u))) lg++;
     const uint32_t items = cnt << lg, rows = 16u >> lg;
     const uint32_t lane = tid;
+    // Rows that hold voxel centres (bit r; the last tiles reach past the grid).
+    const uint32_t ny = min(p.smax[0] - ty * 4u, 4u), nz = min(p.smax[1] - tz * 4u, 4u);
+    const uint32_t inside = ((1u << ny) - 1u) * (0x1111u & ((1u << (4u * nz)) - 1u));
+    const float rW = 1.0f / (float)W;
     uint32_t carries = 0u;  // bit r: crossing parity of row r before the segment
     for (uint32_t s0 = 0; s0 < W; s0 += SW) {
         const uint32_t sw = min(SW, W - s0);
         uint4 *cross4 = reinterpret_cast<uint4 *>(cross);  // 16 * SW words: 4 * SW uint4
         for (uint32_t i = tid; i < 4u * SW; i += kWave) cross4[i] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
-        for (uint32_t i = tid; i < items; i += kWave) {
-            const uint32_t t = list[off + (i >> lg)];
-            // Rows whose subspace queued the triangle (all rows with one subspace).
-            const uint32_t rmask = list_mask ? (uint32_t)list_mask[off + (i >> lg)] : 0xFFFFu;
+        auto cross_at = [&](uint32_t e) {  // a queued centre's crossing
+            const uint32_t k = e >> 4, r = e & 15u;
+            const uint32_t cy = ty * 4u + (r & 3u), cz = tz * 4u + (r >> 2);
+            const uint32_t vx = fill_crossing({tri[0][k], tri[1][k], tri[2][k]}, tri[3][k],
+                                              tri[4][k], tri[5][k], double(cy) * p.d + p.emy,
+                                              double(cz) * p.d + p.emz, p.d);
+            const uint32_t wx = (vx >> 5) - s0;  // wraps for words before s0
+            if (vx < p.X && wx < sw) atomicXor(&cross[r * SW + wx], 1u << (31u - (vx & 31u)));
+        };
+        for (uint32_t i0 = 0; i0 < items; i0 += kWave) {  // uniform
+            const uint32_t i = i0 + lane, at = off + (i >> lg);
             const uint32_t r0 = (i & ((1u << lg) - 1u)) * rows;
-            D3 v[3];
-            load_tri_d(p, t, v);
+            uint32_t rmask = 0u;  // rows to test
             FillSetup fs;
-            fill_setup(v, fs);
-            for (uint32_t r = r0; r < r0 + rows; r++) {
+            if (i < items) {
+                // Rows whose subspace queued the triangle (all with one subspace).
+                rmask = inside & (list_mask ? (uint32_t)list_mask[at] : ~0u);
+                D3 v[3];
+                load_tri_d(p, list[at], v);
+                fill_setup(v, fs);
+                tri[0][lane] = fs.n.x;
+                tri[1][lane] = fs.n.y;
+                tri[2][lane] = fs.n.z;
+                tri[3][lane] = (v[0].x - p.emx) * fs.n.x;
+                tri[4][lane] = v[0].y;
+                tri[5][lane] = v[0].z;
+            }
+            uint32_t nq = 0u;  // queued centres (uniform)
+            for (uint32_t r = r0; r < r0 + rows; r++) {  // `rows` is uniform
                 const uint32_t cy = ty * 4u + (r & 3u), cz = tz * 4u + (r >> 2);
-                if (cy < p.smin[0] || cy >= p.smax[0] || cz < p.smin[1] || cz >= p.smax[1]) continue;
-                if (!((rmask >> r) & 1u)) continue;
-                uint32_t vx;
-                if (fill_center(fs, p.emx, p.emy, p.emz, p.d, cy, cz, vx) && vx < p.X) {
-                    const uint32_t wx = (vx >> 5) - s0;  // wraps for words before s0
-                    if (wx < sw) atomicXor(&cross[r * SW + wx], 1u << (31u - (vx & 31u)));
+                const bool in = ((rmask >> r) & 1u) &&
+                                fill_inside(fs, double(cy) * p.d + p.emy, double(cz) * p.d + p.emz);
+                const unsigned long long m = __ballot(in);
+                if (in)
+                    queue[nq + __builtin_amdgcn_mbcnt_hi(
+                                   (uint32_t)(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                        (uint16_t)(lane << 4 | r);
+                nq += (uint32_t)__popcll(m);
+                wave_lds_sync();
+                if (nq >= (uint32_t)kWave) {
+                    nq -= (uint32_t)kWave;
+                    cross_at(queue[nq + lane]);
+                    wave_lds_sync();
                 }
             }
+            if (lane < nq) cross_at(queue[lane]);
+            wave_lds_sync();
         }
         __syncthreads();
         // Crossing parity -> solid bits (MSB-first bits: x%32 == 0 is bit
         // 31): a prefix XOR inside each word, and across words the parity of
         // the crossings before it (one ballot per 64 words), written
         // straight out.
+        if (SW == W) {
+            // The 16 rows lie one after another in LDS, so 64 consecutive
+            // words are taken at a time whatever the rows' width (a step per
+            // row left most lanes idle on narrow grids): below counts the odd
+            // words before the lane in its own row, and a row that began
+            // before the step carries the parity of its words there.
+            uint32_t carry = 0u;
+            for (uint32_t i0 = 0; i0 < 16u * W; i0 += kWave) {
+                const uint32_t i = i0 + lane;
+                uint32_t r = (uint32_t)((float)i * rW);  // i / W: within one
+                int32_t w = (int32_t)(i - r * W);
+                if (w < 0) { r--; w += (int32_t)W; }
+                if (w >= (int32_t)W) { r++; w -= (int32_t)W; }
+                const bool valid = r < 16u && ((inside >> r) & 1u);
+                const uint32_t c = i < 16u * W ? cross[i] : 0u;
+                const uint32_t sx = prefix_xor(c);
+                const unsigned long long odd = __ballot((__popc(c) & 1) != 0);
+                // Odd words of the lane's row in this step, before it.
+                const uint32_t from = (uint32_t)w < lane ? lane - (uint32_t)w : 0u;
+                const unsigned long long mine = odd & ((1ull << lane) - 1ull) & (~0ull << from);
+                const uint32_t before =
+                    ((uint32_t)__popcll(mine) ^ ((uint32_t)w > lane ? carry : 0u)) & 1u;
+                if (valid) {
+                    const uint32_t cy = ty * 4u + (r & 3u), cz = tz * 4u + (r >> 2);
+                    const size_t row = (size_t)(cz + p.oz) * p.rowsY + (cy + p.oy);
+                    bits[row * W + (uint32_t)w] = sx ^ (before ? 0xFFFFFFFFu : 0u);
+                }
+                // The last lane's row goes on in the next step (or ends here).
+                const uint32_t end = before ^ ((uint32_t)__popc(c) & 1u);
+                carry = (uint32_t)__builtin_amdgcn_readlane((int)end, kWave - 1);
+            }
+            return;
+        }
         for (uint32_t r = 0; r < 16u; r++) {
+            if (!((inside >> r) & 1u)) continue;
             const uint32_t cy = ty * 4u + (r & 3u), cz = tz * 4u + (r >> 2);
-            if (cy < p.smin[0] || cy >= p.smax[0] || cz < p.smin[1] || cz >= p.smax[1]) continue;
             const size_t rowIdx = (size_t)(cz + p.oz) * p.rowsY + (cy + p.oy);
             uint32_t carry = (carries >> r) & 1u;
             for (uint32_t w0 = 0; w0 < sw; w0 += kWave) {
                 const uint32_t w = w0 + lane;
                 const uint32_t c = w < sw ? cross[r * SW + w] : 0u;
-                uint32_t sx = c;
-                sx ^= sx >> 1;
-                sx ^= sx >> 2;
-                sx ^= sx >> 4;
-                sx ^= sx >> 8;
-                sx ^= sx >> 16;
+                const uint32_t sx = prefix_xor(c);
                 const unsigned long long odd = __ballot((__popc(c) & 1) != 0);
                 // Odd-crossing words below this lane, counted by mbcnt.
                 const uint32_t below = __builtin_amdgcn_mbcnt_hi(

@@ -151,14 +151,15 @@ __device__ __forceinline__ bool tile_hit(const TileSetup &ts, uint32_t ty, uint3
     return hit;
 }
 
-// Per-triangle data of the centre test (src/voxelizer.cu:1334-1372).
+// Per-triangle data of the centre test (src/voxelizer.cu:1334-1372).  th: the
+// DBL_MIN top-left tie break; r + DBL_MIN > 0 exactly where r > -DBL_MIN (the
+// sign of a rounded sum is that of the exact one).
 struct FillSetup {
-    D3 v0, n;
+    D3 n;
     D2 ne[3];
-    double de[3];
+    double de[3], th[3];
 };
 __device__ __forceinline__ void fill_setup(const D3 v[3], FillSetup &fs) {
-    fs.v0 = v[0];
     fs.n = dcross(dsub(v[0], v[2]), dsub(v[1], v[0]));
 #pragma unroll
     for (int i = 0; i < 3; i++) {
@@ -168,29 +169,25 @@ __device__ __forceinline__ void fill_setup(const D3 v[3], FillSetup &fs) {
         else
             fs.ne[i] = {b.z - a.z, a.y - b.y};
         fs.de[i] = -(fs.ne[i].x * a.y + fs.ne[i].y * a.z);
+        fs.th[i] = fs.ne[i].x > 0.0 || (fs.ne[i].x == 0.0 && fs.ne[i].y < 0.0) ? -VOX_DBL_MIN : 0.0;
     }
 }
-// Centre test with the DBL_MIN top-left tie break and the x crossing
-// (src/voxelizer.cu:1418-1453); voxelX includes the +1 x padding.
-__device__ __forceinline__ bool fill_center(const FillSetup &fs, double emx, double emy,
-                                            double emz, double d, uint32_t cy, uint32_t cz,
-                                            uint32_t &voxelX) {
-    double px = double(cy) * d + emy;
-    double py = double(cz) * d + emz;
-    uint32_t ok = 0;
+// Centre test (src/voxelizer.cu:1418-1436) at the centre (px, py).
+__device__ __forceinline__ bool fill_inside(const FillSetup &fs, double px, double py) {
+    bool in = true;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        double r = fs.ne[i].x * px + fs.ne[i].y * py + fs.de[i];
-        if (fs.ne[i].x > 0.0 || (fs.ne[i].x == 0.0 && fs.ne[i].y < 0.0)) r += VOX_DBL_MIN;
-        if (r > 0.0) ok++;
-    }
-    if (ok != 3u) return false;
-    double ax = fs.v0.x - emx, ay = fs.v0.y - px, az = fs.v0.z - py;
-    double B = ax * fs.n.x + ay * fs.n.y + az * fs.n.z;
-    double x = B / fs.n.x;
+    for (int i = 0; i < 3; i++) in &= fs.ne[i].x * px + fs.ne[i].y * py + fs.de[i] > fs.th[i];
+    return in;
+}
+// x crossing (src/voxelizer.cu:1437-1453) there, +1 for the x padding; ax: the
+// first vertex's x from the grid's origin, times n.x; y0, z0: its y and z.
+__device__ __forceinline__ uint32_t fill_crossing(const D3 &n, double ax, double y0, double z0,
+                                                  double px, double py, double d) {
+    const double ay = y0 - px, az = z0 - py;
+    const double B = ax + ay * n.y + az * n.z;
+    double x = B / n.x;
     x = x < 0.0 ? 0.0 : x;
-    voxelX = sat_u32(ceil(x / d)) + 1u;
-    return true;
+    return sat_u32(ceil(x / d)) + 1u;
 }
 
 // ---------------------------------------------------------------------------

@@ -371,7 +371,7 @@ BrickDims brick_dims(const vox_grid &g, const int bdim[3]) {
     return d;
 }
 
-// A brick shape the surface and node passes support: powers of two, x a
+// A brick shape that may be set: one of the two by the grid, or powers of two, x a
 // multiple of 64, at most 32 rows (y*z), at most 32 words per z plane (one
 // mask word per brick layer), at least 4 planes (a layer then never spans
 // two waves of the brick pass's epilogue), 256 to kMaxBrickVox voxels (the
@@ -838,6 +838,13 @@ struct ErodeBufs {
 };
 constexpr uint32_t kErodeBatch = 4;  // passes per launch group and read-back
 
+// The brick pairs' places, dead before the brick pass: in the material grid,
+// which that pass is the first to write, where it is large enough.
+vox_status place_buf(vox_ctx *ctx, const Plan &P, uint32_t n, uint32_t **out) {
+    if ((size_t)n * 4 <= P.mat_bytes) return buf(ctx, "a_matgrid", P.mat_bytes / 4, out);
+    return buf(ctx, "f_place", n, out);
+}
+
 vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, ErodeBufs &E) {
     const uint32_t nj = (uint32_t)P.jobs.size();
     const uint32_t nslots = P.tri_b.back(), nTiles = P.tile_b.back(), nbt = P.brick_b.back();
@@ -956,7 +963,7 @@ vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, Erode
     A.cap = total_s;
     A.ovf = ctx->fixed ? ctx->ovf : nullptr;
     if (surf) {
-        VOX_TRY(buf(ctx, "f_place", total_f, &B.place));
+        VOX_TRY(place_buf(ctx, P, total_f, &B.place));
         VOX_TRY(buf(ctx, "f_blist", total_f, &B.list));
         VOX_TRY(buf(ctx, "f_first", block_starts_size(total_f), &first_f));
         B.off = T.off_f;
@@ -2163,7 +2170,7 @@ vox_status graph_capture(vox_graph *g) {
     VOX_TRY(buf(w, "s_pmask", w->cap_solid, &u16));
     VOX_TRY(buf(w, "s_list_mask", w->cap_solid, &u16));
     VOX_TRY(buf(w, "f_blist", w->cap_surf, &u));
-    VOX_TRY(buf(w, "f_place", w->cap_surf, &u));
+    if (P.any_mats) VOX_TRY(place_buf(w, P, w->cap_surf, &u));
     VOX_TRY(buf(w, "s_first", block_starts_size(w->cap_solid), &u));
     VOX_TRY(buf(w, "f_first", block_starts_size(w->cap_surf), &u));
     VOX_TRY(buf(w, "e_changes", (size_t)w->n_passes * nj, &u));

@@ -18,7 +18,7 @@ namespace vk {
 
 // ---------------------------------------------------------------------------
 // Features of one brick, from the (triangle, brick) pairs of its list and
-// the per-triangle class, brick box and voxel extents of k_surf_setup:
+// the per-triangle class, brick box and voxel extents of k_tri_setup:
 //  0 log1p(triangles)            1-3 log1p(1D / 2D / 3D triangles)
 //  4-6 log1p(estimated items of 1D / 2D / 3D triangles in the brick)
 //  7 log1p(estimated 3D voxel tests)   8 log1p(largest estimated items)

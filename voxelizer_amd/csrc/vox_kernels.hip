@@ -264,23 +264,54 @@ __global__ __launch_bounds__(256) void k_block_starts(BlockStarts a, BlockStarts
     }
 }
 
-// The triangle of candidate base + threadIdx.x, for a 256-thread block: the
-// triangles that start among its candidates (few and consecutive) leave their
-// number where they start, and a running maximum over the block spreads them.
-// One coalesced load and one scan, where a binary search per thread took eight
-// or more dependent loads.  Triangles without candidates start where the next
-// one does and lose to its larger number.
+// The triangle of candidate base + threadIdx.x, for a 256-thread block, among
+// the n from that of its first candidate to that of the next block's first.
+// Triangles without candidates count in n: where most of the mesh has none (a
+// slice, a thin partition), a block beside such a run has most of the mesh there.
+//
+// Up to 256, a triangle per thread: those that start among the block's candidates
+// leave their number where they start, and a running maximum over the block
+// spreads them: one coalesced load and one scan, where a search takes eight
+// dependent loads.  Triangles without candidates start where the next one does
+// and lose to its larger number.  Above 256 every thread searches for the last
+// triangle that starts at or before its candidate: 256 samples through LDS, then
+// log2(n / 256) dependent loads.
+//
+// The hall (1.4 M triangles), calls with a walk of the n in steps of 256 instead,
+// with one up to 1024 and with this: z slice at 800 voxels 3281, 301, 302 us (up
+// to 5390 steps), x slice at 400 1664, 577, 573 us, solid bits at 400 246, 213,
+// 212 us, at 1100 243, 234, 232 us, ShortNodes at 1533 1428, 1432, 1431 us.
 __device__ __forceinline__ uint32_t block_owner(const uint32_t *__restrict__ off,
                                                 const uint32_t *__restrict__ first,
                                                 uint32_t nslots, uint32_t base, uint32_t total,
                                                 CandLds &L) {
     const uint32_t b = base / 256u;
     const uint32_t t0 = first[b], t1 = base + 256u < total ? first[b + 1u] : nslots - 1u;
+    const uint32_t n = t1 - t0 + 1u;
+    if (n > 256u) {  // uniform
+        const uint32_t c = min(base + threadIdx.x, total - 1u);
+        const uint32_t step = (n + 255u) / 256u, s = t0 + threadIdx.x * step;
+        L.own[threadIdx.x] = s <= t1 ? off[s] : UINT32_MAX;
+        __syncthreads();
+        uint32_t i = 0u;
+#pragma unroll
+        for (uint32_t d = 128u; d; d >>= 1)
+            if (L.own[i + d] <= c) i += d;
+        uint32_t lo = t0 + i * step, hi = min(lo + step, t1 + 1u);
+        while (lo + 1u < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (off[mid] <= c)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        return lo;
+    }
     L.own[threadIdx.x] = threadIdx.x == 0u ? t0 : 0u;
     __syncthreads();
-    for (uint32_t t = t0 + threadIdx.x; t <= t1; t += 256u) {
-        const uint32_t o = off[t] - base;
-        if (o < 256u) atomicMax(&L.own[o], t);
+    if (threadIdx.x < n) {
+        const uint32_t o = off[t0 + threadIdx.x] - base;
+        if (o < 256u) atomicMax(&L.own[o], t0 + threadIdx.x);
     }
     __syncthreads();
     const uint32_t incl = wave_incl_max(L.own[threadIdx.x]);

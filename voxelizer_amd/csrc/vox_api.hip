@@ -2156,8 +2156,8 @@ vox_status graph_capture(vox_graph *g) {
     Plan P;
     VOX_TRY(graph_plan(g, P));
     const uint32_t nj = (uint32_t)P.jobs.size();
-    w->cap_solid = w->last_solid + w->last_solid / 8 + 256;
-    w->cap_surf = w->last_surf + w->last_surf / 8 + 256;
+    w->cap_solid = graph_capacity(w->last_solid);
+    w->cap_surf = graph_capacity(w->last_surf);
     w->n_passes = w->last_passes + 1;
     // Every buffer the capture uses is sized now: nothing may allocate or
     // synchronise while the stream is captured.

@@ -411,6 +411,24 @@ struct TriSetup {
 };
 __global__ void k_tri_setup(const Job *__restrict__ jobs, const uint32_t *__restrict__ tri_bases,
                             uint32_t njobs, uint32_t tri_blocks, TriSetup o, FillSegs clear);
+// Candidates are taken in blocks of 256.  Totals reach 2^32 - 1, so the passes
+// count blocks (at most 2^24; a candidate index would wrap when stepped past the
+// total): workgroup `block` of `blocks` takes blocks k, k + blocks, ... below n.
+__host__ __device__ __forceinline__ uint32_t cand_blocks(uint32_t total) {
+    return total / 256u + (total % 256u ? 1u : 0u);
+}
+struct CandRange {
+    uint32_t k, n, step;
+    __host__ __device__ __forceinline__ CandRange(uint32_t block, uint32_t blocks, uint32_t total)
+        : k(block), n(cand_blocks(total)), step(blocks) {}
+    __host__ __device__ __forceinline__ bool more() const { return k < n; }
+    __host__ __device__ __forceinline__ void next() { k += step; }
+};
+// List capacity of a replayed graph for a run that needed n pairs.
+inline uint32_t graph_capacity(uint32_t n) {
+    const uint64_t c = (uint64_t)n + n / 8u + 256u;
+    return c < UINT32_MAX ? (uint32_t)c : UINT32_MAX;
+}
 // first[b] = the triangle holding candidate 256*b of a candidate pass (off:
 // exclusive offsets, nslots + 2 entries); candidates at or past cap are skipped.
 struct BlockStarts {
@@ -419,7 +437,7 @@ struct BlockStarts {
     uint32_t *first;
 };
 __global__ void k_block_starts(BlockStarts a, BlockStarts b, uint32_t nslots);
-inline size_t block_starts_size(uint32_t total) { return (size_t)(total + 255u) / 256u + 1u; }
+inline size_t block_starts_size(uint32_t total) { return (size_t)cand_blocks(total) + 1u; }
 // The pair passes take the first min(total, cap) candidates; a total above cap
 // sets *ovf (a replayed graph sized by an earlier run reports that its lists
 // were too short).  With pmask (jobs with several y/z subspaces), pmask[c]

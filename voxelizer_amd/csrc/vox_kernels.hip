@@ -260,11 +260,11 @@ __global__ __launch_bounds__(256) void k_block_starts(BlockStarts a, BlockStarts
     const uint32_t total = S.off[nslots + 1u] ? 0u : min(S.off[nslots], S.cap);
     for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < nslots; t += gridDim.x * 256u) {
         const uint32_t lo = min(S.off[t], total), hi = min(S.off[t + 1u], total);
-        for (uint32_t k = (lo + 255u) / 256u; k * 256u < hi; k++) S.first[k] = t;
+        for (uint32_t k = cand_blocks(lo); k < cand_blocks(hi); k++) S.first[k] = t;
     }
 }
 
-// The triangle of candidate base + threadIdx.x, for a 256-thread block, among
+// The triangle of candidate 256 k + threadIdx.x, for a 256-thread block, among
 // the n from that of its first candidate to that of the next block's first.
 // Triangles without candidates count in n: where most of the mesh has none (a
 // slice, a thin partition), a block beside such a run has most of the mesh there.
@@ -283,10 +283,10 @@ __global__ __launch_bounds__(256) void k_block_starts(BlockStarts a, BlockStarts
 // 212 us, at 1100 243, 234, 232 us, ShortNodes at 1533 1428, 1432, 1431 us.
 __device__ __forceinline__ uint32_t block_owner(const uint32_t *__restrict__ off,
                                                 const uint32_t *__restrict__ first,
-                                                uint32_t nslots, uint32_t base, uint32_t total,
+                                                uint32_t nslots, uint32_t k, uint32_t total,
                                                 CandLds &L) {
-    const uint32_t b = base / 256u;
-    const uint32_t t0 = first[b], t1 = base + 256u < total ? first[b + 1u] : nslots - 1u;
+    const uint32_t base = k * 256u, nb = cand_blocks(total);
+    const uint32_t t0 = first[k], t1 = k + 1u < nb ? first[k + 1u] : nslots - 1u;
     const uint32_t n = t1 - t0 + 1u;
     if (n > 256u) {  // uniform
         const uint32_t c = min(base + threadIdx.x, total - 1u);
@@ -409,11 +409,11 @@ __device__ __forceinline__ void count_solid(const Job *__restrict__ jobs,
     const uint32_t full = a.off[nslots], wrap = a.off[nslots + 1u];
     const uint32_t total = wrap ? 0u : min(full, a.cap);
     if (a.ovf && (full > a.cap || wrap) && block == 0u && threadIdx.x == 0) *a.ovf = 1u;
-    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
+    for (CandRange r(block, blocks, total); r.more(); r.next()) {
         __syncthreads();
         agg_clear(L.agg);
-        const uint32_t c = base + threadIdx.x;
-        const uint32_t t = block_owner(a.off, a.first, nslots, base, total, L);
+        const uint32_t c = r.k * 256u + threadIdx.x;
+        const uint32_t t = block_owner(a.off, a.first, nslots, r.k, total, L);
         bool hit = false;
         uint32_t tile = 0;
         if (c < total) {
@@ -474,11 +474,11 @@ __device__ __forceinline__ void count_surf(const Job *__restrict__ jobs,
     const uint32_t full = a.off[nslots], wrap = a.off[nslots + 1u];
     const uint32_t total = wrap ? 0u : min(full, a.cap);
     if (a.ovf && (full > a.cap || wrap) && block == 0u && threadIdx.x == 0) *a.ovf = 1u;
-    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
+    for (CandRange r(block, blocks, total); r.more(); r.next()) {
         __syncthreads();
         agg_clear(L.agg);
-        const uint32_t c = base + threadIdx.x;
-        const uint32_t t = block_owner(a.off, a.first, nslots, base, total, L);
+        const uint32_t c = r.k * 256u + threadIdx.x;
+        const uint32_t t = block_owner(a.off, a.first, nslots, r.k, total, L);
         const bool live = c < total;
         const uint32_t b = live ? cand_brick<kMulti>(jobs, tri_job, a, t, c) : 0u;
         const uint32_t place = bin_place(L, live, b, a.hist);
@@ -516,10 +516,10 @@ __global__ __launch_bounds__(256) void k_pairs_place(const Job *__restrict__ job
     const uint32_t blocks = solid ? solid_blocks : gridDim.x - solid_blocks;
     const uint32_t *off = solid ? a.off : b.off, *first = solid ? a.first : b.first;
     const uint32_t total = off[nslots + 1u] ? 0u : min(off[nslots], solid ? a.cap : b.cap);
-    for (uint32_t base = block * 256u; base < total; base += blocks * 256u) {
+    for (CandRange r(block, blocks, total); r.more(); r.next()) {
         __syncthreads();
-        const uint32_t c = base + threadIdx.x;
-        const uint32_t t = block_owner(off, first, nslots, base, total, L);
+        const uint32_t c = r.k * 256u + threadIdx.x;
+        const uint32_t t = block_owner(off, first, nslots, r.k, total, L);
         if (c >= total) continue;  // the last trip
         if (solid) {
             const uint2 pr = a.pairs[c];

@@ -169,6 +169,11 @@ struct vox_ctx {
     // instead of hipMalloc.
     uint8_t *scratch_dev = nullptr;
     bool arena = false;
+    bool arena_full = false;  // the call needed more
+    // A no-allocation call with the smallest needs: wide bricks, which thin
+    // triangles share in fewer pairs, and pairs counted twice instead of kept
+    // places.
+    bool lean = false;
     size_t arena_used = 0;
     int arena_n = 0;
     ArenaSlot arena_slot[kArenaSlots];
@@ -231,11 +236,13 @@ vox_status arena_buf(vox_ctx *ctx, const char *name, size_t bytes, void **out) {
         slot->name[sizeof(slot->name) - 1] = '\0';
     }
     const size_t off = (ctx->arena_used + 255) & ~(size_t)255;
-    if (off > kNoAllocScratchBytes || bytes > kNoAllocScratchBytes - off)
+    if (off > kNoAllocScratchBytes || bytes > kNoAllocScratchBytes - off) {
+        ctx->arena_full = true;
         return fail(ctx, VOX_ERR_UNSUPPORTED,
                     "no-allocation call: this grid needs more scratch than the " +
                         std::to_string(kNoAllocScratchBytes >> 20) +
                         " MiB the library holds per device (use vox_voxelize_nodes)");
+    }
     slot->off = off;
     slot->cap = bytes;
     ctx->arena_used = off + bytes;
@@ -408,7 +415,8 @@ void brick_shape(const vox_ctx *ctx, bool fcc, const uint32_t alloc[3], int out[
         const uint64_t n = bricks(pick), nw = bricks(wide);
         const uint64_t v = n * voxels(pick), vw = nw * voxels(wide);
         // A triangle's box of bricks has 16 bits per axis.
-        if (alloc[0] > 0xFFFFu * 32u || (ctx->arena ? v > vw || n > nw : v > vw + vw / 8u))
+        if (alloc[0] > 0xFFFFu * 32u || ctx->lean ||
+            (ctx->arena ? v > vw || n > nw : v > vw + vw / 8u))
             pick = wide;
     }
     for (int a = 0; a < 3; a++) out[a] = pick[a];
@@ -853,6 +861,7 @@ vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, Erode
     const bool fine = nslots / kScanTile < kScanFineTiles;  // 256-slot sums for the scans
     TriSetup T{};
     uint32_t *tile_hist, *tile_off, *brick_hist = nullptr, *brick_off = nullptr;
+    uint32_t *brick_cursor = nullptr;  // pairs placed per brick, where their places aren't kept
     VOX_TRY(buf(ctx, "tri_rec", (size_t)std::max<uint32_t>(nslots, 1) * 3, &R.rec));
     if (nj > 1) VOX_TRY(buf(ctx, "tri_job", nslots, &R.tri_job));
     VOX_TRY(buf(ctx, "s_cand_off", (size_t)nslots + 2, &T.off_s));
@@ -873,6 +882,7 @@ vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, Erode
         VOX_TRY(buf(ctx, "f_part", 2 * (size_t)tri_blocks, &T.part_f));
         VOX_TRY(buf(ctx, "f_brick_hist", nbt, &brick_hist));
         VOX_TRY(buf(ctx, "f_brick_off", (size_t)nbt + 2, &brick_off));
+        if (ctx->lean) VOX_TRY(buf(ctx, "f_brick_cursor", nbt, &brick_cursor));
         VOX_TRY(buf(ctx, "f_order", nbt, &R.order));
         VOX_TRY(buf(ctx, "f_n_list", 1, &R.n_list));
         VOX_TRY(buf(ctx, "f_stats", 1, &R.stats));
@@ -896,6 +906,7 @@ vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, Erode
     const FillSeg zero[] = {{ctx->fixed ? ctx->ovf : nullptr, 1, 0u},
                             {tile_hist, nTiles, 0u},
                             {brick_hist, nbt, 0u},
+                            {brick_cursor, nbt, 0u},
                             {R.wmask, (size_t)nbt * 4u, 0u},
                             {R.stats, 1, 0u},
                             {R.next, kBrickLists * kBrickListPitch, 0u},
@@ -963,7 +974,8 @@ vox_status prepare(vox_ctx *ctx, const Plan &P, const PlanDev &D, Prep &R, Erode
     A.cap = total_s;
     A.ovf = ctx->fixed ? ctx->ovf : nullptr;
     if (surf) {
-        VOX_TRY(place_buf(ctx, P, total_f, &B.place));
+        if (!ctx->lean) VOX_TRY(place_buf(ctx, P, total_f, &B.place));
+        B.cursor = brick_cursor;
         VOX_TRY(buf(ctx, "f_blist", total_f, &B.list));
         VOX_TRY(buf(ctx, "f_first", block_starts_size(total_f), &first_f));
         B.off = T.off_f;
@@ -1699,12 +1711,18 @@ vox_status vox_voxelize_nodes_noalloc(vox_ctx *ctx, const vox_grid *g, vox_node_
     if (ctx->record)
         return fail(ctx, VOX_ERR_UNSUPPORTED,
                     "cost recording is not available in the no-allocation call");
+    // Again with the smallest needs where the scratch ran out.
+    vox_status st = VOX_ERR_UNSUPPORTED;
     ctx->arena = true;
-    ctx->arena_used = 0;
-    ctx->arena_n = 0;
-    const vox_status st =
-        voxelize_nodes_impl(ctx, g, kind, use_materials, vox_split, mat_split, nodes_dev);
-    ctx->arena = false;
+    for (int lean = 0; lean < 2; lean++) {
+        ctx->arena_used = 0;
+        ctx->arena_n = 0;
+        ctx->arena_full = false;
+        ctx->lean = lean != 0;
+        st = voxelize_nodes_impl(ctx, g, kind, use_materials, vox_split, mat_split, nodes_dev);
+        if (st == VOX_OK || !ctx->arena_full) break;
+    }
+    ctx->arena = ctx->lean = false;
     return st;
 }
 

@@ -460,7 +460,8 @@ struct SolidPairs {
 struct SurfPairs {
     const uint32_t *off, *first;
     const uint4 *tri_info;
-    uint32_t *place;    // place in the brick's list per candidate
+    uint32_t *place;    // place in the brick's list per candidate; null: counted again
+    uint32_t *cursor;   // then: pairs placed per brick
     uint32_t *hist;     // pairs per brick
     const uint32_t *bin_off;
     uint32_t *list;

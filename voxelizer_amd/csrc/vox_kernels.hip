@@ -482,13 +482,14 @@ __device__ __forceinline__ void count_surf(const Job *__restrict__ jobs,
         const bool live = c < total;
         const uint32_t b = live ? cand_brick<kMulti>(jobs, tri_job, a, t, c) : 0u;
         const uint32_t place = bin_place(L, live, b, a.hist);
-        if (live) a.place[c] = place;
+        if (live && a.place) a.place[c] = place;
     }
 }
 
 // The counting sorts of (triangle, tile) and (triangle, brick) pairs by tile and
 // by brick: this pass counts the pairs of each bin and keeps every pair's place
-// in its bin, so the placing pass needs no counters of its own.  Both sorts
+// in its bin, so the placing pass needs no counters of its own (unless there was
+// no room for the bricks' places: then it counts again).  Both sorts
 // share a launch: blocks [0, solid_blocks) take the first, the rest the second.
 // Bound by the latency of its chain (starts, triangle, table, atomics): eight
 // waves a SIMD, which the registers allow, against six, hall 86 -> 77 us.
@@ -516,10 +517,18 @@ __global__ __launch_bounds__(256) void k_pairs_place(const Job *__restrict__ job
     const uint32_t blocks = solid ? solid_blocks : gridDim.x - solid_blocks;
     const uint32_t *off = solid ? a.off : b.off, *first = solid ? a.first : b.first;
     const uint32_t total = off[nslots + 1u] ? 0u : min(off[nslots], solid ? a.cap : b.cap);
+    const bool again = !solid && !b.place;
     for (CandRange r(block, blocks, total); r.more(); r.next()) {
         __syncthreads();
+        if (again) agg_clear(L.agg);
         const uint32_t c = r.k * 256u + threadIdx.x;
         const uint32_t t = block_owner(off, first, nslots, r.k, total, L);
+        if (again) {  // uniform
+            const uint32_t brick = c < total ? cand_brick<kMulti>(jobs, tri_job, b, t, c) : 0u;
+            const uint32_t place = bin_place(L, c < total, brick, b.cursor);
+            if (c < total) b.list[b.bin_off[brick] + place] = t;
+            continue;
+        }
         if (c >= total) continue;  // the last trip
         if (solid) {
             const uint2 pr = a.pairs[c];

@@ -342,7 +342,7 @@ def bench_single(args, va, wl):
                    "nodes": n_nodes,
                    "dims": list(ctx.node_dims(grid, kind)), "triangles": mesh.nt,
                    "vox_split": list(vs), "mat_split": list(ms), "parallelism": "single GPU",
-                   "surface_brick": list(bdims)},
+                   "surface_brick": list(bdims) if any(bdims) else "by the grid"},
         "schedules": schedules_block(gv, args.execution, training),
         "stages_ms": {k: round(v, 4) for k, v in stage.items()},
         "roofline": roof, "cpu_baseline": cpu,

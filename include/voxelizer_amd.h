@@ -294,8 +294,9 @@ vox_status vox_mlp_grad(vox_ctx *ctx, const float *params_dev, const float *x_de
  * 128x4x8 on Cartesian grids and 64x4x4 on each FCC sub-grid.  Shapes to set are
  * those two, or powers of two with x a multiple of 64, y*z <= 32 rows and 256 to
  * 4096 voxels; Cartesian shapes need z a multiple of 4.  The shape changes speed
- * only, never output.  vox_get_brick_dims returns the set shape (32x8x16 before
- * one is set). */
+ * only, never output.  {0, 0, 0} is "the grid decides", to set and as
+ * vox_get_brick_dims returns it, so that a shape read and set back leaves the
+ * context as it was. */
 vox_status vox_set_brick_dims(vox_ctx *ctx, int fcc, const uint32_t dims[3]);
 vox_status vox_get_brick_dims(const vox_ctx *ctx, int fcc, uint32_t dims[3]);
 /* Times vox_voxelize_nodes (with materials) for this grid and node kind

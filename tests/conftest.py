@@ -28,3 +28,14 @@ def gpu_ctx():
     ctx = va.Context(0)
     yield ctx
     ctx.close()
+
+
+@pytest.fixture(autouse=True)
+def brick_shape_by_grid(request):
+    """A test that sets a brick shape on the shared context leaves the grid's
+    own choice to the tests after it, which run what users get."""
+    ctx = request.getfixturevalue("gpu_ctx") if "gpu_ctx" in request.fixturenames else None
+    yield
+    if ctx is not None:
+        for fcc in (False, True):
+            ctx.set_brick_dims((0, 0, 0), fcc)

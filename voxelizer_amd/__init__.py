@@ -487,10 +487,13 @@ class Context:
         return Graph(self, h, items)
 
     def set_brick_dims(self, dims, fcc: bool = False):
+        """Surface brick shape of Cartesian grids or FCC sub-grids; (0, 0, 0):
+        the grid decides, as until one is set."""
         d = np.array(dims, np.uint32)
         self._check(lib().vox_set_brick_dims(self.h, 1 if fcc else 0, _ptr(d)))
 
     def brick_dims(self, fcc: bool = False):
+        """The shape that was set, or (0, 0, 0) where the grid decides."""
         d = np.zeros(3, np.uint32)
         self._check(lib().vox_get_brick_dims(self.h, 1 if fcc else 0, _ptr(d)))
         return tuple(int(x) for x in d)

@@ -1941,18 +1941,20 @@ vox_status vox_get_stage_times(const vox_ctx *ctx, vox_stage_times *out) {
 // ---- surface brick shape ----------------------------------------------------
 
 vox_status vox_set_brick_dims(vox_ctx *ctx, int fcc, const uint32_t dims[3]) {
-    if (!ctx || !dims || !brick_ok(dims, fcc == 0))
+    const bool by_grid = dims && !dims[0] && !dims[1] && !dims[2];
+    if (!ctx || !dims || !(by_grid || brick_ok(dims, fcc == 0)))
         return ctx ? fail(ctx, VOX_ERR_INVALID, "unsupported brick shape") : VOX_ERR_INVALID;
+    (fcc ? ctx->fcc_auto : ctx->cart_auto) = by_grid;
     int *d = fcc ? ctx->fcc_bdim : ctx->cart_bdim;
-    for (int a = 0; a < 3; a++) d[a] = (int)dims[a];
-    (fcc ? ctx->fcc_auto : ctx->cart_auto) = false;
+    for (int a = 0; a < 3 && !by_grid; a++) d[a] = (int)dims[a];
     return VOX_OK;
 }
 
 vox_status vox_get_brick_dims(const vox_ctx *ctx, int fcc, uint32_t dims[3]) {
     if (!ctx || !dims) return VOX_ERR_INVALID;
     const int *d = fcc ? ctx->fcc_bdim : ctx->cart_bdim;
-    for (int a = 0; a < 3; a++) dims[a] = (uint32_t)d[a];
+    const bool by_grid = fcc ? ctx->fcc_auto : ctx->cart_auto;
+    for (int a = 0; a < 3; a++) dims[a] = by_grid ? 0u : (uint32_t)d[a];
     return VOX_OK;
 }
 

@@ -300,9 +300,11 @@ vox_status vox_mlp_grad(vox_ctx *ctx, const float *params_dev, const float *x_de
 vox_status vox_set_brick_dims(vox_ctx *ctx, int fcc, const uint32_t dims[3]);
 vox_status vox_get_brick_dims(const vox_ctx *ctx, int fcc, uint32_t dims[3]);
 /* Times vox_voxelize_nodes (with materials) for this grid and node kind
- * with each candidate shape (one warm-up, then the best of `reps` runs),
- * keeps the fastest for the context and returns it and its time.  nodes_dev
- * ends up holding the nodes, as after a vox_voxelize_nodes call. */
+ * with each candidate shape (one warm-up round, then `reps` rounds of a run of
+ * each; a shape's best run counts), sets the fastest for the context and returns
+ * it and its time.  The shape the grid decides on is kept unless another gains
+ * more than that shape's runs differ.  nodes_dev ends up holding the nodes, as
+ * after a vox_voxelize_nodes call. */
 vox_status vox_autotune_bricks(vox_ctx *ctx, const vox_grid *grid, vox_node_kind kind,
                                const uint32_t vox_split[3], const uint32_t mat_split[3],
                                void *nodes_dev, uint32_t reps, uint32_t best_dims[3],

@@ -2,6 +2,9 @@
 number of (triangle, brick) pairs; and the shapes it picks, bit-compared with the
 oracle where a shape could go wrong: slices, partitions, matSplitRes intervals
 that end inside a brick, and bricks cut along z by the learned schedule."""
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -132,3 +135,44 @@ def test_cut_bricks_match_oracle(ctx, oracle, kind, brick):
         ctx.set_brick_dims(BY_GRID, fcc)
     assert used == 1
     assert np.array_equal(got, oracle.voxelize_nodes(m, og, kind, True))
+
+
+def test_autotune_keeps_the_grids_shape_when_its_first_runs_are_slow():
+    """The autotuner starts while another context keeps the device busy for about
+    as long as one shape's three runs: the shape it keeps is no slower than the
+    grid's own (the best of the hall's; the next is 7% slower)."""
+    m = W.hall(seed=0)
+    split = (1024, 1024, 1024)
+    c, other = va.Context(0), va.Context(0)
+    try:
+        for x in (c, other):
+            load(x, m)
+        g = c.plan_grid(va.PLAN_CUBE_LENGTH, 1.0 / 64.0)
+        n = c.node_count(g, va.NODE_SHORT)
+        out, out2 = va.DeviceBuffer(c, n), va.DeviceBuffer(other, n)
+
+        def call(x, o):
+            t = time.perf_counter()
+            x.voxelize_nodes_device(g, va.NODE_SHORT, o.ptr.value, True, split)
+            x.sync()
+            return time.perf_counter() - t
+
+        def busy():
+            end = time.perf_counter() + 0.008
+            while time.perf_counter() < end:
+                call(other, out2)
+
+        call(other, out2)
+        by_grid = min(call(c, out) for _ in range(10))
+        load_thread = threading.Thread(target=busy)
+        load_thread.start()
+        dims, _ = c.autotune_bricks(g, va.NODE_SHORT, out.ptr.value, 2, split)
+        load_thread.join()
+        tuned = min(call(c, out) for _ in range(10))
+        out.free()
+        out2.free()
+    finally:
+        other.close()
+        c.close()
+    print(f"by the grid {by_grid * 1e6:.0f} us, tuned {dims} {tuned * 1e6:.0f} us", flush=True)
+    assert tuned < 1.04 * by_grid

@@ -1970,25 +1970,37 @@ vox_status vox_autotune_bricks(vox_ctx *ctx, const vox_grid *grid, vox_node_kind
                                        {128, 2, 4}, {64, 2, 8}};
     const uint32_t(*cand)[3] = fcc ? fccs : cart;
     const size_t ncand = fcc ? sizeof(fccs) / sizeof(fccs[0]) : sizeof(cart) / sizeof(cart[0]);
-    double best = 1e300;
-    size_t bi = 0;
-    for (size_t c = 0; c < ncand; c++) {
-        VOX_TRY(vox_set_brick_dims(ctx, fcc ? 1 : 0, cand[c]));
-        double t_best = 1e300;
-        for (uint32_t r = 0; r <= reps; r++) {  // run 0 warms up
+    // The shape the grid decides on is among the candidates.
+    int own[3];
+    const bool was_auto = fcc ? ctx->fcc_auto : ctx->cart_auto;
+    (fcc ? ctx->fcc_auto : ctx->cart_auto) = true;
+    brick_shape(ctx, fcc, grid->alloc, own);
+    (fcc ? ctx->fcc_auto : ctx->cart_auto) = was_auto;
+    size_t oi = 0;
+    for (size_t c = 0; c < ncand; c++)
+        if ((int)cand[c][0] == own[0] && (int)cand[c][1] == own[1] && (int)cand[c][2] == own[2]) oi = c;
+    // One run of every shape in turn, so that what slows a while (a device that
+    // was idle or busy elsewhere) slows them all: with a shape's runs one after
+    // another the first shape was measured cold, and the hall (1536x1024x768)
+    // ended with 128x4x8 (1.43 ms) instead of 32x8x16 (1.34 ms) in two of six runs.
+    std::vector<double> lo(ncand, 1e300), hi(ncand, 0.0);
+    for (uint32_t r = 0; r <= reps; r++)  // round 0 warms up
+        for (size_t c = 0; c < ncand; c++) {
+            VOX_TRY(vox_set_brick_dims(ctx, fcc ? 1 : 0, cand[c]));
             VOX_TRY(vox_sync(ctx));
             const auto t0 = std::chrono::steady_clock::now();
             VOX_TRY(vox_voxelize_nodes(ctx, grid, kind, 1, vox_split, mat_split, nodes_dev));
             VOX_TRY(vox_sync(ctx));
             const double dt =
                 std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-            if (r > 0) t_best = std::min(t_best, dt);
+            if (r == 0) continue;
+            lo[c] = std::min(lo[c], dt);
+            hi[c] = std::max(hi[c], dt);
         }
-        if (t_best < best) {
-            best = t_best;
-            bi = c;
-        }
-    }
+    // The grid's own shape stays unless another's gain exceeds its spread.
+    size_t bi = (size_t)(std::min_element(lo.begin(), lo.end()) - lo.begin());
+    if (lo[oi] - lo[bi] <= hi[oi] - lo[oi]) bi = oi;
+    const double best = lo[bi];
     // Every shape writes the same nodes, so nodes_dev already holds them.
     VOX_TRY(vox_set_brick_dims(ctx, fcc ? 1 : 0, cand[bi]));
     if (best_dims)

@@ -219,7 +219,9 @@ size_t vox_node_size(vox_node_kind kind);
 /* ---- instrumentation (no counterpart in the reference) ----------------- */
 
 /* Per-stage device times (ms) of the last vox_voxelize_nodes/vox_solid_bits
- * call, measured with HIP events on the context stream when enabled. */
+ * call, measured with HIP events on the context stream when enabled.
+ * solid_fill_ms holds the preparation of the solid and of the surface stage, which
+ * share their launches, and the fill. */
 typedef struct vox_stage_times {
     float plan_ms, solid_bin_ms, solid_fill_ms, surface_ms, erode_ms, nodes_ms, total_ms;
     uint32_t erosion_passes;

@@ -126,12 +126,13 @@ struct vox_ctx {
     float *cost_params = nullptr;  // device, kCostParams floats
     bool cost_ready = false;
     float heavy_cost = 1.5f;    // standardized log cost above which a brick goes first
-    // Pair count / mean from which a brick's cost is predicted.  Measured on
-    // the large hall and the 256-mesh batch (Gvoxels/s): 6 -> 571 / 365,
-    // 12 -> 576 / 366, 24 -> 579 / 368 in one run, 24 -> 577 / 362,
-    // 48 -> 567 / 359, 96 -> 560 / 342 in another.  Below 24 the features of
-    // light bricks cost more than their order gains; above it heavy bricks
-    // are missed.
+    // Pair count / mean from which a brick's cost is predicted.  Below 24 the
+    // features of light bricks cost more than their order gains on most meshes;
+    // above it heavy bricks are missed.  Calls in us with 6, 12, 24, 48, 96 and
+    // the plain schedule: hall at 1533 voxels 1437, 1424, 1432, 1456, 1479, 1459;
+    // at 800 735, 729, 734, 844, 808, 835; at 400, where heavy bricks are many,
+    // 865, 851, 864, 838, 842, 835; 64-mesh batch 2177, 2161, 2153, 2156, 2147,
+    // 2128.
     float screen_ratio = 24.0f;
     // Sub-bricks per heavy brick at most (1, 2 or 4); 0: from the number of
     // bricks per resident brick-pass workgroup.
@@ -378,19 +379,17 @@ BrickDims brick_dims(const vox_grid &g, const int bdim[3]) {
     return d;
 }
 
-// A brick shape that may be set: one of the two by the grid, or powers of two, x a
-// multiple of 64, at most 32 rows (y*z), at most 32 words per z plane (one
-// mask word per brick layer), at least 4 planes (a layer then never spans
-// two waves of the brick pass's epilogue), 256 to kMaxBrickVox voxels (the
-// brick pass finishes 256 voxels per wave step), and (for the Cartesian node
-// pass, whose threads own kNodeZ planes) z a multiple of kNodeZ.
+// A brick shape that may be set: one of the two by the grid, or powers of two with
+// 256 to kMaxBrickVox voxels (the brick pass finishes 256 voxels per wave step,
+// keeps a key per voxel in LDS and a brick's word mask in 128 bits) and, for the
+// Cartesian node pass, whose threads own kNodeZ planes, z a multiple of kNodeZ.
+// The other limits (x at least 64, at most 32 rows, at most 32 words in a layer of
+// more than 256 voxels and then 4 planes) keep the choice to shapes that are
+// tested; no pass needs them.
 bool brick_ok(const uint32_t b[3], bool cart) {
     for (int a = 0; a < 3; a++)
         if (b[a] == 0 || (b[a] & (b[a] - 1)) != 0) return false;
     const uint32_t nvox = b[0] * b[1] * b[2];
-    // The brick pass's epilogue gives each wave whole layers: a layer of at
-    // most 256 voxels tiles its 256-voxel steps; a larger one needs bricks at
-    // least 4 deep (each wave then takes a multiple of a layer's steps).
     for (const int *d : {kBrick, kFlatBrick})
         if (b[0] == (uint32_t)d[0] && b[1] == (uint32_t)d[1] && b[2] == (uint32_t)d[2]) return true;
     return b[0] >= 64 && b[1] * b[2] <= 32 && (b[0] / 32) * b[1] <= 32 &&

@@ -31,7 +31,6 @@ __device__ __forceinline__ VK_G T *gptr(T *p) {
 }
 // Native 4 x u32 vector for 16-byte global accesses through VK_G pointers.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Workgroups are dispatched round-robin over the XCDs.  Row kernels launch
 // kXcds * ceil(n / kXcds) workgroups and map workgroup i to logical block

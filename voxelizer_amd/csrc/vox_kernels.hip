@@ -1922,8 +1922,10 @@ __device__ __forceinline__ void id_bytes(const IdPlanes &o, uint32_t idw[8]) {
 // OR in their material (bytes of the word's other voxels are 0 in the
 // material grid).  The transpose replaced a loop over the boundary voxels
 // that patched their bytes in LDS: room at 1 cm (512x403x303 LongNodes) 38.9
-// -> 31.2 us, hall (1536x1024x768 ShortNodes) 385 -> 362 us, there bound by
-// its 1.7 GB of reads and writes (4.8 TB/s, where a large copy runs at 5.0).
+// -> 31.2 us, hall (1536x1024x768 ShortNodes) 385 -> 362 us, both with 128x4x8
+// bricks: 4.8 TB/s of the hall's 1.7 GB, where a large copy runs at 5.0.  With
+// 32x8x16 bricks, whose material words of neighbouring lanes lie 4 KB apart, the
+// hall takes 428 us (1.6 GB at 3.75 TB/s); the brick pass gains more.
 //
 // With several erosion subspaces (voxSplitRes y/z smaller than the grid) the
 // reference computes a subspace's ids before later subspaces erode
@@ -2284,7 +2286,7 @@ __device__ __forceinline__ uint32_t fcc_word(uint32_t e, uint32_t o, uint32_t ha
 // of 32 nodes are turned into node masks by a bit-matrix transpose in
 // registers (144 operations whatever the number of boundary nodes), and the
 // wave's nodes go through LDS so that each store writes 1 KB of whole lines.
-// Room at 1.6 cm (640x255x384 LongFCCNodes, 251 MB): 54 us, 4.7 TB/s of node
+// Room at 1.6 cm (640x255x384 LongFCCNodes, 251 MB): 58 us, 4.3 TB/s of node
 // writes; a wave per 64 words of one row (20 of them there), nine interleaved
 // words per plane and a loop over the boundary nodes took 163 us.
 __global__ __launch_bounds__(256) void k_nodes_fcc(const Job *__restrict__ jobs,

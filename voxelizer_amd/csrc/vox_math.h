@@ -50,11 +50,6 @@ __device__ __forceinline__ int32_t f2i(float v) {
     return r;
 }
 
-__device__ __forceinline__ D3 fetch_d(const float *__restrict__ V, const uint32_t *__restrict__ I,
-                                      uint32_t t, int k) {
-    uint32_t i = I[3u * t + (uint32_t)k];
-    return {(double)V[3u * i], (double)V[3u * i + 1u], (double)V[3u * i + 2u]};
-}
 __device__ __forceinline__ F3 fetch_f(const float *__restrict__ V, const uint32_t *__restrict__ I,
                                       uint32_t t, int k) {
     uint32_t i = I[3u * t + (uint32_t)k];
